@@ -189,20 +189,27 @@ __host__ __device__ inline U4 sobol_owen(uint32_t seed, uint32_t pixel, uint32_t
 constexpr uint32_t kKeyCompat = 0x2545F491u;
 
 
-// Traversal node record: the two triangles of node k as (v1, e1 = v2-v1,
-// e2 = v3-v1) -- the same float values Ray::intersect computes on the fly
-// (src/kernels/lib/ray.cuh:25-26) -- followed by the slabs of the node's two
-// children on the children's axis (min/max of their six axis coordinates,
-// src/kernels/lib/intersect.cuh:106-111), and flags.  96 bytes, 16-byte
-// aligned.  One extra record after the last node (index n) holds the root's
-// own slab (axis 0) in cslab[0..1].
-//
-// A tree's records are kNodeBytes apart, or kNodeLineBytes (zero padding
-// after each record) when the array is too large to stay in the Infinity
-// Cache: unpadded, half the records straddle two 128-byte lines, and once
-// node visits go to HBM every extra line is paid for; while the array is
-// cache-resident the compact form keeps more records in L2.
-constexpr uint32_t kNodeSlabsNormal = 1u;  // every cslab value passes normal_coord
+// Traversal node record, 64 bytes: the slabs of node k's two children on the
+// children's axis (min/max of their six axis coordinates, exact floats,
+// src/kernels/lib/intersect.cuh:106-111) and a reduced copy of the node's two
+// triangles for the reject test of traverse.h, which decides which of them
+// need the reference's triangle test on their exact vertices:
+//   scale     2^-k with 2^k at least the extent of the node's two triangles
+//             and of its group (its own, its parent's and its grandparent's
+//             slabs), or infinity: no reject test for this node
+//   ref       scale * v1 of the first triangle (exact float)
+//   e         half pairs (first, second triangle) of scale * e1.xyz, e2.xyz
+//   dxy, dz_a half pairs (dx, dy) and (dz, size of the first triangle):
+//             scale * (v1 of the second - v1 of the first triangle)
+//   scale_b   float bits of scale (the low 23 are zero in it) with the second
+//             triangle's size (half) in bits 0..15 and flags in bits 16..22
+// A triangle's size is at least the largest |component| of its scaled e1 and
+// e2, and at least 2^-10.  One extra record after the last node (index n)
+// holds the root's own slab (axis 0) in cslab[0..1].
+constexpr uint32_t kNodeSlabsNormal = 1u << 16;  // every cslab value passes normal_coord
+// A missing child's slab (lo, hi) = (kNoSlab, -kNoSlab): empty for every ray
+// that takes the reciprocal quotient (|d| <= 16, |o| <= 2^57).
+constexpr float kNoSlab = 0x1p59f;
 
 // Coordinates x = 0 or 2^-72 <= |x| <= 2^59.  For a slab value s and a ray
 // origin coordinate p that both pass, the numerator n = RN(s - p) is 0 or
@@ -212,23 +219,22 @@ __host__ __device__ inline bool normal_coord(float x) {
   const float a = fabsf(x);
   return (x == 0.0f) | ((a >= 0x1p-72f) & (a <= 0x1p59f));
 }
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 struct alignas(16) NodeRec {
-  float tri[2][9];
   float cslab[4];  // left lo, left hi, right lo, right hi
-  uint32_t flags;
-  uint32_t spare;
+  float ref[3];
+  uint32_t scale_b;
+  half2v e[6];
+  half2v dxy, dz_a;
 };
-static_assert(sizeof(NodeRec) == 96, "node record");
-constexpr uint32_t kNodeBytes = 96;       // records back to back
-constexpr uint32_t kNodeLineBytes = 128;  // one record per 128-byte line
+static_assert(sizeof(NodeRec) == 64, "node record");
 
-// Record k of a tree whose records are rec_bytes apart.
-__host__ __device__ inline const NodeRec* node_at(const NodeRec* nodes, uint32_t k, uint32_t rec_bytes) {
-  return reinterpret_cast<const NodeRec*>(reinterpret_cast<const char*>(nodes) + (size_t)k * rec_bytes);
-}
-__host__ __device__ inline NodeRec* node_at(NodeRec* nodes, uint32_t k, uint32_t rec_bytes) {
-  return reinterpret_cast<NodeRec*>(reinterpret_cast<char*>(nodes) + (size_t)k * rec_bytes);
-}
+// The reject test's bounds (traverse.h) hold for scales and ray directions in
+// these ranges and coordinates up to kRejectCoord; outside them every
+// triangle takes the exact test.
+constexpr float kRejectScaleMin = 0x1p-40f, kRejectScaleMax = 0x1p40f;
+constexpr float kRejectDirMin = 0x1p-20f, kRejectDirMax = 0x1p20f;
+constexpr float kRejectCoord = 0x1p40f;
 
 // Subtree arithmetic of a left-complete binary tree of n nodes in heap order.
 // Number of nodes in the subtrees of the consecutive same-depth range [a, b).

@@ -112,6 +112,7 @@ constexpr uint32_t kCounterWords = 12;
 // (ry0 + l / rw) * w + rx0 + l % rw (the whole frame: rx0 = ry0 = 0, rw = w).
 struct JobDev {
   const NodeRec* nodes;
+  const float* tris;     // tree order, 9 floats per triangle (points layout)
   const float* normals;  // tree order, 9 floats per triangle
   const uint16_t* shader_ids;
   const aur_shader* shaders;
@@ -126,7 +127,6 @@ struct JobDev {
   uint32_t w, h, npix, spp, max_depth, rr_start, seed, paths;
   uint32_t rx0, ry0, rw;
   float2 root;  // the tree's root slab (axis 0)
-  uint32_t rec_bytes;  // distance between node records
   aur_camera cam;
 };
 
@@ -134,8 +134,8 @@ struct JobDev {
 struct SceneStore {
   uint32_t count = 0, levels = 0, num_shaders = 0, num_lights = 0, nslots = 0;
   float2 root_slab = make_float2(0.0f, 0.0f);
-  uint32_t rec_bytes = kNodeBytes;
   DevBuf<NodeRec> nodes;
+  DevBuf<float> vertices;
   DevBuf<float> normals;
   DevBuf<uint16_t> shader_ids;
   DevBuf<aur_shader> shaders;
@@ -209,7 +209,6 @@ struct aur_context {
   aur::DevBuf<uint16_t> shader_ids;
   aur::DevBuf<uint32_t> perm;
   aur::DevBuf<aur::NodeRec> nodes;
-  uint32_t rec_bytes = aur::kNodeBytes;  // distance between node records
   float root_lo = 0.0f, root_hi = 0.0f;
 
   // materials and lights

@@ -42,7 +42,6 @@ namespace {
 constexpr uint32_t kTile = 2048;  // radix / emit tile (elements)
 constexpr uint32_t kChunk = 32;   // tiles per chunk of the radix offset scan
 constexpr uint32_t kSubT = 2048;  // max elements of an LDS-resident subtree
-constexpr uint64_t kCompactNodeArrayMax = 128ull << 20;  // bytes
 constexpr int kThreads = 256;
 
 struct TileDesc {
@@ -802,58 +801,75 @@ __device__ inline void slab_of(const float* v, int a, float& lo, float& hi) {
              fmaxf(fmaxf(q[3 * a], q[3 * a + 1]), q[3 * a + 2]));
 }
 
-// Record k at k * rec_bytes; bytes after the 96 of a record are zero.
-__device__ inline void put_record(NodeRec* __restrict__ nodes, uint32_t k, uint32_t rec_bytes,
-                                  const NodeRec& r) {
-  NodeRec* dst = node_at(nodes, k, rec_bytes);
-  *dst = r;
-  float4* pad = reinterpret_cast<float4*>(dst + 1);
-  for (uint32_t q = 0; q < (rec_bytes - kNodeBytes) / 16; ++q) pad[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
-
-__global__ void k_node_records(const float* __restrict__ v, uint32_t n, uint32_t rec_bytes,
-                               NodeRec* __restrict__ nodes) {
+// Traversal record k (common.h); record n holds the root's own slab.
+__global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec* __restrict__ nodes) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k > n) return;
-  NodeRec r;
-  if (k == n) {  // the root's own slab, on axis 0
-#pragma unroll
-    for (int t = 0; t < 18; ++t) (&r.tri[0][0])[t] = 0.0f;
+  NodeRec r = {};
+  if (k == n) {  // on axis 0
     slab_of(v, 0, r.cslab[0], r.cslab[1]);
-    r.cslab[2] = r.cslab[3] = 0.0f;
-    r.flags = 0;
-    r.spare = 0;
-    put_record(nodes, k, rec_bytes, r);
+    nodes[k] = r;
     return;
   }
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const float* p = v + (size_t)(2 * k + t) * 9;  // points layout
-    const V3 v1 = mk(p[0], p[3], p[6]), v2 = mk(p[1], p[4], p[7]), v3 = mk(p[2], p[5], p[8]);
-    const V3 e1 = v2 - v1, e2 = v3 - v1;
-    r.tri[t][0] = v1.x;
-    r.tri[t][1] = v1.y;
-    r.tri[t][2] = v1.z;
-    r.tri[t][3] = e1.x;
-    r.tri[t][4] = e1.y;
-    r.tri[t][5] = e1.z;
-    r.tri[t][6] = e2.x;
-    r.tri[t][7] = e2.y;
-    r.tri[t][8] = e2.z;
-  }
+  const float* p = v + (size_t)k * 18;  // points layout, two triangles
   const uint32_t d = depth_of(k);
   const int ca = (int)((d + 1) % 3);
-  r.cslab[0] = r.cslab[2] = 0.0f;
-  r.cslab[1] = r.cslab[3] = 0.0f;
   const uint64_t cl = 2ull * k + 1;
+  r.cslab[0] = r.cslab[2] = kNoSlab;
+  r.cslab[1] = r.cslab[3] = -kNoSlab;
   if (cl < n) slab_of(v + cl * 18, ca, r.cslab[0], r.cslab[1]);
   if (cl + 1 < n) slab_of(v + (cl + 1) * 18, ca, r.cslab[2], r.cslab[3]);
   bool normal = true;
 #pragma unroll
   for (int c = 0; c < 4; ++c) normal = normal && normal_coord(r.cslab[c]);
-  r.flags = normal ? kNodeSlabsNormal : 0u;
-  r.spare = 0;
-  put_record(nodes, k, rec_bytes, r);
+  // the group's extent: the two triangles on every axis, and the slabs of
+  // the parent and the grandparent on theirs (the node's own is its triangles')
+  float extent = 0.0f, coord = 0.0f;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    float lo, hi;
+    slab_of(p, a, lo, hi);
+    extent = fmaxf(extent, hi - lo);
+    coord = fmaxf(coord, fmaxf(fabsf(lo), fabsf(hi)));
+  }
+  uint32_t anc = k;
+  for (uint32_t up = 1; up <= 2 && up <= d; ++up) {
+    float lo, hi;
+    anc = (anc - 1) / 2;
+    slab_of(v + (size_t)anc * 18, (int)((d - up) % 3), lo, hi);
+    extent = fmaxf(extent, hi - lo);
+  }
+  int ex = 0;
+  (void)frexpf(extent, &ex);  // extent < 2^ex
+  const bool reject = coord <= kRejectCoord && extent >= kRejectScaleMin && extent <= kRejectScaleMax;
+  const float scale = reject ? ldexpf(1.0f, -ex) : __builtin_inff();
+  float size[2], edge[2][6];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float* q = p + 9 * t;
+    size[t] = 0x1p-10f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float e1 = q[3 * a + 1] - q[3 * a], e2 = q[3 * a + 2] - q[3 * a];
+      edge[t][a] = reject ? e1 * scale : 0.0f;
+      edge[t][3 + a] = reject ? e2 * scale : 0.0f;
+      size[t] = fmaxf(size[t], fmaxf(fabsf(edge[t][a]), fabsf(edge[t][3 + a])));
+    }
+    size[t] *= 1.0f + 0x1p-10f;  // not below after rounding to half
+  }
+#pragma unroll
+  for (int c = 0; c < 6; ++c) r.e[c] = half2v{(_Float16)edge[0][c], (_Float16)edge[1][c]};
+  float dv[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    r.ref[a] = reject ? p[3 * a] * scale : 0.0f;
+    dv[a] = reject ? (p[9 + 3 * a] - p[3 * a]) * scale : 0.0f;
+  }
+  r.dxy = half2v{(_Float16)dv[0], (_Float16)dv[1]};
+  r.dz_a = half2v{(_Float16)dv[2], (_Float16)size[0]};
+  const half2v sb = {(_Float16)size[1], (_Float16)0.0f};
+  r.scale_b = __float_as_uint(scale) | (normal ? kNodeSlabsNormal : 0u) | __builtin_bit_cast(uint32_t, sb);
+  nodes[k] = r;
 }
 
 // cudaGenerateTB (utility.cu:136-180).
@@ -1109,19 +1125,13 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   AUR_HIP(ctx, ctx->normals.reserve((size_t)N * 9));
   AUR_HIP(ctx, ctx->texcoords.reserve((size_t)N * 6));
   AUR_HIP(ctx, ctx->shader_ids.reserve(N));
-  // records one cache line apart once the compact array would fill more than
-  // half of the 256 MB Infinity Cache (node visits then go to HBM)
-  const uint32_t rec_bytes =
-      (uint64_t)(n + 1) * kNodeBytes > kCompactNodeArrayMax ? kNodeLineBytes : kNodeBytes;
-  AUR_HIP(ctx, ctx->nodes.reserve(((size_t)(n + 1) * rec_bytes + sizeof(NodeRec) - 1) /
-                                  sizeof(NodeRec)));  // + the root's own slab
+  AUR_HIP(ctx, ctx->nodes.reserve((size_t)n + 1));  // + the root's own slab
   k_gather_geometry<<<blocks(N, 256), 256, 0, s>>>(ctx->perm.p, N, ctx->in_vertices.p,
                                                    ctx->in_normals.p, ctx->in_texcoords.p,
                                                    ctx->in_shader_ids.p, ctx->vertices.p,
                                                    ctx->normals.p, ctx->texcoords.p,
                                                    ctx->shader_ids.p);
-  k_node_records<<<blocks((uint64_t)n + 1, 256), 256, 0, s>>>(ctx->vertices.p, n, rec_bytes,
-                                                               ctx->nodes.p);
+  k_node_records<<<blocks((uint64_t)n + 1, 256), 256, 0, s>>>(ctx->vertices.p, n, ctx->nodes.p);
   AUR_LAUNCH_CHECK(ctx, "gather/node records");
   AUR_HIP(ctx, hipEventRecord(e1, s));
   AUR_HIP(ctx, hipEventSynchronize(e1));
@@ -1132,11 +1142,10 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   // the root's own slab (cslab[0..1] of record n) for launches that start
   // every ray at the root without reading it
   float root[2] = {0.0f, 0.0f};
-  AUR_HIP(ctx, hipMemcpyAsync(root, &node_at(ctx->nodes.p, n, rec_bytes)->cslab[0], sizeof(root),
+  AUR_HIP(ctx, hipMemcpyAsync(root, &ctx->nodes.p[n].cslab[0], sizeof(root),
                               hipMemcpyDeviceToHost, s));
   AUR_HIP(ctx, hipStreamSynchronize(s));
   ctx->root_slab = make_float2(root[0], root[1]);
-  ctx->rec_bytes = rec_bytes;
   ctx->levels = (uint32_t)L;
   ctx->built = true;
   ctx->has_tb = false;

@@ -35,7 +35,6 @@ constexpr int kBlock = 128;
 struct SceneDev {
   const NodeRec* nodes;
   uint32_t n_nodes;
-  uint32_t rec_bytes;
   const float* normals;
   const uint16_t* shader_ids;
   const aur_shader* shaders;
@@ -346,7 +345,7 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
     atomicAdd(&a.stats[1], (unsigned long long)n_sh);
   }
   persistent_trace(
-      TreeRef{a.job.nodes, a.job.n_nodes, a.job.root, a.job.rec_bytes}, (uint64_t)n_ext + n_sh,
+      TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, a.job.root}, (uint64_t)n_ext + n_sh,
       a.refill, stack,
       [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef& tree, bool& any) {
         float4 o4, d4;
@@ -366,7 +365,7 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
         }
         if constexpr (kMulti) {
           const JobDev& J = a.jobs[jb];
-          tree = TreeRef{J.nodes, J.n_nodes, J.root, J.rec_bytes};
+          tree = TreeRef{J.nodes, J.tris, J.n_nodes, J.root};
         }
         o = mk(o4.x, o4.y, o4.z);
         d = mk(d4.x, d4.y, d4.z);
@@ -1428,6 +1427,7 @@ JobDev frame_job(aur_context* ctx, const aur_camera* cam, const aur_render_opts*
   FrameState& fr = ctx->frame;
   JobDev J{};
   J.nodes = ctx->nodes.p;
+  J.tris = ctx->vertices.p;
   J.normals = ctx->normals.p;
   J.shader_ids = ctx->shader_ids.p;
   J.shaders = ctx->shaders.p;
@@ -1440,7 +1440,6 @@ JobDev frame_job(aur_context* ctx, const aur_camera* cam, const aur_render_opts*
   J.path_start = 0;
   J.n_nodes = ctx->count / 2;
   J.root = ctx->root_slab;
-  J.rec_bytes = ctx->rec_bytes;
   J.num_shaders = ctx->num_shaders;
   J.num_lights = ctx->num_lights;
   J.nslots = ctx->num_slots;
@@ -1513,10 +1512,9 @@ aur_status compat_passes(aur_context* ctx, const aur_camera* cam, const aur_rend
   st = trace_shape<false>(ctx, ctx->levels, (uint64_t)cap * per_pixel, a, lds, grid_trace);
   if (st != AUR_OK) return st;
   CwArgs c{};
-  c.sc = SceneDev{ctx->nodes.p,      ctx->count / 2,   ctx->rec_bytes,   ctx->normals.p,
-                  ctx->shader_ids.p, ctx->shaders.p,   ctx->num_shaders, ctx->lights.p,
-                  ctx->num_lights,   ctx->texcoords.p, ctx->textures.p,  ctx->texels.p,
-                  ctx->num_textures};
+  c.sc = SceneDev{ctx->nodes.p,      ctx->count / 2,   ctx->normals.p,    ctx->shader_ids.p,
+                  ctx->shaders.p,    ctx->num_shaders, ctx->lights.p,     ctx->num_lights,
+                  ctx->texcoords.p,  ctx->textures.p,  ctx->texels.p,     ctx->num_textures};
   c.cam = *cam;
   c.w = fr.width;
   c.h = fr.height;

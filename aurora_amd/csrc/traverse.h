@@ -25,16 +25,20 @@
 //     2^-96 <= |n| <= 2^60, true division otherwise.  Inside the loop the
 //     numerator range follows from a per-node flag (all four child slab
 //     values pass normal_coord) and a per-ray check of the origin;
-//   * both triangles of a node are tested without branches (every value is
-//     computed, the reference's early outs become one accept predicate with
-//     the same NaN behaviour), and 1/det is HIP's correctly rounded
-//     reciprocal sequence without its scaling and fix-up steps, which are
-//     identities for 2^-24 <= det <= 2^64 (det < kEpsilon is rejected before
-//     the value is used; det > 2^64 takes true division); the ray's
-//     reciprocals use the same sequence (needed only for 2^-60 <= |d| <= 16).
+//   * a node's two triangles first take a reject test on the record's
+//     reduced copy (trav_test), whose threshold bounds every rounding and
+//     quantisation error: a triangle it rejects fails the reference's test.
+//     The others (about one visit in 80 for meshes) take the reference's test on
+//     their exact vertices (trav_exact), in order, before the traversal of
+//     their ray goes on;
+//   * 1/det is HIP's correctly rounded reciprocal sequence without its
+//     scaling and fix-up steps, which are identities for 2^-24 <= det <= 2^64
+//     (det < kEpsilon is rejected before the value is used; det > 2^64 takes
+//     true division); the ray's reciprocals use the same sequence (needed
+//     only for 2^-60 <= |d| <= 16).
 //
-// The traversal is a small state machine (trav_init / trav_step, one node
-// visit per step) so that persistent kernels can refill finished lanes.
+// The traversal is a small state machine (trav_init, then trav_test,
+// trav_exact while candidates remain and trav_next per node visit) so that persistent kernels can refill finished lanes.
 #pragma once
 
 #include "common.h"
@@ -86,24 +90,6 @@ __device__ __forceinline__ float2 narrow(float2 r, float slo, float shi, float p
   return clip(r, d0, d1);
 }
 
-// Both children's slabs on one axis; `fast`: the divisor and all four
-// numerators are in the reciprocal quotient's range (else one shared, rarely
-// taken branch to true division).
-__device__ __forceinline__ void narrow2(float2 r, float4 slabs, float p, float d, float y,
-                                        bool fast, float2& rl, float2& rr) {
-  const float n0 = slabs.x - p, n1 = slabs.y - p, n2 = slabs.z - p, n3 = slabs.w - p;
-  float d0 = quot_fast(n0, d, y), d1 = quot_fast(n1, d, y);
-  float d2 = quot_fast(n2, d, y), d3 = quot_fast(n3, d, y);
-  if (!fast) {
-    d0 = n0 / d;
-    d1 = n1 / d;
-    d2 = n2 / d;
-    d3 = n3 / d;
-  }
-  rl = clip(r, d0, d1);
-  rr = clip(r, d2, d3);
-}
-
 // RN(1/x) for 2^-60 <= |x| <= 2^64: the steps of HIP's IEEE division 1/x
 // (reciprocal estimate, one Newton step, quotient and two residual
 // corrections) without the operand scaling and result fix-up, which do
@@ -129,11 +115,6 @@ __device__ __forceinline__ bool tri_finish(V3 o, V3 d, V3 v1, V3 e1, V3 e2, V3 P
   return !(det < kEpsilon) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !(u + v > 1.0f);
 }
 
-struct TraceResult {
-  int32_t id;
-  float t, u, v;
-};
-
 // Traversal counters of the reference's loop: popped = states popped with an
 // in-range index (P), passed = states whose slab test passed (S).  Exact for
 // closest-hit traversal, where every pushed state is eventually popped.
@@ -141,18 +122,30 @@ struct TraceCount {
   uint32_t popped = 0, passed = 0;
 };
 
+// Node indices are kept 1-based (K = k + 1: children 2K and 2K + 1, sibling
+// K ^ 1, ancestor by shift) and depths one-hot (depth d: 1 << d), so that the
+// axis and a pending entry's depth are bit tests.
 struct Trav {
   V3 o, d, y;      // origin, direction, RN(1/direction)
-  uint32_t fast;   // bit a: 2^-60 <= |d_a| <= 16 and normal_coord(o_a)
+  float dmax;      // largest |direction component|; NaN: no reject test for this ray
+  uint32_t fast;   // bit m: the children of a node at depth m take the reciprocal quotient
   float t, u, v;   // current closest hit (t = ray.t)
   int32_t id;
-  uint32_t k, depth, trail;
-  uint32_t axis;   // depth % 3
+  uint32_t K, depth;  // node, one-hot depth
+  uint32_t trail;  // depths with a pending entry
+  uint32_t top;    // stack position (units of the stack)
+  uint32_t cand;   // triangles of the node still to test exactly (bits 0, 1), kStop, kPop
   bool any;        // any-hit query (persistent_trace's mixed launches)
-  float2 r;        // range of node k after its slab test
+  float2 r;        // range of the node after its slab test
+  float4 slab;     // the node's children's slabs
+  uint32_t flags;  // the node's scale_b
 };
-
-__device__ __forceinline__ float compf(V3 v, int a) { return a == 0 ? v.x : (a == 1 ? v.y : v.z); }
+// kStop: an any hit is found; kPop: the node is done, the next pending entry
+// is to be taken.
+constexpr uint32_t kCand = 3u, kStop = 4u, kPop = 8u;
+// Depths whose children's axis (depth + 1) % 3 is x, y, z.
+constexpr uint32_t kChildX = 0x24924924u, kChildY = 0x49249249u, kChildZ = 0x92492492u;
+constexpr uint32_t kExactShare = 5u;  // exact tests run once candidates wait in a fifth of the active lanes
 
 // Per-lane stack of deferred ranges.  A deferred child is always deeper
 // than every entry already pending (entries sit on the current path's
@@ -160,12 +153,19 @@ __device__ __forceinline__ float compf(V3 v, int a) { return a == 0 ? v.x : (a =
 // sorted by depth and entry i is at index i = popcount(trail) at push time:
 // at most levels - 1 entries, indices <= levels - 2.
 //
-// LdsStack: every row in LDS (lane-strided, conflict-free).
+// LdsStack: every row in LDS (lane-strided, conflict-free); the state's top
+// is the number of entries in 8-byte units of the row stride.
 struct LdsStack {
   float2* lds;  // row r of this lane at lds[r * stride]
   uint32_t stride;
-  __device__ __forceinline__ void store(uint32_t r, float2 v) const { lds[r * stride] = v; }
-  __device__ __forceinline__ float2 load(uint32_t r) const { return lds[r * stride]; }
+  __device__ __forceinline__ void push(uint32_t& top, float2 v) const {
+    lds[top] = v;
+    top += stride;
+  }
+  __device__ __forceinline__ float2 pop(uint32_t& top) const {
+    top -= stride;
+    return lds[top];
+  }
 };
 
 // SplitStack: rows [0, klds) in LDS, deeper rows in a per-lane column of
@@ -185,14 +185,16 @@ struct SplitStack {
   uint32_t lane_bytes;     // byte offset of glb from the buffer start
   uint32_t gstride;
   uint32_t klds;
-  __device__ __forceinline__ void store(uint32_t r, float2 v) const {
+  __device__ __forceinline__ void push(uint32_t& top, float2 v) const {
     const vf2 w = {v.x, v.y};
+    const uint32_t r = top++;
     if (r < klds)
       lds[r * lstride] = w;
     else
       glb[(size_t)(r - klds) * gstride] = w;
   }
-  __device__ __forceinline__ float2 load(uint32_t r) const {
+  __device__ __forceinline__ float2 pop(uint32_t& top) const {
+    const uint32_t r = --top;
     if (r < klds) {
       const vf2 w = lds[r * lstride];
       return make_float2(w.x, w.y);
@@ -207,16 +209,35 @@ __device__ __forceinline__ LdsStack lds_stack(float2* lane_column, uint32_t stri
   return LdsStack{lane_column, stride};
 }
 
-__device__ __forceinline__ uint32_t fast_axis(float o, float d) {
+// The reciprocal quotient's range.  (An origin below 2^57 keeps the slabs of
+// missing children, kNoSlab, beyond any range.)
+__device__ __forceinline__ bool fast_axis(float o, float d) {
   const float a = fabsf(d);
-  return (uint32_t)((a >= 0x1p-60f) & (a <= 16.0f) & normal_coord(o));
+  const bool normal = normal_coord(o);
+  return (a >= 0x1p-60f) & (a <= 16.0f) & normal & (fabsf(o) <= 0x1p57f);
+}
+
+// The tree a lane traverses: node records, the triangles' vertices in tree
+// order, the node count and the root's own slab (cslab[0..1] of the record
+// after the last node).
+struct TreeRef {
+  const NodeRec* nodes;
+  const float* tris;
+  uint32_t n_nodes;
+  float2 root;
+};
+
+// dmax of a ray, or NaN when the reject test's bounds do not cover it.
+__device__ __forceinline__ float reject_dmax(V3 o, V3 d) {
+  const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+  const float c = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+  const float all = ((d.x + d.y) + d.z) + ((o.x + o.y) + o.z);  // NaN if any is
+  return ((m >= kRejectDirMin) & (m <= kRejectDirMax) & (c <= kRejectCoord) & (all == all)) ? m : __builtin_nanf("");
 }
 
 // The root's own slab: cslab[0..1] of the record after the last node.
-__device__ __forceinline__ float2 root_slab(const NodeRec* __restrict__ nodes, uint32_t n_nodes,
-                                            uint32_t rec_bytes) {
-  const float4 rs = reinterpret_cast<const float4*>(node_at(nodes, n_nodes, rec_bytes))[4];
-  return make_float2(rs.z, rs.w);
+__device__ __forceinline__ float2 root_slab(const NodeRec* __restrict__ nodes, uint32_t n_nodes) {
+  return make_float2(nodes[n_nodes].cslab[0], nodes[n_nodes].cslab[1]);
 }
 
 // Sets up a ray; returns false when the root's slab culls it (finished, miss).
@@ -231,140 +252,230 @@ __device__ __forceinline__ bool trav_init_root(Trav& s, float2 root, V3 o, V3 d,
   // keep the reciprocals in registers: without this barrier the compiler
   // re-derives them at every use inside the loop
   __asm__ volatile("" : "+v"(s.y.x), "+v"(s.y.y), "+v"(s.y.z));
-  s.fast = fast_axis(o.x, d.x) | (fast_axis(o.y, d.y) << 1) | (fast_axis(o.z, d.z) << 2);
+  const bool fx = fast_axis(o.x, d.x), fy = fast_axis(o.y, d.y), fz = fast_axis(o.z, d.z);
+  s.fast = (fx ? kChildX : 0u) | (fy ? kChildY : 0u) | (fz ? kChildZ : 0u);
+  s.dmax = reject_dmax(o, d);
   s.t = tmax;
   s.u = s.v = 0.0f;
   s.id = -1;
-  s.k = s.depth = s.trail = s.axis = 0;
+  s.K = s.depth = 1;
+  s.trail = s.top = s.cand = 0;
   s.any = false;
   if (kCount) cnt->popped += 1;  // the root
-  s.r = narrow(make_float2(kEpsilon, kInfinity), root.x, root.y, o.x, d.x, s.y.x, s.fast & 1u);
+  s.r = narrow(make_float2(kEpsilon, kInfinity), root.x, root.y, o.x, d.x, s.y.x, fx);
   return (s.r.x <= s.r.y) && (s.r.x <= s.t);
 }
 
 template <bool kCount>
-__device__ __forceinline__ bool trav_init(Trav& s, const NodeRec* __restrict__ nodes,
-                                          uint32_t n_nodes, uint32_t rec_bytes, V3 o, V3 d,
-                                          float tmax, TraceCount* cnt) {
-  return trav_init_root<kCount>(s, root_slab(nodes, n_nodes, rec_bytes), o, d, tmax, cnt);
+__device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3 d, float tmax,
+                                          TraceCount* cnt) {
+  return trav_init_root<kCount>(s, root_slab(tree.nodes, tree.n_nodes), o, d, tmax, cnt);
 }
 
-// Visits node s.k; returns true when the traversal has finished.  All paths
-// (take a child, resume a deferred child, finish) leave through one exit and
-// the next node is chosen by selects: with several early exits the compiler's
-// structured control flow ran the node visit separately for lanes arriving
-// from different paths, doubling the instructions issued per visit.
-// kMixed: the query kind is the lane's s.any instead of kAny.
-template <bool kAny, bool kCount, bool kMixed = false, class Stk>
-__device__ __forceinline__ bool trav_step(Trav& s, const NodeRec* __restrict__ nodes,
-                                          uint32_t n_nodes, uint32_t rec_bytes, const Stk& stk,
-                                          TraceCount* cnt) {
-  const bool any = kAny || (kMixed && s.any);
-  const uint32_t k = s.k;
+// ---- the reject test ----
+//
+// Loads the node's record and leaves in s.cand the triangles that may pass
+// the reference's test.  Two things bound a visit when every lane reads
+// another node: VALU issue and the vector L1, which looks up one lane's 16
+// bytes per cycle and CU.  Both triangles' exact test took 125 VALU
+// instructions and a 96-byte record 6 loads; this test takes 90 and the
+// 64-byte record 4, and what it leaves over (1.2% of the visits at 1M
+// triangles) costs 6 more per visit.  With the visit's second half
+// (trav_next) rewritten at the same time: 2^24 incoherent rays into 1M
+// triangles 7.28 -> 5.72 ms (3.63e9 -> 2.81e9 VALU instructions, L1 lookups
+// 4.43e9 -> 3.00e9), 2^21 into 10M triangles 6.48 -> 5.97 ms, a 1080p frame
+// of 8 samples over 1M triangles 41.2 -> 37.0 ms.
+//
+// With T = p - v1 for any point p of the ray's line and C = T x d, the
+// Moller-Trumbore numerators are u det = e2 . C, v det = -(e1 . C) and
+// det = -d . (e1 x e2); the reference's test accepts only if none of the
+// three edge functions u det, v det and (1 - u - v) det is negative (but for
+// rounding).  p is the ray's entry into the node's range, so that T is no
+// larger than the node's group, and lengths are in units of the group's size.
+//
+// Bound.  D = dmax, z = the triangle's size (each |e| component <= z),
+// q = 2^-11 + 2^-15, t = the range's entry.
+//   edges: rounding to half moves a component by at most q z (2^-11 relative,
+//     2^-25 absolute, z >= 2^-10);
+//   T: off by at most 2^-12 (dv, |dv| <= 1) + 2^-15 (roundings of dv and T,
+//     |T| <= 4) + 2^-24 scale |p|max (one fma for p); C by 2 D times that and
+//     2^-22 D;
+//   u det, v det: z (3 q |C|max + D (6.82 2^-12 + 6 2^-24 scale |p|max));
+//   det: e1 x e2 in half, 3 D ((4.01 q + 3 2^-11) z^2 + 2^-24);
+//   the reference's floats: 36 2^-24 z D scale |o - v1|max per numerator
+//     (T, P or Q and the dot product), scale |o - v1|max <= scale t D + 5.
+// So a triangle that the reference accepts has, with
+//   thr = A |C|max + 3.4 A z D + D (B + 2^-18 scale (t D + |p|max)),
+// u det >= -z thr, v det >= -z thr and (1 - u - v) det >= -2 z thr:
+// A = 1.6e-3 >= 3 q = 1.557e-3; half the third function's error is that of
+// one numerator plus z D 5.32e-3 z, below 3.4 A z = 5.44e-3 z, plus 0.38 2^-12
+// z D, and B = 8 2^-12 >= (6.82 + 0.38) 2^-12 with a margin for the float
+// roundings of this test itself (below 2^-18 z D).
+// Comparisons are written so that NaN and infinity keep a triangle.
+constexpr float kRejA = 1.6e-3f, kRejA2 = 3.4f * 1.6e-3f, kRejB = 0x1p-9f, kRejC = 0x1p-18f;
+
+__device__ __forceinline__ float lo16(half2v h) { return (float)h.x; }
+__device__ __forceinline__ float hi16(half2v h) { return (float)h.y; }
+__device__ __forceinline__ float max3abs(float a, float b, float c) {
+  return fmaxf(fmaxf(fabsf(a), fabsf(b)), fabsf(c));
+}
+
+// Whether the triangle may be accepted: T = p - v1, edges e1 and e2, size, det
+// (all scaled); base = D (B + 2^-18 scale (t D + |p|max)).
+__device__ __forceinline__ bool may_hit(V3 T, V3 d, V3 e1, V3 e2, float det, float size, float dmax, float base) {
+  const float cx = __builtin_fmaf(T.y, d.z, -(T.z * d.y));
+  const float cy = __builtin_fmaf(T.z, d.x, -(T.x * d.z));
+  const float cz = __builtin_fmaf(T.x, d.y, -(T.y * d.x));
+  const float un = __builtin_fmaf(e2.z, cz, __builtin_fmaf(e2.y, cy, __builtin_fmaf(e2.x, cx, 0.0f)));
+  const float vn = __builtin_fmaf(-e1.z, cz, __builtin_fmaf(-e1.y, cy, __builtin_fmaf(-e1.x, cx, 0.0f)));
+  const float wn = 0.5f * (det - un - vn);
+  const float m = fminf(fminf(un, vn), wn);
+  const float thr = __builtin_fmaf(max3abs(cx, cy, cz), kRejA,
+                                   __builtin_fmaf(__builtin_fmaf(size, dmax, 0.0f), kRejA2, base));
+  return !(__builtin_fmaf(size, thr, m) < 0.0f);
+}
+
+template <bool kCount>
+__device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCount* cnt) {
   if (kCount) {
     cnt->passed += 1;
-    cnt->popped += (2 * k + 1 < n_nodes) + (2 * k + 2 < n_nodes);
+    cnt->popped += (2 * s.K <= tree.n_nodes) + (2 * s.K + 1 <= tree.n_nodes);
   }
-  // the whole record in one round of loads (the right child's slab too, used
-  // only when the node has two children: a load issued inside that branch
-  // would wait a second memory latency per visit)
-  const float4* rec = reinterpret_cast<const float4*>(node_at(nodes, k, rec_bytes));
-  const float4 a0 = rec[0], a1 = rec[1], a2 = rec[2], a3 = rec[3], a4 = rec[4];
-  const float4 a5 = rec[5];  // right child's slab, flags
-  // both triangles up to their determinants, then both reciprocals
-  const V3 v1a = mk(a0.x, a0.y, a0.z), e1a = mk(a0.w, a1.x, a1.y), e2a = mk(a1.z, a1.w, a2.x);
-  const V3 v1b = mk(a2.y, a2.z, a2.w), e1b = mk(a3.x, a3.y, a3.z), e2b = mk(a3.w, a4.x, a4.y);
-  const V3 Pa = cross(s.d, e2a), Pb = cross(s.d, e2b);
-  const float deta = dot(e1a, Pa), detb = dot(e1b, Pb);
-  float ia = recip_rn(deta), ib = recip_rn(detb);
-  if ((deta > kRecipMax) | (detb > kRecipMax)) {
-    ia = deta > kRecipMax ? 1.0f / deta : ia;
-    ib = detb > kRecipMax ? 1.0f / detb : ib;
-  }
-  float ua, va, ta, ub, vb, tb;
-  const bool hita = tri_finish(s.o, s.d, v1a, e1a, e2a, Pa, deta, ia, ua, va, ta) &
-                    (ta > kEpsilon) & (ta < s.t);
-  if (hita) {
-    s.t = ta;
-    s.u = ua;
-    s.v = va;
-    s.id = (int32_t)(2 * k);
-  }
-  const bool hitb = tri_finish(s.o, s.d, v1b, e1b, e2b, Pb, detb, ib, ub, vb, tb) &
-                    (tb > kEpsilon) & (tb < s.t) & !(any & hita);
-  if (hitb) {
-    s.t = tb;
-    s.u = ub;
-    s.v = vb;
-    s.id = (int32_t)(2 * k + 1);
-  }
-  const bool stop = any & (hita | hitb);  // any hit found
-  bool found = false;
-  uint32_t nk = 0, nd = 0, na = 0;
-  float2 nrg = s.r;
-  const uint32_t cl = 2 * k + 1;
-  if (!stop && cl < n_nodes) {
-    const uint32_t cd = s.depth + 1;
-    const int ca = s.axis == 2 ? 0 : (int)s.axis + 1;
-    const float oc = compf(s.o, ca), dc = compf(s.d, ca), yc = compf(s.y, ca);
-    const bool fast = ((s.fast >> ca) & __float_as_uint(a5.z) & kNodeSlabsNormal) != 0u;
-    float2 rl, rr;
-    narrow2(s.r, make_float4(a4.z, a4.w, a5.x, a5.y), oc, dc, yc, fast, rl, rr);
-    const bool okl = rl.x <= rl.y;
-    const bool okr = (cl + 1 < n_nodes) & (rr.x <= rr.y);
-    const bool sw = dc < 0.0f;
-    const float2 near_r = sw ? rr : rl, far_r = sw ? rl : rr;
-    // lane-mask logic rather than selects of booleans
-    const bool nok = (sw & okr) | (!sw & okl), fok = (sw & okl) | (!sw & okr);
-    const bool take_near = nok & (near_r.x <= s.t);
-    const bool take_far = !take_near & fok & (far_r.x <= s.t);
-    if (take_near && fok) {
-      stk.store((uint32_t)__popc(s.trail), far_r);
-      s.trail |= 1u << cd;
-    }
-    found = take_near || take_far;
-    nk = (take_near != sw) ? cl : cl + 1;  // near = cl unless swapped; far is the other
-    nrg = take_near ? near_r : far_r;
-    nd = cd;
-    na = (uint32_t)ca;
-  }
-  if (!stop && !found) {
-    while (s.trail) {
-      const uint32_t dd = 31u - (uint32_t)__clz(s.trail);
-      const float2 frv = stk.load((uint32_t)__popc(s.trail) - 1u);
-      // both halves in one LDS read (else the second is issued after the
-      // test and the next step's loads wait for it)
-      float fx = frv.x, fy = frv.y;
-      __asm__ volatile("" : "+v"(fx), "+v"(fy));
-      const float2 fr = make_float2(fx, fy);
-      s.trail &= ~(1u << dd);
-      if (fr.x <= s.t) {
-        const uint32_t anc = ((k + 1) >> (s.depth - dd)) - 1;
-        nk = (anc & 1u) ? anc + 1 : anc - 1;
-        nd = dd;
-        na = dd % 3;
-        nrg = fr;
-        found = true;
-        break;
-      }
-    }
-  }
-  s.k = nk;
-  s.depth = nd;
-  s.axis = na;
-  s.r = nrg;
-  return !found;
+  const uint4* rec = reinterpret_cast<const uint4*>(tree.nodes + s.K - 1);
+  const uint4 a0 = rec[0], a1 = rec[1], a2 = rec[2], a3 = rec[3];
+  s.slab = make_float4(__uint_as_float(a0.x), __uint_as_float(a0.y), __uint_as_float(a0.z), __uint_as_float(a0.w));
+  s.flags = a1.w;
+  const auto h2 = [](uint32_t x) { return __builtin_bit_cast(half2v, x); };
+  const half2v e1x = h2(a2.x), e1y = h2(a2.y), e1z = h2(a2.z), e2x = h2(a2.w), e2y = h2(a3.x), e2z = h2(a3.y);
+  const half2v dxy = h2(a3.z), dza = h2(a3.w), szb = h2(a1.w);
+  const float scale = __uint_as_float(a1.w & 0xFF800000u);
+  const V3 d = s.d;
+  const V3 p = mk(__builtin_fmaf(s.r.x, d.x, s.o.x), __builtin_fmaf(s.r.x, d.y, s.o.y),
+                  __builtin_fmaf(s.r.x, d.z, s.o.z));
+  const V3 Ta = mk(__builtin_fmaf(p.x, scale, -__uint_as_float(a1.x)), __builtin_fmaf(p.y, scale, -__uint_as_float(a1.y)),
+                   __builtin_fmaf(p.z, scale, -__uint_as_float(a1.z)));
+  const V3 Tb = mk(__builtin_fmaf(lo16(dxy), -1.0f, Ta.x), __builtin_fmaf(hi16(dxy), -1.0f, Ta.y),
+                   __builtin_fmaf(lo16(dza), -1.0f, Ta.z));
+  const float reach = __builtin_fmaf(s.r.x, s.dmax, max3abs(p.x, p.y, p.z)) * scale;
+  const float base = __builtin_fmaf(reach, kRejC, kRejB) * s.dmax;
+  // e1 x e2 of both triangles at once
+  const half2v nx = __builtin_elementwise_fma(e1y, e2z, -(e1z * e2y));
+  const half2v ny = __builtin_elementwise_fma(e1z, e2x, -(e1x * e2z));
+  const half2v nz = __builtin_elementwise_fma(e1x, e2y, -(e1y * e2x));
+  const float deta = __builtin_fmaf(-lo16(nz), d.z, __builtin_fmaf(-lo16(ny), d.y, __builtin_fmaf(-lo16(nx), d.x, 0.0f)));
+  const float detb = __builtin_fmaf(-hi16(nz), d.z, __builtin_fmaf(-hi16(ny), d.y, __builtin_fmaf(-hi16(nx), d.x, 0.0f)));
+  const bool ca = may_hit(Ta, d, mk(lo16(e1x), lo16(e1y), lo16(e1z)), mk(lo16(e2x), lo16(e2y), lo16(e2z)), deta,
+                          hi16(dza), s.dmax, base);
+  const bool cb = may_hit(Tb, d, mk(hi16(e1x), hi16(e1y), hi16(e1z)), mk(hi16(e2x), hi16(e2y), hi16(e2z)), detb,
+                          lo16(szb), s.dmax, base);
+  const bool far = !(max3abs(Ta.x, Ta.y, Ta.z) <= 4.0f);
+  s.cand = (uint32_t)(ca | far) | ((uint32_t)(cb | far) << 1);
 }
 
-// The tree a lane traverses: node records, their count, the root's own
-// slab (cslab[0..1] of the record after the last node) and the distance
-// between records.
-struct TreeRef {
-  const NodeRec* nodes;
-  uint32_t n_nodes;
-  float2 root;
-  uint32_t rec_bytes;
-};
+// The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of the
+// first candidate of the node, on the vertices it was uploaded with.
+template <bool kAny, bool kMixed = false>
+__device__ __forceinline__ void trav_exact(Trav& s, const float* __restrict__ tris) {
+  const uint32_t tri = 2 * s.K - 1u - (s.cand & 1u);
+  const float* p = tris + (size_t)tri * 9;  // points layout: x1 x2 x3 y1 y2 y3 z1 z2 z3
+  const V3 v1 = mk(p[0], p[3], p[6]);
+  const V3 e1 = mk(p[1], p[4], p[7]) - v1, e2 = mk(p[2], p[5], p[8]) - v1;
+  s.cand &= s.cand - 1u;
+  const V3 P = cross(s.d, e2);
+  const float det = dot(e1, P);
+  float inv = recip_rn(det);
+  if (det > kRecipMax) inv = 1.0f / det;
+  float u, v, t;
+  const bool hit = tri_finish(s.o, s.d, v1, e1, e2, P, det, inv, u, v, t) & (t > kEpsilon) & (t < s.t);
+  if (hit) {
+    s.t = t;
+    s.u = u;
+    s.v = v;
+    s.id = (int32_t)tri;
+    if (kAny || (kMixed && s.any)) s.cand = kStop;
+  }
+}
+
+// Leaves the node (no candidates left) for the next one; returns true when
+// the traversal has finished.  The near child is taken directly, the far one
+// deferred; without a child to take, one pending entry is popped, and if its
+// range now starts beyond the closest hit the lane keeps kPop and pops again
+// in the next step (1.8% of the steps at 1M triangles; an inner loop until an
+// entry passes made every lane of the wave wait through its iterations).
+template <class Stk>
+__device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& stk) {
+  const bool ax = (s.depth & kChildX) != 0u, ay = (s.depth & kChildY) != 0u;
+  // by value: a select of members would keep the state in memory
+  const auto pick = [](bool c, float a, float b) { return c ? a : b; };
+  const float oc = pick(ax, s.o.x, pick(ay, s.o.y, s.o.z));
+  const float dc = pick(ax, s.d.x, pick(ay, s.d.y, s.d.z));
+  const float yc = pick(ax, s.y.x, pick(ay, s.y.y, s.y.z));
+  // the near child and each child's entry plane by the direction's sign: the
+  // quotients of a slab's planes are ordered as the planes are (rounded
+  // division is monotonic), so fminf / fmaxf of them are selections
+  const bool sw = dc < 0.0f;
+  const float n0 = pick(sw, s.slab.w, s.slab.x) - oc, n1 = pick(sw, s.slab.z, s.slab.y) - oc;
+  const float n2 = pick(sw, s.slab.y, s.slab.z) - oc, n3 = pick(sw, s.slab.x, s.slab.w) - oc;
+  float nx = quot_fast(n0, dc, yc), ny = quot_fast(n1, dc, yc);
+  float fx = quot_fast(n2, dc, yc), fy = quot_fast(n3, dc, yc);
+  const uint32_t normal = (uint32_t)((int32_t)(s.flags << 15) >> 31);  // kNodeSlabsNormal as a mask
+  if ((s.fast & s.depth & normal) == 0u) {
+    // true division, with the reference's fminf / fmaxf (NaN, division by 0)
+    const float a = n0 / dc, b = n1 / dc, c = n2 / dc, e = n3 / dc;
+    nx = min_q(a, b);
+    ny = max_q(a, b);
+    fx = min_q(c, e);
+    fy = max_q(c, e);
+    const bool left = 2 * s.K <= n_nodes, right = 2 * s.K < n_nodes;  // which children exist
+    if (!(sw ? right : left)) nx = __builtin_inff();
+    if (!(sw ? left : right)) fx = __builtin_inff();
+  }
+  nx = max_q(nx, s.r.x);
+  ny = min_q(ny, s.r.y);
+  fx = max_q(fx, s.r.x);
+  fy = min_q(fy, s.r.y);
+  const bool live = s.cand == 0u;
+  const bool far = live & (fx <= fy);
+  const bool take_near = live & (nx <= ny) & (nx <= s.t);
+  const bool take_far = !take_near & far & (fx <= s.t);
+  if (take_near & far) {
+    stk.push(s.top, make_float2(fx, fy));
+    s.trail |= s.depth << 1;
+  }
+  if (take_near | take_far) {
+    s.K = 2 * s.K + (uint32_t)(sw ^ take_far);
+    s.depth <<= 1;
+    s.r = make_float2(take_near ? nx : fx, take_near ? ny : fy);
+    return false;
+  }
+  if ((s.trail == 0u) | ((s.cand & kStop) != 0u)) return true;
+  const float2 e = stk.pop(s.top);
+  const uint32_t z = (uint32_t)__builtin_clz(s.trail);
+  const uint32_t bit = 0x80000000u >> z;
+  s.trail ^= bit;
+  // the entry is the sibling of the path's node at its depth
+  s.K = (s.K >> (z - (uint32_t)__builtin_clz(s.depth))) ^ 1u;
+  s.depth = bit;
+  s.r = e;
+  s.cand = e.x <= s.t ? 0u : kPop;
+  return false;
+}
+
+// Lane mask of a condition, without materialising it as an integer.
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// One step of a persistent wave; returns true in lanes whose traversal has
+// finished.  Lanes whose node left candidates wait until they are a fifth of
+// the active lanes (or all of them): the exact test costs nearly a visit's
+// instructions for however few lanes run it.
+template <bool kAny, bool kMixed, class Stk>
+__device__ __forceinline__ bool trav_visit(Trav& s, const TreeRef& tree, const Stk& stk, bool active) {
+  if (active && s.cand == 0u) trav_test<false>(s, tree, nullptr);
+  const bool pending = active && (s.cand & kCand);
+  const uint32_t np = (uint32_t)__popcll(ballot(pending));
+  if (np * kExactShare >= (uint32_t)__popcll(ballot(active)) && pending) trav_exact<kAny, kMixed>(s, tree.tris);
+  return active && !(s.cand & kCand) && trav_next(s, tree.n_nodes, stk);
+}
 
 // Persistent-wave traversal of a work range [0, n) of closest-hit and
 // any-hit queries.  Wave w owns [w*chunk, (w+1)*chunk); between node visits,
@@ -392,7 +503,7 @@ __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint
   bool active = false;
   uint64_t item = 0;
   for (;;) {
-    const uint64_t idle = __ballot(!active);
+    const uint64_t idle = ballot(!active);
     const uint32_t nidle = __popcll(idle);
     if (nidle >= refill || nidle == 64) {
       if (next < end) {
@@ -415,27 +526,24 @@ __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint
         break;
       }
     }
-    if (active && trav_step<false, false, true>(s, tree.nodes, tree.n_nodes, tree.rec_bytes, stk, nullptr)) {
+    if (trav_visit<false, true>(s, tree, stk, active)) {
       store(item, s);
       active = false;
     }
   }
 }
 
-// Whole traversal of one ray by one lane (used by the render kernels).
+// Whole traversal of one ray by one lane.
 // stk: this lane's stack column, stk[depth * stride].
 template <bool kAny, bool kCount = false>
-__device__ __forceinline__ TraceResult trace_ray(const NodeRec* __restrict__ nodes, uint32_t n_nodes,
-                                                 uint32_t rec_bytes, V3 o, V3 d, float tmax,
-                                                 float2* stk, uint32_t stride,
-                                                 TraceCount* cnt = nullptr) {
-  Trav s;
+__device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3 d, float tmax, float2* stk,
+                                          uint32_t stride, TraceCount* cnt = nullptr) {
   const LdsStack st = lds_stack(stk, stride);
-  if (trav_init<kCount>(s, nodes, n_nodes, rec_bytes, o, d, tmax, cnt)) {
-    while (!trav_step<kAny, kCount>(s, nodes, n_nodes, rec_bytes, st, cnt)) {
-    }
-  }
-  return TraceResult{s.id, s.t, s.u, s.v};
+  if (!trav_init<kCount>(s, tree, o, d, tmax, cnt)) return;
+  do {
+    if (s.cand == 0u) trav_test<kCount>(s, tree, cnt);
+    while (s.cand & kCand) trav_exact<kAny>(s, tree.tris);
+  } while (!trav_next(s, tree.n_nodes, st));
 }
 
 }  // namespace aur
