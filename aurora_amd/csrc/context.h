@@ -99,10 +99,12 @@ constexpr uint32_t kDefaultMaxPaths = 1u << 24;
 constexpr uint32_t kDefaultRenderRefill = 16;
 constexpr uint32_t kDefaultRenderStackRows = 12;
 // Frame counters (u32): three 64-bit queue-count words of the wavefront
-// passes, then two u64 ray counters (camera + extension, shadow) at
-// kStatsOffset.
+// passes, two u64 ray counters (camera + extension, shadow) at kStatsOffset,
+// and the work counters (kWorkWords) of the trace launches that use each word.
 constexpr uint32_t kStatsOffset = 8;
-constexpr uint32_t kCounterWords = 12;
+constexpr uint32_t kWorkWords = 8 * 32;
+constexpr uint32_t kTicketOffset = 32;
+constexpr uint32_t kCounterWords = kTicketOffset + 3 * kWorkWords;
 
 // One render job of the PBR wavefront: a camera over one built scene.  A
 // frame render is a single job; a batch is many.  Paths are numbered
@@ -191,6 +193,7 @@ struct aur_context {
   // limited residency: fastest shape measured at 1M triangles / 2^24 rays
   aur_trace_params trace_params{1, 256, 24, 0, 0};
   aur::DevBuf<float2> gstack;  // global rows of the persistent traversal stack
+  aur::DevBuf<uint32_t> trace_work;  // work counters of the persistent trace launches
   float2 root_slab = make_float2(0.0f, 0.0f);  // host copy of the built tree's root slab
   aur_render_params render_params{aur::kDefaultMaxPaths, 0, aur::kDefaultRenderRefill,
                                   aur::kDefaultRenderStackRows};

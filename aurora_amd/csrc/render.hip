@@ -31,6 +31,7 @@ namespace aur {
 namespace {
 
 constexpr int kBlock = 128;
+static_assert(kWorkWords == kWorkGroups * kWorkStride, "work counters");
 
 struct SceneDev {
   const NodeRec* nodes;
@@ -275,6 +276,7 @@ __global__ void k_pbr_camera(PbrArgs a, uint32_t* __restrict__ queue) {
     a.counters[0] = n;
     a.counters[1] = 0;
   }
+  if (q < kWorkWords) a.counters[kTicketOffset + q] = 0;
   if (q >= n) return;
   const unsigned long long g = g0 + q;
   uint32_t jb = 0;
@@ -344,9 +346,12 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
     atomicAdd(&a.stats[0], (unsigned long long)n_ext);
     atomicAdd(&a.stats[1], (unsigned long long)n_sh);
   }
-  persistent_trace(
+  if (blockIdx.x == 0)
+    for (uint32_t i = threadIdx.x; i < kWorkWords; i += blockDim.x)
+      a.counters[kTicketOffset + (w == 2u ? 0u : w + 1u) * kWorkWords + i] = 0;
+  persistent_trace<false, true>(
       TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, a.job.root}, (uint64_t)n_ext + n_sh,
-      a.refill, stack,
+      a.counters + kTicketOffset + w * kWorkWords, a.refill, stack,
       [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef& tree, bool& any) {
         float4 o4, d4;
         uint32_t jb = 0;
@@ -370,7 +375,6 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
         o = mk(o4.x, o4.y, o4.z);
         d = mk(d4.x, d4.y, d4.z);
         tmax = o4.w;
-        return true;
       },
       [&](uint64_t i, const Trav& st) {
         if (i < n_ext)
@@ -905,6 +909,7 @@ __global__ void k_cw_init(CwArgs c, PbrArgs a, uint32_t* __restrict__ qin) {
     a.counters[0] = c.n;
     a.counters[1] = 0;
   }
+  if (l < kWorkWords) a.counters[kTicketOffset + l] = 0;
   if (l >= c.n) return;
   const uint32_t rl = c.l0 + l % c.nchunk;
   const uint32_t x = c.region.x + rl % c.region.z, y = c.region.y + rl / c.region.z;

@@ -1,8 +1,8 @@
 // Standalone traversal launches (src/kernels/lib/intersect.cuh:36-152).
 //
-// k_trace_pt: persistent waves (trace_rays below): each wave owns a
-// contiguous range of rays and refills idle lanes from it, so lanes whose
-// rays finish early do not idle until the slowest ray of the wave ends.
+// k_trace_pt: persistent waves (trace_rays below): a wave refills idle lanes
+// from its range of rays, so lanes whose rays finish early do not idle until
+// the slowest ray of the wave ends, and takes further ranges from a counter.
 // Each lane keeps its deferred ranges in an LDS column of levels - 1 float2
 // entries (or the first rows in LDS and the rest in global memory).
 //
@@ -28,52 +28,26 @@ __device__ __forceinline__ void store_result(uint64_t i, const Trav& s, aur_hit*
     reinterpret_cast<float4*>(hits)[i] = make_float4(__int_as_float(s.id), s.t, s.u, s.v);
 }
 
-// Persistent traversal of rays [0, n) with the refill of persistent_trace;
-// the tree is wave-uniform, so its root slab is read once per wave and a
-// refill waits on the ray loads only.  (Keeping the next 64 rays in
-// registers and handing them out by lane permutes measured slower: the
-// permutes' register reuse makes every refill wait for them.)
+// Persistent traversal of rays [0, n); the tree is wave-uniform, so its root
+// slab is read once per wave and a refill waits on the ray loads only.
+// (Keeping the next 64 rays in registers and handing them out by lane
+// permutes measured slower: the permutes' register reuse makes every refill
+// wait for them.)
 template <bool kAny, class Stk>
 __device__ __forceinline__ void trace_rays(TreeRef tree, const aur_ray* __restrict__ rays, uint64_t n,
-                                           uint32_t refill, const Stk& stk,
-                                           aur_hit* __restrict__ hits, int32_t* __restrict__ ids) {
-  const uint64_t waves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-  const uint64_t chunk = (n + waves - 1) / waves;
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  uint64_t next = wave * chunk;
-  const uint64_t end = next + chunk < n ? next + chunk : n;
-  const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-  const float2 root = root_slab(tree.nodes, tree.n_nodes);  // once per wave
-  Trav s;
-  bool active = false;
-  uint64_t item = 0;
-  for (;;) {
-    const uint64_t idle = ballot(!active);
-    const uint32_t nidle = __popcll(idle);
-    if (nidle >= refill || nidle == 64) {
-      if (next < end) {
-        if (!active) {
-          const uint64_t i = next + __popcll(idle & lt);
-          if (i < end) {
-            const float4* r = reinterpret_cast<const float4*>(rays + i);
-            const float4 a = r[0], b = r[1];
-            item = i;
-            active = trav_init_root<false>(s, root, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w,
-                                           nullptr);
-            if (!active) store_result(i, s, hits, ids);
-          }
-        }
-        next += nidle;
-      } else if (nidle == 64) {
-        break;
-      }
-    }
-    if (trav_visit<kAny, false>(s, tree, stk, active)) {
-      store_result(item, s, hits, ids);
-      active = false;
-    }
-  }
+                                           uint32_t refill, const Stk& stk, aur_hit* __restrict__ hits,
+                                           int32_t* __restrict__ ids, uint32_t* __restrict__ work) {
+  tree.root = root_slab(tree.nodes, tree.n_nodes);
+  persistent_trace<kAny, false>(
+      tree, n, work, refill, stk,
+      [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef&, bool&) {
+        const float4* r = reinterpret_cast<const float4*>(rays + i);
+        const float4 a = r[0], b = r[1];
+        o = mk(a.x, a.y, a.z);
+        d = mk(b.x, b.y, b.z);
+        tmax = a.w;
+      },
+      [&](uint64_t i, const Trav& s) { store_result(i, s, hits, ids); });
 }
 
 template <bool kAny, bool kSplit>
@@ -81,9 +55,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_trace_pt(const NodeRec* __restric
                                                         const float* __restrict__ tris, uint32_t n_nodes,
                                                         const aur_ray* __restrict__ rays, uint64_t n,
                                                         aur_hit* __restrict__ hits,
-                                                        int32_t* __restrict__ ids, uint32_t refill,
-                                                        float2* __restrict__ gstack, uint32_t klds,
-                                                        uint32_t gstack_rows) {
+                                                        int32_t* __restrict__ ids, uint32_t* __restrict__ work,
+                                                        uint32_t refill, float2* __restrict__ gstack,
+                                                        uint32_t klds, uint32_t gstack_rows) {
   extern __shared__ float2 stk_mem[];
   if constexpr (kSplit) {
     // the first klds stack rows in LDS, deeper ones in global memory (the
@@ -95,10 +69,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_trace_pt(const NodeRec* __restric
                          (glb_vf2*)(gstack + gtid),
                          __builtin_amdgcn_make_buffer_rsrc(gstack, (short)0, (int)bytes, 0x00020000),
                          gtid * 8u, lanes, klds};
-    trace_rays<kAny>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill, stk, hits, ids);
+    trace_rays<kAny>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill, stk, hits, ids, work);
   } else {
     trace_rays<kAny>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill,
-                     lds_stack(stk_mem + threadIdx.x, blockDim.x), hits, ids);
+                     lds_stack(stk_mem + threadIdx.x, blockDim.x), hits, ids, work);
   }
 }
 
@@ -195,6 +169,9 @@ __global__ __launch_bounds__(256) void k_division_check(uint32_t lo, uint32_t hi
   }
 }
 
+// The work counters of the next persistent launch.
+__global__ void k_zero_work(uint32_t* p) { p[threadIdx.x] = 0u; }
+
 template <bool kAny>
 aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_hit* hits,
                         int32_t* ids) {
@@ -221,7 +198,7 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
   if (tp.refill < 1 || tp.refill > 64)
     return ctx->fail(AUR_ERR_INVALID_ARG, "trace: refill must be in 1..64");
   using Kern = void (*)(const NodeRec*, const float*, uint32_t, const aur_ray*, uint64_t, aur_hit*,
-                        int32_t*, uint32_t, float2*, uint32_t, uint32_t);
+                        int32_t*, uint32_t*, uint32_t, float2*, uint32_t, uint32_t);
   const Kern fn = klds != 0 ? k_trace_pt<kAny, true> : k_trace_pt<kAny, false>;
   AUR_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, (int)block, lds_pt));
   if (per_cu < 1) per_cu = 1;
@@ -239,8 +216,14 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
     AUR_HIP(ctx, ctx->gstack.reserve(entries));
     gstack = ctx->gstack.p;
   }
+  // (Clearing the counters in the launch itself, by the last block of each
+  // group, put 128 atomics on one address at its end: 36 us at 2^20 rays.)
+  if (n > (uint64_t)grid * block) {
+    k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(ctx->trace_work.p);
+    AUR_LAUNCH_CHECK(ctx, "k_zero_work");
+  }
   hipLaunchKernelGGL(fn, dim3(grid), dim3(block), lds_pt, ctx->stream, ctx->nodes.p, ctx->vertices.p,
-                     ctx->count / 2, rays, n, hits, ids, tp.refill, gstack, klds, maxrows - rows);
+                     ctx->count / 2, rays, n, hits, ids, ctx->trace_work.p, tp.refill, gstack, klds, maxrows - rows);
   AUR_LAUNCH_CHECK(ctx, "k_trace_pt");
   return AUR_OK;
 }

@@ -370,6 +370,10 @@ __device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCou
                           lo16(szb), s.dmax, base);
   const bool far = !(max3abs(Ta.x, Ta.y, Ta.z) <= 4.0f);
   s.cand = (uint32_t)(ca | far) | ((uint32_t)(cb | far) << 1);
+  // every load has returned here: with the slabs' still in flight on some
+  // path, the next visit's address, in one of their registers, waited for all
+  // outstanding memory operations, stores included
+  __asm__ volatile("" : "+v"(s.slab.x), "+v"(s.slab.y), "+v"(s.slab.z), "+v"(s.slab.w));
 }
 
 // The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of the
@@ -477,57 +481,108 @@ __device__ __forceinline__ bool trav_visit(Trav& s, const TreeRef& tree, const S
   return active && !(s.cand & kCand) && trav_next(s, tree.n_nodes, stk);
 }
 
-// Persistent-wave traversal of a work range [0, n) of closest-hit and
-// any-hit queries.  Wave w owns [w*chunk, (w+1)*chunk); between node visits,
-// once at least `refill` lanes are idle (or all are), idle lanes take the
-// next items of the range, ranked by ballot (no atomics).
+// The items a wave of a persistent launch takes from [0, n): first a range of
+// its own, then chunks from a counter, so that waves whose rays end early take
+// over the work of others.  With one fixed range per wave, a launch lasted as
+// long as its dearest range: 2^21 camera rays, whose ranges see sky or
+// geometry, took 1.00 ms alone, now 0.62 ms; a 256^2 Cornell frame 2.35 ->
+// 2.17 ms; the differentiable step at 512^2 25.1 -> 20.1 ms.  The first range
+// is one ray per lane below 512 rays a wave and half of an even share above; a
+// chunk is a sixteenth of a share, at least one ray per lane (first ranges of
+// 128 and 192 rays, chunks of 128 and first ranges of 3/4 of a share were up
+// to 25% slower on the camera rays).  Launches of at most one first range per
+// wave use no counter.  The blocks form kWorkGroups groups, each with a
+// counter of its own in its own cache line (group g's t-th chunk is chunk
+// t * groups + g): one address takes an atomic about every 12 ns, which
+// bounded launches of short rays (the Cornell frame took 2.68 ms with a
+// single counter).  (Asking for the next ticket ahead and letting a request
+// reach over the end of a chunk was 10% slower on the camera rays.)
+constexpr uint32_t kWorkGroups = 8;
+constexpr uint32_t kWorkStride = 32;  // words between groups' counters
+struct WaveWork {
+  uint64_t next, end;  // the current range
+  uint64_t n, first_total;
+  uint32_t chunk, group, groups;
+  uint32_t* ticket;  // the group's, zero before the launch
+  bool more;         // the counter may have chunks left
+
+  __device__ __forceinline__ WaveWork(uint64_t items, uint32_t* tickets) : n(items) {
+    const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const uint64_t share = n >> 32 ? n / waves : (uint64_t)((uint32_t)n / waves);
+    const uint64_t first = share < 512 ? 64 : (share / 2) & ~63ull;
+    const uint64_t sixteenth = (share / 16 + 63) & ~63ull;
+    chunk = sixteenth < 64 ? 64u : (sixteenth > (1u << 20) ? 1u << 20 : (uint32_t)sixteenth);
+    groups = gridDim.x < kWorkGroups ? gridDim.x : kWorkGroups;
+    group = blockIdx.x % kWorkGroups;
+    ticket = tickets + group * kWorkStride;
+    first_total = first * waves;
+    more = first_total < n;
+    next = first * wave;
+    end = next + first < n ? next + first : n;
+  }
+  // The next chunk, when the range is used up; wave-uniform.
+  __device__ __forceinline__ void refill() {
+    if (next < end || !more) return;
+    uint32_t t = 0;
+    if ((threadIdx.x & 63u) == 0) t = atomicAdd(ticket, 1u);
+    t = __builtin_amdgcn_readfirstlane(t);
+    next = first_total + ((uint64_t)t * groups + group) * chunk;
+    end = next + chunk < n ? next + chunk : n;
+    more = next < n;
+  }
+};
+
+// Persistent-wave traversal of a work range [0, n) of closest-hit and any-hit
+// queries: between node visits, once at least `refill` lanes are idle (or all
+// are), idle lanes take the next items of the wave's work, ranked by ballot.
 // fetch(i, o, d, tmax, tree, any) loads item i, may replace the lane's tree
-// (initially tree0; batches of scenes), sets any for an any-hit query and
-// returns false if the item needs no traversal; store(i, s) receives the
-// finished state.  A fetch that never writes `tree` keeps the tree
-// wave-uniform.  (Splitting a refill over two iterations, so that the item
-// loads overlap the active lanes' node step, measured slower: the new lanes
-// lose a step.)
-template <class Stk, class Fetch, class Store>
-__device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint32_t refill,
+// (initially tree0; batches of scenes) and, with kMixed, sets any for an
+// any-hit query; store(i, s) receives the finished
+// state.  A fetch that never
+// writes `tree` keeps the tree wave-uniform.  (Splitting a refill over two
+// iterations, so that the item loads overlap the active lanes' node step,
+// measured slower: the new lanes lose a step.)
+template <bool kAny, bool kMixed, class Stk, class Fetch, class Store>
+__device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint32_t* ticket, uint32_t refill,
                                                  const Stk& stk, Fetch fetch, Store store) {
   TreeRef tree = tree0;
-  const uint64_t waves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-  const uint64_t chunk = (n + waves - 1) / waves;
+  WaveWork work(n, ticket);
   const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  uint64_t next = wave * chunk;
-  const uint64_t end = next + chunk < n ? next + chunk : n;
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   Trav s;
-  bool active = false;
+  bool active = false, done = false;  // done: s holds the result of `item`, not stored yet
   uint64_t item = 0;
   for (;;) {
     const uint64_t idle = ballot(!active);
     const uint32_t nidle = __popcll(idle);
     if (nidle >= refill || nidle == 64) {
-      if (next < end) {
+      // finished lanes' results together: loads and stores complete in order,
+      // so a store per finished ray would hold up the next visit's loads
+      if (done) store(item, s);
+      done = false;
+      work.refill();
+      if (work.next < work.end) {
         if (!active) {
-          const uint64_t i = next + __popcll(idle & lt);
-          if (i < end) {
+          const uint64_t i = work.next + __popcll(idle & lt);
+          if (i < work.end) {
             V3 o, d;
             float tmax;
             bool any = false;
-            if (fetch(i, o, d, tmax, tree, any)) {
-              item = i;
-              active = trav_init_root<false>(s, tree.root, o, d, tmax, nullptr);
-              s.any = any;
-              if (!active) store(i, s);
-            }
+            fetch(i, o, d, tmax, tree, any);
+            item = i;
+            active = trav_init_root<false>(s, tree.root, o, d, tmax, nullptr);
+            s.any = any;
+            done = !active;
           }
         }
-        next += nidle;
+        work.next += nidle;
       } else if (nidle == 64) {
         break;
       }
     }
-    if (trav_visit<false, true>(s, tree, stk, active)) {
-      store(item, s);
+    if (trav_visit<kAny, kMixed>(s, tree, stk, active)) {
+      done = true;
       active = false;
     }
   }
