@@ -194,19 +194,22 @@ constexpr uint32_t kKeyCompat = 0x2545F491u;
 // src/kernels/lib/intersect.cuh:106-111) and a reduced copy of the node's two
 // triangles for the reject test of traverse.h, which decides which of them
 // need the reference's triangle test on their exact vertices:
-//   scale     2^-k with 2^k at least the extent of the node's two triangles
+//   scale     2^(1-k) with 2^k at least the extent of the node's two triangles
 //             and of its group (its own, its parent's and its grandparent's
 //             slabs), or infinity: no reject test for this node
 //   ref       scale * v1 of the first triangle (exact float)
-//   e         half pairs (first, second triangle) of scale * e1.xyz, e2.xyz
+//   e         half pairs (first, second triangle) of scale / 2 * e1.xyz, e2.xyz
 //   dxy, dz_a half pairs (dx, dy) and (dz, size of the first triangle):
 //             scale * (v1 of the second - v1 of the first triangle)
 //   scale_b   float bits of scale (the low 23 are zero in it) with the second
-//             triangle's size (half) in bits 0..15 and flags in bits 16..22
-// A triangle's size is at least the largest |component| of its scaled e1 and
-// e2, and at least 2^-10.  One extra record after the last node (index n)
-// holds the root's own slab (axis 0) in cslab[0..1].
-constexpr uint32_t kNodeSlabsNormal = 1u << 16;  // every cslab value passes normal_coord
+//             triangle's size (half) in bits 0..15 and kNodeSlabsOdd as the sign
+// A triangle's size is at least the largest |component| of its scaled edges,
+// and at least 2^-10.  Record K holds node K - 1, so that siblings share a
+// 128-byte line; record 0 holds the root's own slab (axis 0) in cslab[0..1]
+// and the largest |coordinate| of the tree's vertices in ref[0].
+constexpr uint32_t kNodeSlabsOdd = 1u << 31;  // some cslab value fails normal_coord
+// Trees from here on have records beyond a 32-bit byte offset.
+constexpr uint32_t kWideNodes = 1u << 26;
 // A missing child's slab (lo, hi) = (kNoSlab, -kNoSlab): empty for every ray
 // that takes the reciprocal quotient (|d| <= 16, |o| <= 2^57).
 constexpr float kNoSlab = 0x1p59f;

@@ -128,14 +128,14 @@ struct JobDev {
   uint32_t n_nodes, num_shaders, num_lights, nslots;
   uint32_t w, h, npix, spp, max_depth, rr_start, seed, paths;
   uint32_t rx0, ry0, rw;
-  float2 root;  // the tree's root slab (axis 0)
+  float root_lo, root_hi, bound;  // record 0 of the tree's nodes
   aur_camera cam;
 };
 
 // A built scene kept for batches: tree-order arrays as the frame render uses.
 struct SceneStore {
   uint32_t count = 0, levels = 0, num_shaders = 0, num_lights = 0, nslots = 0;
-  float2 root_slab = make_float2(0.0f, 0.0f);
+  float root_lo = 0.0f, root_hi = 0.0f, bound = 0.0f;  // record 0 of the nodes
   DevBuf<NodeRec> nodes;
   DevBuf<float> vertices;
   DevBuf<float> normals;
@@ -194,7 +194,6 @@ struct aur_context {
   aur_trace_params trace_params{1, 256, 24, 0, 0};
   aur::DevBuf<float2> gstack;  // global rows of the persistent traversal stack
   aur::DevBuf<uint32_t> trace_work;  // work counters of the persistent trace launches
-  float2 root_slab = make_float2(0.0f, 0.0f);  // host copy of the built tree's root slab
   aur_render_params render_params{aur::kDefaultMaxPaths, 0, aur::kDefaultRenderRefill,
                                   aur::kDefaultRenderStackRows};
   std::atomic<uint32_t> cancel{0};  // set by aur_cancel, consumed by the render it stops
@@ -212,7 +211,7 @@ struct aur_context {
   aur::DevBuf<uint16_t> shader_ids;
   aur::DevBuf<uint32_t> perm;
   aur::DevBuf<aur::NodeRec> nodes;
-  float root_lo = 0.0f, root_hi = 0.0f;
+  float root_lo = 0.0f, root_hi = 0.0f, bound = 0.0f;  // host copy of record 0
 
   // materials and lights
   aur::DevBuf<aur_shader> shaders;

@@ -801,16 +801,21 @@ __device__ inline void slab_of(const float* v, int a, float& lo, float& hi) {
              fmaxf(fmaxf(q[3 * a], q[3 * a + 1]), q[3 * a + 2]));
 }
 
-// Traversal record k (common.h); record n holds the root's own slab.
+// Traversal records (common.h): thread K writes record K, of node K - 1.
 __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec* __restrict__ nodes) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > n) return;
+  const uint32_t K = blockIdx.x * blockDim.x + threadIdx.x;
+  if (K > n) return;
   NodeRec r = {};
-  if (k == n) {  // on axis 0
+  if (K == 0) {
     slab_of(v, 0, r.cslab[0], r.cslab[1]);
-    nodes[k] = r;
+    // the triangles of depths 0..2 hold the extremes of x, y and z
+    for (uint32_t k = 0; k < min(n, 7u); ++k)
+#pragma unroll
+      for (int i = 0; i < 18; ++i) r.ref[0] = fmaxf(r.ref[0], fabsf(v[18 * k + i]));
+    nodes[0] = r;
     return;
   }
+  const uint32_t k = K - 1;
   const float* p = v + (size_t)k * 18;  // points layout, two triangles
   const uint32_t d = depth_of(k);
   const int ca = (int)((d + 1) % 3);
@@ -842,7 +847,7 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
   int ex = 0;
   (void)frexpf(extent, &ex);  // extent < 2^ex
   const bool reject = coord <= kRejectCoord && extent >= kRejectScaleMin && extent <= kRejectScaleMax;
-  const float scale = reject ? ldexpf(1.0f, -ex) : __builtin_inff();
+  const float unit = reject ? ldexpf(1.0f, -ex) : __builtin_inff(), scale = 2.0f * unit;
   float size[2], edge[2][6];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -851,8 +856,8 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const float e1 = q[3 * a + 1] - q[3 * a], e2 = q[3 * a + 2] - q[3 * a];
-      edge[t][a] = reject ? e1 * scale : 0.0f;
-      edge[t][3 + a] = reject ? e2 * scale : 0.0f;
+      edge[t][a] = reject ? e1 * unit : 0.0f;
+      edge[t][3 + a] = reject ? e2 * unit : 0.0f;
       size[t] = fmaxf(size[t], fmaxf(fabsf(edge[t][a]), fabsf(edge[t][3 + a])));
     }
     size[t] *= 1.0f + 0x1p-10f;  // not below after rounding to half
@@ -868,8 +873,8 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
   r.dxy = half2v{(_Float16)dv[0], (_Float16)dv[1]};
   r.dz_a = half2v{(_Float16)dv[2], (_Float16)size[0]};
   const half2v sb = {(_Float16)size[1], (_Float16)0.0f};
-  r.scale_b = __float_as_uint(scale) | (normal ? kNodeSlabsNormal : 0u) | __builtin_bit_cast(uint32_t, sb);
-  nodes[k] = r;
+  r.scale_b = __float_as_uint(scale) | (normal ? 0u : kNodeSlabsOdd) | __builtin_bit_cast(uint32_t, sb);
+  nodes[K] = r;
 }
 
 // cudaGenerateTB (utility.cu:136-180).
@@ -1125,7 +1130,7 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   AUR_HIP(ctx, ctx->normals.reserve((size_t)N * 9));
   AUR_HIP(ctx, ctx->texcoords.reserve((size_t)N * 6));
   AUR_HIP(ctx, ctx->shader_ids.reserve(N));
-  AUR_HIP(ctx, ctx->nodes.reserve((size_t)n + 1));  // + the root's own slab
+  AUR_HIP(ctx, ctx->nodes.reserve((size_t)n + 1));
   AUR_HIP(ctx, ctx->trace_work.reserve(kWorkWords));
   k_gather_geometry<<<blocks(N, 256), 256, 0, s>>>(ctx->perm.p, N, ctx->in_vertices.p,
                                                    ctx->in_normals.p, ctx->in_texcoords.p,
@@ -1140,13 +1145,13 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   AUR_HIP(ctx, hipEventElapsedTime(&ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  // the root's own slab (cslab[0..1] of record n) for launches that start
-  // every ray at the root without reading it
-  float root[2] = {0.0f, 0.0f};
-  AUR_HIP(ctx, hipMemcpyAsync(root, &ctx->nodes.p[n].cslab[0], sizeof(root),
-                              hipMemcpyDeviceToHost, s));
+  // record 0, for launches that start every ray at the root without reading it
+  NodeRec root;
+  AUR_HIP(ctx, hipMemcpyAsync(&root, ctx->nodes.p, sizeof(root), hipMemcpyDeviceToHost, s));
   AUR_HIP(ctx, hipStreamSynchronize(s));
-  ctx->root_slab = make_float2(root[0], root[1]);
+  ctx->root_lo = root.cslab[0];
+  ctx->root_hi = root.cslab[1];
+  ctx->bound = root.ref[0];
   ctx->levels = (uint32_t)L;
   ctx->built = true;
   ctx->has_tb = false;

@@ -319,7 +319,7 @@ __global__ void k_pbr_camera(PbrArgs a, uint32_t* __restrict__ queue) {
 // counts in word w = k % 3.  parts bit 0:
 // extension rays, bit 1: shadow rays.  The two sets are independent, so one
 // launch overlaps their tails.
-template <bool kMulti, bool kSplit>
+template <bool kMulti, bool kSplit, bool kWide>
 __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uint32_t parts,
                                                       uint32_t roff) {
   extern __shared__ float2 stk_mem[];
@@ -349,8 +349,8 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
   if (blockIdx.x == 0)
     for (uint32_t i = threadIdx.x; i < kWorkWords; i += blockDim.x)
       a.counters[kTicketOffset + (w == 2u ? 0u : w + 1u) * kWorkWords + i] = 0;
-  persistent_trace<false, true>(
-      TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, a.job.root}, (uint64_t)n_ext + n_sh,
+  persistent_trace<false, true, kWide>(
+      TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, RootInfo{a.job.root_lo, a.job.root_hi, a.job.bound}}, (uint64_t)n_ext + n_sh,
       a.counters + kTicketOffset + w * kWorkWords, a.refill, stack,
       [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef& tree, bool& any) {
         float4 o4, d4;
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
         }
         if constexpr (kMulti) {
           const JobDev& J = a.jobs[jb];
-          tree = TreeRef{J.nodes, J.tris, J.n_nodes, J.root};
+          tree = TreeRef{J.nodes, J.tris, J.n_nodes, RootInfo{J.root_lo, J.root_hi, J.bound}};
         }
         o = mk(o4.x, o4.y, o4.z);
         d = mk(d4.x, d4.y, d4.z);
@@ -1220,6 +1220,15 @@ aur_status pbr_reserve(aur_context* ctx, uint32_t cap, uint32_t nslots, uint32_t
   return AUR_OK;
 }
 
+// k_pbr_trace with part of the stack in global memory (split) or not, for one
+// tree of n_nodes (kMulti: each lane's own tree, always 64-bit addresses).
+template <bool kMulti>
+void (*trace_kernel(bool split, uint32_t n_nodes))(PbrArgs, uint32_t, uint32_t, uint32_t) {
+  if (kMulti || n_nodes >= kWideNodes)
+    return split ? k_pbr_trace<kMulti, true, true> : k_pbr_trace<kMulti, false, true>;
+  return split ? k_pbr_trace<kMulti, true, kMulti> : k_pbr_trace<kMulti, false, kMulti>;
+}
+
 // Launch shape of k_pbr_trace for up to max_items rays: the traversal stack
 // takes at most levels - 1 rows per lane, the first `rows` in LDS, the rest
 // (with a window) in global memory; the grid is the resident one.
@@ -1231,8 +1240,7 @@ aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, Pb
   const uint32_t want = ctx->render_params.stack_lds_rows;
   const uint32_t rows = want >= maxrows ? maxrows : want;
   lds = (size_t)rows * kBlock * sizeof(float2);
-  grid = resident_grid(ctx, rows < maxrows ? (const void*)k_pbr_trace<kMulti, true> : (const void*)k_pbr_trace<kMulti, false>,
-                       lds, max_items);
+  grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, a.job.n_nodes), lds, max_items);
   a.gstack = nullptr;
   a.klds = rows;
   a.gstack_rows = 0;
@@ -1260,10 +1268,7 @@ void pbr_pass(aur_context* ctx, PbrArgs& a, size_t lds, uint32_t grid_trace,
   // with bounce b's shadow rays, then bounce b's next-event resolve
   const uint32_t sh = a.nslots ? 2u : 0u;
   const auto trace = [&](uint32_t w, uint32_t parts, uint32_t roff) {
-    if (a.gstack)
-      k_pbr_trace<kMulti, true><<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
-    else
-      k_pbr_trace<kMulti, false><<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
+    trace_kernel<kMulti>(a.gstack != nullptr, a.job.n_nodes)<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
   };
   trace(0u, 1u, 0u);
   for (uint32_t b = 0; b < a.max_depth; ++b) {
@@ -1444,7 +1449,9 @@ JobDev frame_job(aur_context* ctx, const aur_camera* cam, const aur_render_opts*
   J.num_textures = ctx->num_textures;
   J.path_start = 0;
   J.n_nodes = ctx->count / 2;
-  J.root = ctx->root_slab;
+  J.root_lo = ctx->root_lo;
+  J.root_hi = ctx->root_hi;
+  J.bound = ctx->bound;
   J.num_shaders = ctx->num_shaders;
   J.num_lights = ctx->num_lights;
   J.nslots = ctx->num_slots;
@@ -1539,10 +1546,7 @@ aur_status compat_passes(aur_context* ctx, const aur_camera* cam, const aur_rend
   c.fin = fr.cw_fin.p;
   c.pixels = fr.pixels.p;
   const auto trace = [&](uint32_t w, uint32_t parts, uint32_t roff) {
-    if (a.gstack)
-      k_pbr_trace<false, true><<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
-    else
-      k_pbr_trace<false, false><<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
+    trace_kernel<false>(a.gstack != nullptr, a.job.n_nodes)<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
   };
   // every stack ray is a hit of depth <= 8 or below one: at most 1 + 2 * 9
   // rays per pixel sample, so the stacks empty within that many levels

@@ -33,12 +33,12 @@ __device__ __forceinline__ void store_result(uint64_t i, const Trav& s, aur_hit*
 // (Keeping the next 64 rays in registers and handing them out by lane
 // permutes measured slower: the permutes' register reuse makes every refill
 // wait for them.)
-template <bool kAny, class Stk>
+template <bool kAny, bool kWide, class Stk>
 __device__ __forceinline__ void trace_rays(TreeRef tree, const aur_ray* __restrict__ rays, uint64_t n,
                                            uint32_t refill, const Stk& stk, aur_hit* __restrict__ hits,
                                            int32_t* __restrict__ ids, uint32_t* __restrict__ work) {
-  tree.root = root_slab(tree.nodes, tree.n_nodes);
-  persistent_trace<kAny, false>(
+  tree.root = root_info(tree.nodes);
+  persistent_trace<kAny, false, kWide>(
       tree, n, work, refill, stk,
       [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef&, bool&) {
         const float4* r = reinterpret_cast<const float4*>(rays + i);
@@ -50,7 +50,7 @@ __device__ __forceinline__ void trace_rays(TreeRef tree, const aur_ray* __restri
       [&](uint64_t i, const Trav& s) { store_result(i, s, hits, ids); });
 }
 
-template <bool kAny, bool kSplit>
+template <bool kAny, bool kSplit, bool kWide>
 __global__ __launch_bounds__(kMaxBlock) void k_trace_pt(const NodeRec* __restrict__ nodes,
                                                         const float* __restrict__ tris, uint32_t n_nodes,
                                                         const aur_ray* __restrict__ rays, uint64_t n,
@@ -69,9 +69,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_trace_pt(const NodeRec* __restric
                          (glb_vf2*)(gstack + gtid),
                          __builtin_amdgcn_make_buffer_rsrc(gstack, (short)0, (int)bytes, 0x00020000),
                          gtid * 8u, lanes, klds};
-    trace_rays<kAny>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill, stk, hits, ids, work);
+    trace_rays<kAny, kWide>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill, stk, hits, ids, work);
   } else {
-    trace_rays<kAny>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill,
+    trace_rays<kAny, kWide>(TreeRef{nodes, tris, n_nodes, {}}, rays, n, refill,
                      lds_stack(stk_mem + threadIdx.x, blockDim.x), hits, ids, work);
   }
 }
@@ -199,7 +199,9 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
     return ctx->fail(AUR_ERR_INVALID_ARG, "trace: refill must be in 1..64");
   using Kern = void (*)(const NodeRec*, const float*, uint32_t, const aur_ray*, uint64_t, aur_hit*,
                         int32_t*, uint32_t*, uint32_t, float2*, uint32_t, uint32_t);
-  const Kern fn = klds != 0 ? k_trace_pt<kAny, true> : k_trace_pt<kAny, false>;
+  const bool wide = ctx->count / 2 >= kWideNodes;
+  const Kern fn = klds != 0 ? (wide ? k_trace_pt<kAny, true, true> : k_trace_pt<kAny, true, false>)
+                            : (wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>);
   AUR_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, (int)block, lds_pt));
   if (per_cu < 1) per_cu = 1;
   uint64_t blocks_total = (uint64_t)per_cu * ctx->num_cus;

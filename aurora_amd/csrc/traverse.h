@@ -127,25 +127,20 @@ struct TraceCount {
 // axis and a pending entry's depth are bit tests.
 struct Trav {
   V3 o, d, y;      // origin, direction, RN(1/direction)
-  float dmax;      // largest |direction component|; NaN: no reject test for this ray
+  float rj_size, rj_scale, rj;  // the reject test's threshold terms (trav_test)
   uint32_t fast;   // bit m: the children of a node at depth m take the reciprocal quotient
   float t, u, v;   // current closest hit (t = ray.t)
   int32_t id;
   uint32_t K, depth;  // node, one-hot depth
   uint32_t trail;  // depths with a pending entry
   uint32_t top;    // stack position (units of the stack)
-  uint32_t cand;   // triangles of the node still to test exactly (bits 0, 1), kStop, kPop
-  bool any;        // any-hit query (persistent_trace's mixed launches)
   float2 r;        // range of the node after its slab test
   float4 slab;     // the node's children's slabs
   uint32_t flags;  // the node's scale_b
 };
-// kStop: an any hit is found; kPop: the node is done, the next pending entry
-// is to be taken.
-constexpr uint32_t kCand = 3u, kStop = 4u, kPop = 8u;
 // Depths whose children's axis (depth + 1) % 3 is x, y, z.
 constexpr uint32_t kChildX = 0x24924924u, kChildY = 0x49249249u, kChildZ = 0x92492492u;
-constexpr uint32_t kExactShare = 5u;  // exact tests run once candidates wait in a fifth of the active lanes
+constexpr uint32_t kExactShare = 12u;  // exact tests run once candidates wait in a twelfth of the active lanes
 
 // Per-lane stack of deferred ranges.  A deferred child is always deeper
 // than every entry already pending (entries sit on the current path's
@@ -217,34 +212,36 @@ __device__ __forceinline__ bool fast_axis(float o, float d) {
   return (a >= 0x1p-60f) & (a <= 16.0f) & normal & (fabsf(o) <= 0x1p57f);
 }
 
+// What record 0 says of a tree: the root's own slab and the largest
+// |coordinate| of its vertices.
+struct RootInfo {
+  float lo, hi, bound;
+};
+
 // The tree a lane traverses: node records, the triangles' vertices in tree
-// order, the node count and the root's own slab (cslab[0..1] of the record
-// after the last node).
+// order and the node count.
 struct TreeRef {
   const NodeRec* nodes;
   const float* tris;
   uint32_t n_nodes;
-  float2 root;
+  RootInfo root;
 };
 
-// dmax of a ray, or NaN when the reject test's bounds do not cover it.
-__device__ __forceinline__ float reject_dmax(V3 o, V3 d) {
-  const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
-  const float c = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
-  const float all = ((d.x + d.y) + d.z) + ((o.x + o.y) + o.z);  // NaN if any is
-  return ((m >= kRejectDirMin) & (m <= kRejectDirMax) & (c <= kRejectCoord) & (all == all)) ? m : __builtin_nanf("");
+__device__ __forceinline__ RootInfo root_info(const NodeRec* __restrict__ nodes) {
+  return RootInfo{nodes[0].cslab[0], nodes[0].cslab[1], nodes[0].ref[0]};
 }
 
-// The root's own slab: cslab[0..1] of the record after the last node.
-__device__ __forceinline__ float2 root_slab(const NodeRec* __restrict__ nodes, uint32_t n_nodes) {
-  return make_float2(nodes[n_nodes].cslab[0], nodes[n_nodes].cslab[1]);
-}
+// The reject test's threshold (trav_test).
+constexpr float kRejA = 1.6e-3f;                            // times 2 |C|max
+constexpr float kRejSize = 2.0f * 3.4f * kRejA;             // 2 thr's terms times D: z,
+constexpr float kRejB = 2.0f * 8.125f * 0x1p-12f;           // constant,
+constexpr float kRejScale = 0x1p-18f;                       // and the record's scale (2 P + O)
 
 // Sets up a ray; returns false when the root's slab culls it (finished, miss).
 // The reciprocals y serve only axes with 2^-60 <= |d| <= 16, where recip_rn
 // equals 1.0f / d.
 template <bool kCount>
-__device__ __forceinline__ bool trav_init_root(Trav& s, float2 root, V3 o, V3 d, float tmax,
+__device__ __forceinline__ bool trav_init_root(Trav& s, RootInfo root, V3 o, V3 d, float tmax,
                                                TraceCount* cnt) {
   s.o = o;
   s.d = d;
@@ -254,37 +251,46 @@ __device__ __forceinline__ bool trav_init_root(Trav& s, float2 root, V3 o, V3 d,
   __asm__ volatile("" : "+v"(s.y.x), "+v"(s.y.y), "+v"(s.y.z));
   const bool fx = fast_axis(o.x, d.x), fy = fast_axis(o.y, d.y), fz = fast_axis(o.z, d.z);
   s.fast = (fx ? kChildX : 0u) | (fy ? kChildY : 0u) | (fz ? kChildZ : 0u);
-  s.dmax = reject_dmax(o, d);
+  {
+    // terms of the reject test's threshold, or NaN (no triangle is rejected)
+    // for rays outside its bound's range
+    const float dm = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+    const float om = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+    const float all = ((d.x + d.y) + d.z) + ((o.x + o.y) + o.z);  // NaN if any is
+    const bool in = (dm >= kRejectDirMin) & (dm <= kRejectDirMax) & (om <= kRejectCoord) & (all == all);
+    s.rj = in ? dm * kRejB : __builtin_nanf("");
+    s.rj_size = dm * kRejSize;
+    s.rj_scale = dm * __builtin_fmaf(2.0f, root.bound, om) * kRejScale;
+  }
   s.t = tmax;
   s.u = s.v = 0.0f;
   s.id = -1;
   s.K = s.depth = 1;
-  s.trail = s.top = s.cand = 0;
-  s.any = false;
+  s.trail = s.top = 0;
   if (kCount) cnt->popped += 1;  // the root
-  s.r = narrow(make_float2(kEpsilon, kInfinity), root.x, root.y, o.x, d.x, s.y.x, fx);
+  s.r = narrow(make_float2(kEpsilon, kInfinity), root.lo, root.hi, o.x, d.x, s.y.x, fx);
   return (s.r.x <= s.r.y) && (s.r.x <= s.t);
 }
 
 template <bool kCount>
 __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3 d, float tmax,
                                           TraceCount* cnt) {
-  return trav_init_root<kCount>(s, root_slab(tree.nodes, tree.n_nodes), o, d, tmax, cnt);
+  return trav_init_root<kCount>(s, root_info(tree.nodes), o, d, tmax, cnt);
 }
 
 // ---- the reject test ----
 //
-// Loads the node's record and leaves in s.cand the triangles that may pass
-// the reference's test.  Two things bound a visit when every lane reads
+// Loads the node's record and says which of its triangles may
+// pass the reference's test.  Two things bound a visit when every lane reads
 // another node: VALU issue and the vector L1, which looks up one lane's 16
 // bytes per cycle and CU.  Both triangles' exact test took 125 VALU
-// instructions and a 96-byte record 6 loads; this test takes 90 and the
+// instructions and a 96-byte record 6 loads; this test takes 66 and the
 // 64-byte record 4, and what it leaves over (1.2% of the visits at 1M
-// triangles) costs 6 more per visit.  With the visit's second half
-// (trav_next) rewritten at the same time: 2^24 incoherent rays into 1M
-// triangles 7.28 -> 5.72 ms (3.63e9 -> 2.81e9 VALU instructions, L1 lookups
-// 4.43e9 -> 3.00e9), 2^21 into 10M triangles 6.48 -> 5.97 ms, a 1080p frame
-// of 8 samples over 1M triangles 41.2 -> 37.0 ms.
+// triangles) costs 6 more per visit.  2^24 incoherent rays into 1M triangles
+// take 4.6 ms (7.3 with the exact tests in every visit): 2.35e9 VALU
+// instructions at 0.86 of the issue rate, 2.97e9 L1 lookups at 1.08 per cycle
+// and CU.  More resident waves than 16 per CU are slower: the lines of their
+// visits no longer fit the 32 KB L1 between a record's four loads.
 //
 // With T = p - v1 for any point p of the ray's line and C = T x d, the
 // Moller-Trumbore numerators are u det = e2 . C, v det = -(e1 . C) and
@@ -293,83 +299,98 @@ __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3
 // rounding).  p is the ray's entry into the node's range, so that T is no
 // larger than the node's group, and lengths are in units of the group's size.
 //
-// Bound.  D = dmax, z = the triangle's size (each |e| component <= z),
-// q = 2^-11 + 2^-15, t = the range's entry.
+// Bound.  D = the largest |direction component|, z = the triangle's size (each
+// |e| component <= z), q = 2^-11 + 2^-15, t = the range's entry, P = the
+// largest |coordinate| of the tree, O of the origin; sigma = 2^-k, half of
+// the record's scale (T, and so C and the numerators, come out doubled).
 //   edges: rounding to half moves a component by at most q z (2^-11 relative,
 //     2^-25 absolute, z >= 2^-10);
 //   T: off by at most 2^-12 (dv, |dv| <= 1) + 2^-15 (roundings of dv and T,
-//     |T| <= 4) + 2^-24 scale |p|max (one fma for p); C by 2 D times that and
+//     |T| <= 4) + 2^-24 sigma |p|max (one fma for p); C by 2 D times that and
 //     2^-22 D;
-//   u det, v det: z (3 q |C|max + D (6.82 2^-12 + 6 2^-24 scale |p|max));
+//   u det, v det: z (3 q |C|max + D (6.82 2^-12 + 6 2^-24 sigma |p|max));
 //   det: e1 x e2 in half, 3 D ((4.01 q + 3 2^-11) z^2 + 2^-24);
-//   the reference's floats: 36 2^-24 z D scale |o - v1|max per numerator
-//     (T, P or Q and the dot product), scale |o - v1|max <= scale t D + 5.
-// So a triangle that the reference accepts has, with
-//   thr = A |C|max + 3.4 A z D + D (B + 2^-18 scale (t D + |p|max)),
+//   the reference's floats: 36 2^-24 z D sigma |o - v1|max per numerator
+//     (T, P or Q and the dot product), sigma |o - v1|max <= sigma t D + 5.
+// With |T| <= 4, |p|max <= P + 4 / sigma and t D <= |p|max + O, so the terms in
+// sigma are at most 36 2^-24 z D (sigma (2 P + O) + 8).  A triangle that the
+// reference accepts has, with
+//   thr = A |C|max + 3.4 A z D + D (B + 2^-18 sigma (2 P + O)),
 // u det >= -z thr, v det >= -z thr and (1 - u - v) det >= -2 z thr:
 // A = 1.6e-3 >= 3 q = 1.557e-3; half the third function's error is that of
 // one numerator plus z D 5.32e-3 z, below 3.4 A z = 5.44e-3 z, plus 0.38 2^-12
-// z D, and B = 8 2^-12 >= (6.82 + 0.38) 2^-12 with a margin for the float
-// roundings of this test itself (below 2^-18 z D).
+// z D, and B = 8.125 2^-12 >= (6.82 + 0.38) 2^-12 + 2^-15 with a margin for the
+// float roundings of this test itself (below 2^-18 z D).
 // Comparisons are written so that NaN and infinity keep a triangle.
-constexpr float kRejA = 1.6e-3f, kRejA2 = 3.4f * 1.6e-3f, kRejB = 0x1p-9f, kRejC = 0x1p-18f;
-
 __device__ __forceinline__ float lo16(half2v h) { return (float)h.x; }
 __device__ __forceinline__ float hi16(half2v h) { return (float)h.y; }
 __device__ __forceinline__ float max3abs(float a, float b, float c) {
   return fmaxf(fmaxf(fabsf(a), fabsf(b)), fabsf(c));
 }
 
-// Whether the triangle may be accepted: T = p - v1, edges e1 and e2, size, det
-// (all scaled); base = D (B + 2^-18 scale (t D + |p|max)).
-__device__ __forceinline__ bool may_hit(V3 T, V3 d, V3 e1, V3 e2, float det, float size, float dmax, float base) {
+// a - b with b the low or high half of h (one instruction; the compiler would
+// convert first).
+__device__ __forceinline__ float sub_lo16(float a, half2v h) {
+  float r;
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+  return r;
+}
+__device__ __forceinline__ float sub_hi16(float a, half2v h) {
+  float r;
+  __asm__("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(a));
+  return r;
+}
+
+// Whether the triangle may be accepted: T doubled, edges e1 and e2, size and
+// det in the record's units; base = 2 D (B + 2^-18 sigma (2 P + O)).
+__device__ __forceinline__ bool may_hit(V3 T, V3 d, V3 e1, V3 e2, float det, float size, float rj_size, float base) {
   const float cx = __builtin_fmaf(T.y, d.z, -(T.z * d.y));
   const float cy = __builtin_fmaf(T.z, d.x, -(T.x * d.z));
   const float cz = __builtin_fmaf(T.x, d.y, -(T.y * d.x));
   const float un = __builtin_fmaf(e2.z, cz, __builtin_fmaf(e2.y, cy, __builtin_fmaf(e2.x, cx, 0.0f)));
   const float vn = __builtin_fmaf(-e1.z, cz, __builtin_fmaf(-e1.y, cy, __builtin_fmaf(-e1.x, cx, 0.0f)));
-  const float wn = 0.5f * (det - un - vn);
+  const float wn = __builtin_fmaf(-0.5f, un + vn, det);
   const float m = fminf(fminf(un, vn), wn);
-  const float thr = __builtin_fmaf(max3abs(cx, cy, cz), kRejA,
-                                   __builtin_fmaf(__builtin_fmaf(size, dmax, 0.0f), kRejA2, base));
+  const float thr = __builtin_fmaf(max3abs(cx, cy, cz), kRejA, __builtin_fmaf(size, rj_size, base));
   return !(__builtin_fmaf(size, thr, m) < 0.0f);
 }
 
-template <bool kCount>
-__device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCount* cnt) {
+// kWide: the record's address takes 64-bit arithmetic per lane (trees of 2^26
+// nodes and more, and lanes with trees of their own); else it is a 32-bit
+// offset from a wave-uniform base.
+template <bool kCount, bool kWide>
+__device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCount* cnt, bool& may_a, bool& may_b) {
   if (kCount) {
     cnt->passed += 1;
     cnt->popped += (2 * s.K <= tree.n_nodes) + (2 * s.K + 1 <= tree.n_nodes);
   }
-  const uint4* rec = reinterpret_cast<const uint4*>(tree.nodes + s.K - 1);
-  const uint4 a0 = rec[0], a1 = rec[1], a2 = rec[2], a3 = rec[3];
+  const size_t offset = kWide ? (size_t)s.K * sizeof(NodeRec) : (size_t)(s.K * (uint32_t)sizeof(NodeRec));
+  const uint4* rec = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(tree.nodes) + offset);
+  const uint4 a1 = rec[1], a2 = rec[2], a3 = rec[3], a0 = rec[0];
   s.slab = make_float4(__uint_as_float(a0.x), __uint_as_float(a0.y), __uint_as_float(a0.z), __uint_as_float(a0.w));
   s.flags = a1.w;
   const auto h2 = [](uint32_t x) { return __builtin_bit_cast(half2v, x); };
   const half2v e1x = h2(a2.x), e1y = h2(a2.y), e1z = h2(a2.z), e2x = h2(a2.w), e2y = h2(a3.x), e2z = h2(a3.y);
   const half2v dxy = h2(a3.z), dza = h2(a3.w), szb = h2(a1.w);
-  const float scale = __uint_as_float(a1.w & 0xFF800000u);
+  const float scale = __uint_as_float(a1.w & 0x7F800000u);
   const V3 d = s.d;
   const V3 p = mk(__builtin_fmaf(s.r.x, d.x, s.o.x), __builtin_fmaf(s.r.x, d.y, s.o.y),
                   __builtin_fmaf(s.r.x, d.z, s.o.z));
   const V3 Ta = mk(__builtin_fmaf(p.x, scale, -__uint_as_float(a1.x)), __builtin_fmaf(p.y, scale, -__uint_as_float(a1.y)),
                    __builtin_fmaf(p.z, scale, -__uint_as_float(a1.z)));
-  const V3 Tb = mk(__builtin_fmaf(lo16(dxy), -1.0f, Ta.x), __builtin_fmaf(hi16(dxy), -1.0f, Ta.y),
-                   __builtin_fmaf(lo16(dza), -1.0f, Ta.z));
-  const float reach = __builtin_fmaf(s.r.x, s.dmax, max3abs(p.x, p.y, p.z)) * scale;
-  const float base = __builtin_fmaf(reach, kRejC, kRejB) * s.dmax;
+  const V3 Tb = mk(sub_lo16(Ta.x, dxy), sub_hi16(Ta.y, dxy), sub_lo16(Ta.z, dza));
+  const float base = __builtin_fmaf(scale, s.rj_scale, s.rj);
   // e1 x e2 of both triangles at once
   const half2v nx = __builtin_elementwise_fma(e1y, e2z, -(e1z * e2y));
   const half2v ny = __builtin_elementwise_fma(e1z, e2x, -(e1x * e2z));
   const half2v nz = __builtin_elementwise_fma(e1x, e2y, -(e1y * e2x));
   const float deta = __builtin_fmaf(-lo16(nz), d.z, __builtin_fmaf(-lo16(ny), d.y, __builtin_fmaf(-lo16(nx), d.x, 0.0f)));
   const float detb = __builtin_fmaf(-hi16(nz), d.z, __builtin_fmaf(-hi16(ny), d.y, __builtin_fmaf(-hi16(nx), d.x, 0.0f)));
-  const bool ca = may_hit(Ta, d, mk(lo16(e1x), lo16(e1y), lo16(e1z)), mk(lo16(e2x), lo16(e2y), lo16(e2z)), deta,
-                          hi16(dza), s.dmax, base);
-  const bool cb = may_hit(Tb, d, mk(hi16(e1x), hi16(e1y), hi16(e1z)), mk(hi16(e2x), hi16(e2y), hi16(e2z)), detb,
-                          lo16(szb), s.dmax, base);
-  const bool far = !(max3abs(Ta.x, Ta.y, Ta.z) <= 4.0f);
-  s.cand = (uint32_t)(ca | far) | ((uint32_t)(cb | far) << 1);
+  const bool far = !(max3abs(Ta.x, Ta.y, Ta.z) <= 8.0f);
+  may_a = far | may_hit(Ta, d, mk(lo16(e1x), lo16(e1y), lo16(e1z)), mk(lo16(e2x), lo16(e2y), lo16(e2z)), deta,
+                        hi16(dza), s.rj_size, base);
+  may_b = far | may_hit(Tb, d, mk(hi16(e1x), hi16(e1y), hi16(e1z)), mk(hi16(e2x), hi16(e2y), hi16(e2z)), detb,
+                        lo16(szb), s.rj_size, base);
   // every load has returned here: with the slabs' still in flight on some
   // path, the next visit's address, in one of their registers, waited for all
   // outstanding memory operations, stores included
@@ -377,14 +398,13 @@ __device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCou
 }
 
 // The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of the
-// first candidate of the node, on the vertices it was uploaded with.
-template <bool kAny, bool kMixed = false>
-__device__ __forceinline__ void trav_exact(Trav& s, const float* __restrict__ tris) {
-  const uint32_t tri = 2 * s.K - 1u - (s.cand & 1u);
+// node's first or second triangle, on the vertices it was uploaded with;
+// returns whether it became the closest hit.
+__device__ __forceinline__ bool trav_exact(Trav& s, const float* __restrict__ tris, bool first) {
+  const uint32_t tri = 2 * s.K - (first ? 2u : 1u);
   const float* p = tris + (size_t)tri * 9;  // points layout: x1 x2 x3 y1 y2 y3 z1 z2 z3
   const V3 v1 = mk(p[0], p[3], p[6]);
   const V3 e1 = mk(p[1], p[4], p[7]) - v1, e2 = mk(p[2], p[5], p[8]) - v1;
-  s.cand &= s.cand - 1u;
   const V3 P = cross(s.d, e2);
   const float det = dot(e1, P);
   float inv = recip_rn(det);
@@ -396,18 +416,18 @@ __device__ __forceinline__ void trav_exact(Trav& s, const float* __restrict__ tr
     s.u = u;
     s.v = v;
     s.id = (int32_t)tri;
-    if (kAny || (kMixed && s.any)) s.cand = kStop;
   }
+  return hit;
 }
 
-// Leaves the node (no candidates left) for the next one; returns true when
+// Leaves the node (both triangles done) for the next one; returns true when
 // the traversal has finished.  The near child is taken directly, the far one
 // deferred; without a child to take, one pending entry is popped, and if its
-// range now starts beyond the closest hit the lane keeps kPop and pops again
-// in the next step (1.8% of the steps at 1M triangles; an inner loop until an
+// range now starts beyond the closest hit (again = true) the lane pops again,
+// with popping set, in the next step (1.8% of the steps at 1M triangles; an inner loop until an
 // entry passes made every lane of the wave wait through its iterations).
 template <class Stk>
-__device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& stk) {
+__device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& stk, bool popping, bool& again) {
   const bool ax = (s.depth & kChildX) != 0u, ay = (s.depth & kChildY) != 0u;
   // by value: a select of members would keep the state in memory
   const auto pick = [](bool c, float a, float b) { return c ? a : b; };
@@ -422,8 +442,7 @@ __device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& 
   const float n2 = pick(sw, s.slab.y, s.slab.z) - oc, n3 = pick(sw, s.slab.x, s.slab.w) - oc;
   float nx = quot_fast(n0, dc, yc), ny = quot_fast(n1, dc, yc);
   float fx = quot_fast(n2, dc, yc), fy = quot_fast(n3, dc, yc);
-  const uint32_t normal = (uint32_t)((int32_t)(s.flags << 15) >> 31);  // kNodeSlabsNormal as a mask
-  if ((s.fast & s.depth & normal) == 0u) {
+  if (((s.fast & s.depth) == 0u) | ((int32_t)s.flags < 0)) {
     // true division, with the reference's fminf / fmaxf (NaN, division by 0)
     const float a = n0 / dc, b = n1 / dc, c = n2 / dc, e = n3 / dc;
     nx = min_q(a, b);
@@ -438,9 +457,8 @@ __device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& 
   ny = min_q(ny, s.r.y);
   fx = max_q(fx, s.r.x);
   fy = min_q(fy, s.r.y);
-  const bool live = s.cand == 0u;
-  const bool far = live & (fx <= fy);
-  const bool take_near = live & (nx <= ny) & (nx <= s.t);
+  const bool far = !popping & (fx <= fy);
+  const bool take_near = !popping & (nx <= ny) & (nx <= s.t);
   const bool take_far = !take_near & far & (fx <= s.t);
   if (take_near & far) {
     stk.push(s.top, make_float2(fx, fy));
@@ -452,7 +470,7 @@ __device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& 
     s.r = make_float2(take_near ? nx : fx, take_near ? ny : fy);
     return false;
   }
-  if ((s.trail == 0u) | ((s.cand & kStop) != 0u)) return true;
+  if (s.trail == 0u) return true;
   const float2 e = stk.pop(s.top);
   const uint32_t z = (uint32_t)__builtin_clz(s.trail);
   const uint32_t bit = 0x80000000u >> z;
@@ -461,24 +479,54 @@ __device__ __forceinline__ bool trav_next(Trav& s, uint32_t n_nodes, const Stk& 
   s.K = (s.K >> (z - (uint32_t)__builtin_clz(s.depth))) ^ 1u;
   s.depth = bit;
   s.r = e;
-  s.cand = e.x <= s.t ? 0u : kPop;
+  again = !(e.x <= s.t);
   return false;
 }
 
 // Lane mask of a condition, without materialising it as an integer.
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
-// One step of a persistent wave; returns true in lanes whose traversal has
-// finished.  Lanes whose node left candidates wait until they are a fifth of
-// the active lanes (or all of them): the exact test costs nearly a visit's
-// instructions for however few lanes run it.
-template <bool kAny, bool kMixed, class Stk>
-__device__ __forceinline__ bool trav_visit(Trav& s, const TreeRef& tree, const Stk& stk, bool active) {
-  if (active && s.cand == 0u) trav_test<false>(s, tree, nullptr);
-  const bool pending = active && (s.cand & kCand);
-  const uint32_t np = (uint32_t)__popcll(ballot(pending));
-  if (np * kExactShare >= (uint32_t)__popcll(ballot(active)) && pending) trav_exact<kAny, kMixed>(s, tree.tris);
-  return active && !(s.cand & kCand) && trav_next(s, tree.n_nodes, stk);
+// A persistent wave's lanes as masks, so that their states live in scalar
+// registers and branch conditions cost no vector instructions.
+struct WaveState {
+  uint64_t active = 0;        // lanes with a ray
+  uint64_t may_a = 0, may_b = 0;  // ... whose node's first, second triangle is still to be tested exactly
+  uint64_t popping = 0;       // ... that take the next pending entry
+  uint64_t any = 0;           // lanes with an any-hit query (mixed launches)
+};
+__device__ __forceinline__ bool in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// One step of a persistent wave; returns the lanes whose traversal has
+// finished.  Lanes whose node left candidates wait until they are a twelfth of
+// the active lanes (or all of them): the exact test costs about a visit's
+// instructions for however few lanes run it (a fifth was 3% slower on the
+// 1080p frame, an eighth 1%).
+template <bool kAny, bool kMixed, bool kWide, class Stk>
+__device__ __forceinline__ uint64_t trav_visit(Trav& s, WaveState& w, const TreeRef& tree, const Stk& stk) {
+  bool a = false, b = false;
+  if (in(w.active & ~(w.may_a | w.may_b | w.popping))) trav_test<false, kWide>(s, tree, nullptr, a, b);
+  w.may_a |= ballot(a);
+  w.may_b |= ballot(b);
+  const uint64_t pending = w.may_a | w.may_b;
+  uint64_t finished = 0;
+  if (pending != 0 && (uint32_t)__popcll(pending) * kExactShare >= (uint32_t)__popcll(w.active)) {
+    bool hit = false;
+    if (in(pending)) hit = trav_exact(s, tree.tris, in(w.may_a));
+    w.may_b &= w.may_a;  // lanes that tested their first triangle
+    w.may_a = 0;
+    if (kAny || kMixed) {
+      finished = ballot(hit) & (kAny ? ~0ull : w.any);
+      w.may_b &= ~finished;
+      w.active &= ~finished;
+    }
+  }
+  const uint64_t go = w.active & ~(w.may_a | w.may_b);
+  bool end = false, again = false;
+  if (in(go)) end = trav_next(s, tree.n_nodes, stk, in(w.popping), again);
+  w.popping = (w.popping & ~go) | ballot(again);
+  const uint64_t ended = ballot(end);
+  w.active &= ~ended;
+  return finished | ended;
 }
 
 // The items a wave of a persistent launch takes from [0, n): first a range of
@@ -543,7 +591,7 @@ struct WaveWork {
 // writes `tree` keeps the tree wave-uniform.  (Splitting a refill over two
 // iterations, so that the item loads overlap the active lanes' node step,
 // measured slower: the new lanes lose a step.)
-template <bool kAny, bool kMixed, class Stk, class Fetch, class Store>
+template <bool kAny, bool kMixed, bool kWide, class Stk, class Fetch, class Store>
 __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint32_t* ticket, uint32_t refill,
                                                  const Stk& stk, Fetch fetch, Store store) {
   TreeRef tree = tree0;
@@ -551,40 +599,40 @@ __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   Trav s;
-  bool active = false, done = false;  // done: s holds the result of `item`, not stored yet
+  WaveState w;
+  uint64_t done = 0;  // lanes whose result of `item` is not stored yet
   uint64_t item = 0;
   for (;;) {
-    const uint64_t idle = ballot(!active);
+    const uint64_t idle = ~w.active;
     const uint32_t nidle = __popcll(idle);
     if (nidle >= refill || nidle == 64) {
       // finished lanes' results together: loads and stores complete in order,
       // so a store per finished ray would hold up the next visit's loads
-      if (done) store(item, s);
-      done = false;
+      if (in(done)) store(item, s);
+      done = 0;
       work.refill();
       if (work.next < work.end) {
-        if (!active) {
+        bool enter = false, miss = false, any = false;
+        if (in(idle)) {
           const uint64_t i = work.next + __popcll(idle & lt);
           if (i < work.end) {
             V3 o, d;
             float tmax;
-            bool any = false;
             fetch(i, o, d, tmax, tree, any);
             item = i;
-            active = trav_init_root<false>(s, tree.root, o, d, tmax, nullptr);
-            s.any = any;
-            done = !active;
+            enter = trav_init_root<false>(s, tree.root, o, d, tmax, nullptr);
+            miss = !enter;
           }
         }
+        w.active |= ballot(enter);
+        if (kMixed) w.any = (w.any & ~idle) | ballot(any);
+        done = ballot(miss);
         work.next += nidle;
       } else if (nidle == 64) {
         break;
       }
     }
-    if (trav_visit<kAny, kMixed>(s, tree, stk, active)) {
-      done = true;
-      active = false;
-    }
+    done |= trav_visit<kAny, kMixed, kWide>(s, w, tree, stk);
   }
 }
 
@@ -595,10 +643,18 @@ __device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3
                                           uint32_t stride, TraceCount* cnt = nullptr) {
   const LdsStack st = lds_stack(stk, stride);
   if (!trav_init<kCount>(s, tree, o, d, tmax, cnt)) return;
-  do {
-    if (s.cand == 0u) trav_test<kCount>(s, tree, cnt);
-    while (s.cand & kCand) trav_exact<kAny>(s, tree.tris);
-  } while (!trav_next(s, tree.n_nodes, st));
+  bool popping = false;
+  for (;;) {
+    if (!popping) {
+      bool a, b;
+      trav_test<kCount, true>(s, tree, cnt, a, b);
+      if (a && trav_exact(s, tree.tris, true) && kAny) return;
+      if (b && trav_exact(s, tree.tris, false) && kAny) return;
+    }
+    bool again = false;
+    if (trav_next(s, tree.n_nodes, st, popping, again)) return;
+    popping = again;
+  }
 }
 
 }  // namespace aur
