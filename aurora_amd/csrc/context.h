@@ -196,6 +196,7 @@ struct aur_context {
   aur::DevBuf<uint32_t> trace_work;  // work counters of the persistent trace launches
   aur_render_params render_params{aur::kDefaultMaxPaths, 0, aur::kDefaultRenderRefill,
                                   aur::kDefaultRenderStackRows};
+  bool render_rows_default = true;  // stack_lds_rows was not chosen by the caller
   std::atomic<uint32_t> cancel{0};  // set by aur_cancel, consumed by the render it stops
 
   // uploaded geometry (input order)

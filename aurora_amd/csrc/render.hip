@@ -1237,7 +1237,16 @@ aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, Pb
                        uint32_t& grid) {
   FrameState& fr = ctx->frame;
   const uint32_t maxrows = levels > 1 ? levels - 1 : 1;
-  const uint32_t want = ctx->render_params.stack_lds_rows;
+  // By default a frame keeps every row in LDS, which leaves 10 (30 levels) to
+  // 28 waves per CU.  A 12-row window lets 28 reside at any depth, but the
+  // lines of that many waves' visits push each other out of the L1: 1080p
+  // frame of 1M triangles (19 levels) 32.1 ms with the window, 27.3 with all
+  // rows; compat 7.70 / 7.12 ms; 102,424 triangles at 512^2 21.0 / 18.9 ms.  A
+  // batch's lanes walk several smaller trees and spend more instructions per
+  // visit on them, so it keeps the window: 5 jobs of two bounces 4.00 ms with
+  // it, 4.18 with all rows; 16 jobs of six 25.2 / 25.6 ms.
+  const uint32_t want = !ctx->render_rows_default ? ctx->render_params.stack_lds_rows
+                                                  : (kMulti ? kDefaultRenderStackRows : maxrows);
   const uint32_t rows = want >= maxrows ? maxrows : want;
   lds = (size_t)rows * kBlock * sizeof(float2);
   grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, a.job.n_nodes), lds, max_items);

@@ -244,8 +244,9 @@ aur_status aur_frame_render(aur_context* ctx, const aur_camera* camera,
  * this many (1..64) are idle; 0 selects the default (16).
  * stack_lds_rows: how many rows of each lane's traversal stack live in LDS
  * in those launches; deeper rows go to global memory, leaving LDS for more
- * resident waves.  0 selects the default (12); a value of at least the
- * tree's levels - 1 keeps every row in LDS.
+ * resident waves.  0 selects the default (aur_get_render_params reports 12):
+ * 12 rows in batches, every row in frames, as a value of at least the tree's
+ * levels - 1 does.
  * Images do not depend on any of them: samples are accumulated in sample
  * order. */
 typedef struct aur_render_params {
