@@ -57,37 +57,27 @@ struct SubGroup {
   uint32_t off, size, first, count;
 };
 
-// Triangle bounds on one axis, (min, max), stored [axis][triangle].
-// kx, ky: the min keys of x and y on the axis of the last level (L - 1),
-// loaded by the caller; level <= L - 2.
-// orig (optional): triangle id of each renumbered index x, y (the subtree
-// phase works on positions, renumbered by the last k_emit).
-__device__ inline void write_pair_k(uint32_t h, uint32_t x, uint32_t y, float kx, float ky,
-                                    int level, int L, const float2* __restrict__ bb, uint32_t N,
-                                    uint32_t* __restrict__ P, const uint32_t* __restrict__ orig = nullptr) {
-  bool y_first = ky < kx;
-  if (!y_first && !(kx < ky)) {
-    const int lo = max(level + 1, L - 3);
-    for (int lev = L - 2; lev >= lo; --lev) {
-      const float2* km = bb + (size_t)(lev % 3) * N;
-      const float ax = km[x].x, ay = km[y].x;
-      if (ay < ax) {
-        y_first = true;
-        break;
-      }
-      if (ax < ay) break;
-    }
+// Order of a finished pair x, y of a level <= L - 2: whether y comes first.
+// The reference re-sorts every finished pair at the later levels; only the
+// last three can differ.  key(axis, element): the element's min key.
+template <class Key>
+__device__ __forceinline__ bool second_first(uint32_t x, uint32_t y, int level, int L, Key key) {
+  const int lo = max(level + 1, L - 3);
+  for (int lev = L - 1; lev >= lo; --lev) {
+    const auto kx = key(lev % 3, x), ky = key(lev % 3, y);
+    if (ky < kx) return true;
+    if (kx < ky) return false;
   }
-  const uint32_t a = y_first ? y : x, b = y_first ? x : y;
-  P[2 * (size_t)h] = orig ? orig[a] : a;
-  P[2 * (size_t)h + 1] = orig ? orig[b] : b;
+  return false;
 }
 
+// bb: triangle bounds (min, max), [axis][triangle].
 __device__ inline void write_pair(uint32_t h, uint32_t x, uint32_t y, int level, int L,
                                   const float2* __restrict__ bb, uint32_t N,
                                   uint32_t* __restrict__ P) {
-  const float2* km = bb + (size_t)((L - 1) % 3) * N;
-  write_pair_k(h, x, y, km[x].x, km[y].x, level, L, bb, N, P);
+  const bool swap = second_first(x, y, level, L, [&](int a, uint32_t i) { return bb[(size_t)a * N + i].x; });
+  P[2 * (size_t)h] = swap ? y : x;
+  P[2 * (size_t)h + 1] = swap ? x : y;
 }
 
 // computeTriangleBounds (rebuilder.cu:72-91), (min, max) pairs [axis][triangle]:
@@ -540,50 +530,80 @@ __global__ __launch_bounds__(kThreads) void k_emit(const TileDesc* __restrict__ 
   }
 }
 
-// One workgroup per group: all remaining levels of the group's subtree(s).
-// With orig, the pending region is renumbered (by the last k_emit): element values
-// are positions, bb is bbR with stride N = m, and orig maps positions back to
-// triangle ids where the tree order is written.
-// 37 KB of LDS and at most 128 VGPRs, so four groups reside per CU.
-__global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restrict__ groups,
-                                                         const uint2* __restrict__ V,
-                                                         const float2* __restrict__ bb, uint32_t N,
-                                                         uint32_t n, int L, int level0,
-                                                         uint32_t* __restrict__ P,
-                                                         const uint32_t* __restrict__ orig) {
-  __shared__ uint32_t E[kSubT];
-  __shared__ uint16_t G[kSubT];
+// One workgroup per group: all remaining levels of the group's subtree(s),
+// in LDS.  Elements are their positions in the group's window of bb (the
+// bounds in position order: written by the last k_emit, or the input order of
+// a tree that starts here); orig (optional) maps positions to triangle ids
+// where the tree order is written.
+//
+// A group is one chain of dependent stages (286 compare stages of the sorts
+// over the 11 levels of 2048 elements, and about ten LDS round trips a level),
+// so its latency is the launch: 1M triangles give two groups per CU.  1024
+// threads take a stage in one step, and the keys of all axes are in LDS (six
+// dwords per element), so that no level waits for global memory; the triangle
+// ids of a level's pairs, read from orig, are stored one level later.  A launch
+// of two groups takes 101 us and one of 512 (1M triangles) 163; with 256
+// threads in four rounds per stage and the bounds gathered from memory at
+// every level they took 227 and 268 (8192 groups of 10M triangles gain
+// nothing: there the sorts' LDS traffic binds, 1.5 ms either way).
+// 77 KB of LDS and at most 64 VGPRs: two groups reside per CU.
+constexpr int kSubThreads = 1024;
+__global__ __launch_bounds__(kSubThreads, 8) void k_subtree(const SubGroup* __restrict__ groups,
+                                                            const float2* __restrict__ bb, uint32_t N,
+                                                            uint32_t n, int L, int level0,
+                                                            uint32_t* __restrict__ P,
+                                                            const uint32_t* __restrict__ orig) {
+  __shared__ uint32_t kmin[3][kSubT], kmax[3][kSubT];
   __shared__ unsigned long long K[kSubT];
-  __shared__ uint32_t nodeOff[kSubT / 2 + 1];
-  __shared__ uint32_t nodeArg[kSubT / 2];
+  __shared__ uint16_t E[kSubT], G[kSubT];
+  __shared__ uint16_t nodeOff[kSubT / 2 + 1];
+  __shared__ uint16_t nodeArg[kSubT / 2];
   __shared__ uint32_t gmax;  // largest sort group of the level
-  // once the sorted order is read out, the sort buffer holds the sorted ids
-  // (E2) and their max keys (MK)
+  // once the sorted order is read out, the sort buffer holds the sorted
+  // elements (E2) and their max keys (MK)
   uint32_t* E2 = reinterpret_cast<uint32_t*>(K);
   uint32_t* MK = E2 + kSubT;
+  constexpr int kPer = kSubT / kSubThreads;  // elements per thread
+  static_assert(kSubT / 2 <= kSubThreads, "one node per thread");
 
   const SubGroup g = groups[blockIdx.x];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  uint32_t m = g.size;
-  for (uint32_t i = tid; i < m; i += kThreads) {
-    E[i] = orig ? g.off + i : clampi(V[g.off + i].x, N);
+  const uint32_t tid = threadIdx.x;
+  uint32_t m = min(g.size, kSubT);
+  for (uint32_t i = tid; i < m; i += kSubThreads) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float2 b = bb[(size_t)a * N + g.off + i];
+      kmin[a][i] = fkey(b.x);
+      kmax[a][i] = fkey(b.y);
+    }
+    E[i] = (uint16_t)i;
     G[i] = 0;
   }
   uint32_t f = g.first, c = g.count;
+  // the pair of the previous level's node `tid`: written once its ids are here
+  bool held = false;
+  uint32_t held_h = 0, held_x = 0, held_y = 0;
+  const auto put = [&](uint32_t h, uint32_t x, uint32_t y) {
+    held = true;
+    held_h = h;
+    held_x = orig ? orig[g.off + x] : g.off + x;
+    held_y = orig ? orig[g.off + y] : g.off + y;
+  };
+  const auto flush = [&]() {
+    if (held) {
+      P[2 * (size_t)held_h] = held_x;
+      P[2 * (size_t)held_h + 1] = held_y;
+    }
+    held = false;
+  };
   __syncthreads();
   for (int level = level0; level < L && m > 0; ++level) {
     const int a = level % 3;
-    const float2* ba = bb + (size_t)a * N;  // (min, max) on this level's axis
-    // every thread's key loads are issued together, before the offsets
-    constexpr int kPer = kSubT / kThreads;  // elements per thread
-    uint32_t kv[kPer];
-#pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
-      kv[r] = i < m ? fkey(ba[E[i]].x) : 0u;
+    if (tid <= c) nodeOff[tid] = (uint16_t)(2u * (uint32_t)desc_count(f, f + tid, n));
+    if (tid == 0) {
+      gmax = 0;
+      if (c == kSubThreads) nodeOff[c] = (uint16_t)m;
     }
-    for (uint32_t j = tid; j <= c; j += kThreads) nodeOff[j] = 2u * (uint32_t)desc_count(f, f + j, n);
-    if (tid == 0) gmax = 0;
     __syncthreads();
     // Sort groups are the remainders of one node of the previous level: the
     // ranges of this level's node pairs (2q, 2q+1), contiguous and in order,
@@ -592,35 +612,37 @@ __global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restr
     // (log2(S) bitonic phases instead of log2(M)); otherwise the whole region
     // is sorted on (group, key, position).
     const uint32_t ng = (c + 1) / 2;
-    for (uint32_t q = tid; q < ng; q += kThreads)
-      atomicMax(&gmax, nodeOff[min(2 * q + 2, c)] - nodeOff[2 * q]);
+    if (tid < ng) atomicMax(&gmax, (uint32_t)nodeOff[min(2 * tid + 2, c)] - nodeOff[2 * tid]);
     uint32_t M = 1;
     while (M < m) M <<= 1;
     __syncthreads();
+    const uint32_t gm = gmax;
     uint32_t S = 2;
-    while (S < gmax) S <<= 1;
+    while (S < gm) S <<= 1;
     const bool seg = (uint64_t)ng * S <= kSubT;
     const uint32_t span = seg ? ng * S : M;  // sorted entries
     const uint32_t top = seg ? S : M;        // size of one sorted run
-    for (uint32_t q = tid; q < span; q += kThreads) K[q] = ~0ull;
+    for (uint32_t q = tid; q < span; q += kSubThreads) K[q] = ~0ull;
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
+      const uint32_t i = tid + r * kSubThreads;
       if (i >= m) break;
-      const unsigned long long key = kv[r];
+      const unsigned long long key = kmin[a][E[i]];
+      const uint32_t q = G[i];
       if (seg) {
-        const uint32_t q = G[i], p = i - nodeOff[2 * q];
+        const uint32_t p = i - nodeOff[2 * q];
         K[q * S + p] = (key << 11) | p;
       } else {
-        K[i] = ((unsigned long long)G[i] << 43) | (key << 11) | i;
+        K[i] = ((unsigned long long)q << 43) | (key << 11) | i;
       }
     }
+    flush();
     __syncthreads();
     for (uint32_t k = 2; k <= top; k <<= 1) {
       for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-        for (uint32_t t = tid; t < span / 2; t += kThreads) {
-          const uint32_t i = ((t & ~(j - 1)) << 1) | (t & (j - 1));  // j is a power of two
+        if (tid < span / 2) {
+          const uint32_t i = ((tid & ~(j - 1)) << 1) | (tid & (j - 1));  // j is a power of two
           const uint32_t ixj = i + j;
           const bool up = (i & k & (top - 1)) == 0;  // every run ascending at k == top
           const unsigned long long x = K[i], y = K[ixj];
@@ -629,9 +651,9 @@ __global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restr
             K[ixj] = x;
           }
         }
-        // With j <= 64, the pairs of thread t lie in entries [2t - 2t%128,
-        // +128): wave w owns entries 128w + 512r .. +127 in this stage and in
-        // the next one if that also has j <= 64, so a wave barrier orders it.
+        // With j <= 64, the pairs of a wave's threads lie in its own 128
+        // entries in this stage, and in the next one if that also has
+        // j <= 64, so a wave barrier orders it.
         const uint32_t jn = j > 1 ? (j >> 1) : k;  // next stage: (k, j/2) or (2k, k)
         if ((j == 1 && k == top) || j > 64 || jn > 64) {
           __syncthreads();
@@ -643,26 +665,27 @@ __global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restr
       }
     }
     const bool last = level == L - 1;
-    uint32_t ev[kPer];
+    uint32_t ev[kPer], kv[kPer], qv[kPer];
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
-      uint32_t e = 0;
+      const uint32_t i = tid + r * kSubThreads;
+      ev[r] = kv[r] = qv[r] = 0;
       if (i < m) {
+        const uint32_t q = G[i];
         if (seg) {
-          const uint32_t q = G[i], gs = nodeOff[2 * q];
-          e = E[gs + (uint32_t)(K[q * S + (i - gs)] & 0x7FFull)];
+          const uint32_t gs = nodeOff[2 * q];
+          ev[r] = E[gs + (uint32_t)(K[q * S + (i - gs)] & 0x7FFull)];
         } else {
-          e = E[(uint32_t)(K[i] & 0x7FFull)];
+          ev[r] = E[(uint32_t)(K[i] & 0x7FFull)];
         }
+        qv[r] = q;
+        kv[r] = kmax[a][ev[r]];
       }
-      ev[r] = e;
-      kv[r] = (i < m && !last) ? fkey(ba[e].y) : 0u;  // max keys, issued together
     }
     __syncthreads();  // every sorted slot is read: E2 and MK overwrite them
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
+      const uint32_t i = tid + r * kSubThreads;
       if (i < m) {
         E2[i] = ev[r];
         MK[i] = kv[r];
@@ -670,96 +693,55 @@ __global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restr
     }
     __syncthreads();
     if (last) {
-      for (uint32_t j = tid; j < c; j += kThreads) {
-        const uint32_t o = nodeOff[j];
-        P[2 * (size_t)(f + j)] = orig ? orig[E2[o]] : E2[o];
-        P[2 * (size_t)(f + j) + 1] = orig ? orig[E2[o + 1]] : E2[o + 1];
-      }
+      if (tid < c) put(f + tid, E2[nodeOff[tid]], E2[nodeOff[tid] + 1]);
       break;
     }
-    // first maximum of the max key over each node's [o + 1, e): one wave per
-    // node while nodes are large, one thread per node once a sort group (two
-    // nodes) holds at most 64 entries
-    if (gmax > 64) {
-      for (uint32_t j = wave; j < c; j += kThreads / 64) {
-        const uint32_t o = nodeOff[j], e = nodeOff[j + 1];
-        uint32_t bk = 0, bp = 0xFFFFFFFFu;
-        for (uint32_t i = o + 1 + lane; i < e; i += 64) {
+    // first maximum of the max key over each node's [o + 1, e): W lanes per
+    // node, as many as there are threads for
+    uint32_t W = 64;
+    while (W > 1 && W * c > kSubThreads) W >>= 1;
+    for (uint32_t j0 = 0; j0 < c; j0 += kSubThreads / W) {
+      const uint32_t j = j0 + tid / W, w = tid & (W - 1);
+      uint32_t bk = 0, bp = 0xFFFFFFFFu, o = 0, e = 0;
+      if (j < c) {
+        o = nodeOff[j];
+        e = nodeOff[j + 1];
+        for (uint32_t i = o + 1 + w; i < e; i += W) {
           const uint32_t k = MK[i];
           if (k > bk) {
             bk = k;
             bp = i;
           }
         }
-        for (int off = 32; off > 0; off >>= 1) {
-          const uint32_t ok = __shfl_xor(bk, off), op = __shfl_xor(bp, off);
-          if (ok > bk || (ok == bk && op < bp)) {
-            bk = ok;
-            bp = op;
-          }
-        }
-        if (lane == 0) nodeArg[j] = (bp > o && bp < e) ? bp : o + 1;  // sizes are >= 2
       }
-    } else {
-      for (uint32_t j = tid; j < c; j += kThreads) {
-        const uint32_t o = nodeOff[j], e = nodeOff[j + 1];
-        uint32_t bk = 0, bp = 0xFFFFFFFFu;
-        for (uint32_t i = o + 1; i < e; ++i) {
-          const uint32_t k = MK[i];
-          if (k > bk) {
-            bk = k;
-            bp = i;
-          }
+      for (uint32_t off = W >> 1; off > 0; off >>= 1) {
+        const uint32_t ok = __shfl_xor(bk, off), op = __shfl_xor(bp, off);
+        if (ok > bk || (ok == bk && op < bp)) {
+          bk = ok;
+          bp = op;
         }
-        nodeArg[j] = (bp > o && bp < e) ? bp : o + 1;
       }
+      if (j < c && w == 0) nodeArg[j] = (uint16_t)((bp > o && bp < e) ? bp : o + 1);  // sizes are >= 2
     }
     __syncthreads();
-    {
-      // each thread's pairs (c <= kSubT / 2): last-level keys loaded together
-      constexpr int kPairs = kSubT / 2 / kThreads;
-      const float2* knew = bb + (size_t)((L - 1) % 3) * N;
-      uint32_t px[kPairs], py[kPairs];
-      float fx[kPairs], fy[kPairs];
-#pragma unroll
-      for (int r = 0; r < kPairs; ++r) {
-        const uint32_t j = tid + r * kThreads;
-        px[r] = j < c ? E2[nodeOff[j]] : 0u;
-        py[r] = j < c ? E2[nodeArg[j]] : 0u;
-        fx[r] = j < c ? knew[px[r]].x : 0.0f;
-        fy[r] = j < c ? knew[py[r]].x : 0.0f;
-      }
-#pragma unroll
-      for (int r = 0; r < kPairs; ++r) {
-        const uint32_t j = tid + r * kThreads;
-        if (j < c) write_pair_k(f + j, px[r], py[r], fx[r], fy[r], level, L, bb, N, P, orig);
-      }
+    if (tid < c) {
+      const uint32_t x = E2[nodeOff[tid]], y = E2[nodeArg[tid]];
+      const bool swap = second_first(x, y, level, L, [&](int ax, uint32_t i) { return kmin[ax][i]; });
+      put(f + tid, swap ? y : x, swap ? x : y);
     }
     // compaction: the node of sorted position i is one of its sort group's
     // two nodes (groups are contiguous and keep their ranges through the
-    // sort); all reads of G come before the writes
-    uint32_t nodeOf[kPer];
+    // sort); G and E were read above
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
-      uint32_t j = 0;
-      if (i < m) {
-        j = 2u * G[i];
-        if (j + 1 < c && i >= nodeOff[j + 1]) ++j;
-      }
-      nodeOf[r] = j;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kThreads;
+      const uint32_t i = tid + r * kSubThreads;
       if (i >= m) break;
-      const uint32_t lo = nodeOf[r], o = nodeOff[lo];
-      if (i >= o + 2) {
-        const uint32_t val = (i == nodeArg[lo]) ? E2[o + 1] : E2[i];
-        const uint32_t dst = i - 2 * (lo + 1);
-        E[dst] = val;
-        G[dst] = (uint16_t)lo;
+      uint32_t j = 2u * qv[r];
+      if (j + 1 < c && i >= nodeOff[j + 1]) ++j;
+      if (i >= nodeOff[j] + 2u) {
+        const uint32_t dst = i - 2 * (j + 1);
+        E[dst] = (uint16_t)((i == nodeArg[j]) ? E2[nodeOff[j] + 1] : ev[r]);
+        G[dst] = (uint16_t)j;
       }
     }
     __syncthreads();
@@ -770,6 +752,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_subtree(const SubGroup* __restr
     f = (uint32_t)nf;
     c = (uint32_t)nc;
   }
+  flush();
 }
 
 // applyIndices (rebuilder.cu:217-245): gather every per-triangle array.
@@ -1118,11 +1101,9 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   AUR_LAUNCH_CHECK(ctx, "nmh level kernels");
   if (level0 > 0) {
     // the subtree phase on positions (renumbered by the last k_emit)
-    k_subtree<<<(uint32_t)sub.size(), kThreads, 0, s>>>(dsub.p, Vcur, bbR.p, m0, n, L, level0,
-                                                        ctx->perm.p, Ka.p);
+    k_subtree<<<(uint32_t)sub.size(), kSubThreads, 0, s>>>(dsub.p, bbR.p, m0, n, L, level0, ctx->perm.p, Ka.p);
   } else {
-    k_subtree<<<(uint32_t)sub.size(), kThreads, 0, s>>>(dsub.p, Vcur, bb.p, N, n, L, level0,
-                                                        ctx->perm.p, nullptr);
+    k_subtree<<<(uint32_t)sub.size(), kSubThreads, 0, s>>>(dsub.p, bb.p, N, n, L, level0, ctx->perm.p, nullptr);
   }
   AUR_LAUNCH_CHECK(ctx, "k_subtree");
 
