@@ -38,9 +38,8 @@ aur_status aur_scene_add(aur_context* ctx, uint32_t count, const float* vertices
   if (st != AUR_OK) return st;
   st = aur_lights_upload(ctx, num_lights, lights);
   if (st != AUR_OK) return st;
-  st = aur::nmh_build(ctx, nullptr);
+  st = aur::nmh_build(ctx, nullptr, false);
   if (st != AUR_OK) return st;
-  AUR_HIP(ctx, hipStreamSynchronize(ctx->stream));
   auto sc = std::make_unique<aur::SceneStore>();
   sc->count = ctx->count;
   sc->levels = ctx->levels;

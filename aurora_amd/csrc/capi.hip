@@ -60,6 +60,11 @@ aur_status aur_create(int32_t device, aur_context** out) {
     delete ctx;
     return AUR_ERR_DEVICE;
   }
+  if (hipHostMalloc((void**)&ctx->root_host, sizeof(aur::NodeRec)) != hipSuccess) {
+    (void)hipStreamDestroy(ctx->stream);
+    delete ctx;
+    return AUR_ERR_OOM;
+  }
   // device address of the allocation-free entry points' scratch on this
   // device (once per device); on failure only those entry points refuse
   (void)aur::scratch_setup(device);
@@ -250,12 +255,7 @@ aur_status aur_lights_upload(aur_context* ctx, uint32_t count, const aur_light* 
 aur_status aur_rebuild_nmh(aur_context* ctx, aur_build_stats* stats) {
   if (!ctx) return AUR_ERR_INVALID_ARG;
   AUR_HIP(ctx, hipSetDevice(ctx->device));
-  aur_status st = aur::nmh_build(ctx, stats);
-  if (st != AUR_OK) return st;
-  st = aur::generate_tb(ctx);
-  if (st != AUR_OK) return st;
-  AUR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return AUR_OK;
+  return aur::nmh_build(ctx, stats, true);
 }
 
 aur_status aur_generate_tb(aur_context* ctx) {

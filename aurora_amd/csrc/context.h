@@ -184,7 +184,13 @@ struct FrameState {
 
 }  // namespace aur
 
+namespace aur {
+struct BuildPlan;  // nmh_build.hip
+}
+
 struct aur_context {
+  aur_context();
+  ~aur_context();
   int device = 0;
   hipStream_t stream = nullptr;
   std::string last_error;
@@ -203,6 +209,13 @@ struct aur_context {
   uint32_t count = 0;
   aur::DevBuf<float> in_vertices, in_normals, in_texcoords;
   aur::DevBuf<uint16_t> in_shader_ids;
+
+  // tree build: scratch and descriptors kept for the next one, the plan they
+  // belong to, timing events and the host copy of record 0
+  aur::DevBuf<uint8_t> build_scratch, build_desc;
+  std::unique_ptr<aur::BuildPlan> build_plan;
+  hipEvent_t build_event[2] = {nullptr, nullptr};
+  aur::NodeRec* root_host = nullptr;  // pinned
 
   // tree-order geometry and traversal records (valid after the build)
   bool built = false;
@@ -289,7 +302,8 @@ namespace aur {
 hipError_t scratch_setup(int device);
 void* scratch_ptr(int device);
 
-aur_status nmh_build(aur_context* ctx, aur_build_stats* stats);
+// tangents: also the tangent frames (aur_generate_tb).  Synchronous.
+aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents);
 aur_status generate_tb(aur_context* ctx);
 aur_status trace_closest(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_hit* hits);
 aur_status trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int32_t* ids);

@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "context.h"
@@ -82,25 +83,23 @@ __device__ inline void write_pair(uint32_t h, uint32_t x, uint32_t y, int level,
 
 // computeTriangleBounds (rebuilder.cu:72-91), (min, max) pairs [axis][triangle]:
 // one 8-byte load gives both keys of a triangle on an axis.
-__global__ void k_bounds(const float* __restrict__ v, uint32_t N, float2* __restrict__ bb) {
+// With V also the identity order with the axis-0 max keys (the sort's payload)
+// and the first level's axis-0 sort keys K.
+__global__ void k_bounds(const float* __restrict__ v, uint32_t N, float2* __restrict__ bb, uint2* __restrict__ V,
+                         uint32_t* __restrict__ K) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   const float* p = v + (size_t)i * 9;
 #pragma unroll
-  for (int a = 0; a < 3; ++a)
-    bb[(size_t)a * N + i] = make_float2(fminf(fminf(p[3 * a], p[3 * a + 1]), p[3 * a + 2]),
-                                        fmaxf(fmaxf(p[3 * a], p[3 * a + 1]), p[3 * a + 2]));
-}
-
-// Identity order with the axis-0 max keys (the sort's payload: triangle id,
-// max key), and (when K is given) the first level's axis-0 sort keys.
-__global__ void k_iota(uint2* __restrict__ V, uint32_t N, const float2* __restrict__ bb0,
-                       uint32_t* __restrict__ K) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const float2 b = bb0[i];
-  V[i] = make_uint2(i, fkey(b.y));
-  if (K) K[i] = fkey(b.x);
+  for (int a = 0; a < 3; ++a) {
+    const float2 b = make_float2(fminf(fminf(p[3 * a], p[3 * a + 1]), p[3 * a + 2]),
+                                 fmaxf(fmaxf(p[3 * a], p[3 * a + 1]), p[3 * a + 2]));
+    bb[(size_t)a * N + i] = b;
+    if (a == 0 && V) {
+      V[i] = make_uint2(i, fkey(b.y));
+      K[i] = fkey(b.x);
+    }
+  }
 }
 
 // Indices read back from device arrays are clamped to [0, N) before they
@@ -785,7 +784,9 @@ __device__ inline void slab_of(const float* v, int a, float& lo, float& hi) {
 }
 
 // Traversal records (common.h): thread K writes record K, of node K - 1.
-__global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec* __restrict__ nodes) {
+// Record 0 also goes to host memory (root).
+__global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec* __restrict__ nodes,
+                               NodeRec* __restrict__ root) {
   const uint32_t K = blockIdx.x * blockDim.x + threadIdx.x;
   if (K > n) return;
   NodeRec r = {};
@@ -796,6 +797,7 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
 #pragma unroll
       for (int i = 0; i < 18; ++i) r.ref[0] = fmaxf(r.ref[0], fabsf(v[18 * k + i]));
     nodes[0] = r;
+    *root = r;
     return;
   }
   const uint32_t k = K - 1;
@@ -885,35 +887,53 @@ __global__ void k_generate_tb(const float* __restrict__ normals, uint32_t N,
 
 inline uint32_t blocks(uint64_t n, uint32_t b) { return (uint32_t)((n + b - 1) / b); }
 
+// Above this much, a build's scratch is freed when it ends.
+constexpr size_t kKeepScratch = 256ull << 20;
+
+}  // namespace
+
 struct LevelPlan {
   int level;
   uint32_t m, first, nchildren, ngroups, ntiles, nchunks;
   size_t child_base, group_base, tile_base, chunk_base;
 };
 
-}  // namespace
+struct BuildPlan {
+  uint32_t count = 0;  // triangles (0: none)
+  int L = 0, level0 = 0;
+  uint32_t nsub = 0;
+  size_t max_tiles = 1, max_children = 1, max_chunks = 1;
+  std::vector<LevelPlan> levels;
+  std::vector<uint8_t> image;  // every descriptor array; empty once on the device
+  size_t at_tiles = 0, at_children = 0, at_groups = 0, at_chunk_tiles = 0, at_sub = 0;
+};
 
-aur_status generate_tb(aur_context* ctx) {
-  if (!ctx->built) return ctx->fail(AUR_ERR_STATE, "generate_tb: geometry not built");
+// Queues the tangent frames of the tree-order normals.
+static aur_status launch_tb(aur_context* ctx) {
   const uint32_t N = ctx->count;
   AUR_HIP(ctx, ctx->tangents.reserve((size_t)N * 9));
   AUR_HIP(ctx, ctx->bitangents.reserve((size_t)N * 9));
   k_generate_tb<<<blocks(N, 256), 256, 0, ctx->stream>>>(ctx->normals.p, N, ctx->tangents.p,
                                                          ctx->bitangents.p);
   AUR_LAUNCH_CHECK(ctx, "k_generate_tb");
-  ctx->has_tb = true;
   return AUR_OK;
 }
 
-aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
-  const uint32_t N = ctx->count;
-  if (N < 2 || (N & 1u)) return ctx->fail(AUR_ERR_STATE, "rebuild: no even-sized geometry uploaded");
+aur_status generate_tb(aur_context* ctx) {
+  if (!ctx->built) return ctx->fail(AUR_ERR_STATE, "generate_tb: geometry not built");
+  const aur_status st = launch_tb(ctx);
+  ctx->has_tb = ctx->has_tb || st == AUR_OK;
+  return st;
+}
+
+// The host's part of a build: it depends on the triangle count alone, so the
+// context keeps the last one and its device copy.
+static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+void make_plan(uint32_t N, BuildPlan& bp) {
   const uint32_t n = N / 2;
   int L = 0;
   for (uint32_t x = n; x; x >>= 1) ++L;  // log2i(n) + 1
-  hipStream_t s = ctx->stream;
-
-  // ---- host plan (closed forms only; no device data needed) ----
   int level0 = 0;
   if (N > kSubT) {
     level0 = L - 1;
@@ -931,7 +951,8 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   std::vector<GroupDesc> groups;
   uint32_t chunk_count = 0;  // chunks of kChunk tiles of one group, per level
   std::vector<uint32_t> chunk_tiles;  // per level: first tile of each chunk, then the level's tile count
-  std::vector<LevelPlan> plan;
+  std::vector<LevelPlan>& plan = bp.levels;
+  plan.clear();
   size_t max_tiles = 1, max_children = 1, max_chunks = 1;
   for (int l = 0; l < level0; ++l) {
     LevelPlan lp{};
@@ -999,99 +1020,128 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
       sub.push_back(SubGroup{(uint32_t)off, (uint32_t)size, (uint32_t)c0, (uint32_t)(c1 - c0)});
     }
   }
+  bp.count = N;
+  bp.L = L;
+  bp.level0 = level0;
+  bp.nsub = (uint32_t)sub.size();
+  bp.max_tiles = max_tiles;
+  bp.max_children = max_children;
+  bp.max_chunks = max_chunks;
+  // one image of every descriptor array, 256-byte aligned
+  bp.image.clear();
+  const auto put = [&](const void* p, size_t bytes) {
+    const size_t at = bp.image.size();
+    bp.image.resize(align256(at + std::max<size_t>(bytes, 1)));
+    if (bytes) memcpy(bp.image.data() + at, p, bytes);
+    return at;
+  };
+  bp.at_tiles = put(tiles.data(), tiles.size() * sizeof(TileDesc));
+  bp.at_children = put(children.data(), children.size() * sizeof(ChildDesc));
+  bp.at_groups = put(groups.data(), groups.size() * sizeof(GroupDesc));
+  bp.at_chunk_tiles = put(chunk_tiles.data(), chunk_tiles.size() * sizeof(uint32_t));
+  bp.at_sub = put(sub.data(), sub.size() * sizeof(SubGroup));
+}
 
-  // ---- device buffers ----
-  DevBuf<float2> bb;          // (min, max) per axis and triangle
-  DevBuf<float2> bbR;         // the same for the subtree phase's pending region, by position
-  // sort payload (triangle id, max key on the level's axis): the level's
-  // input, the other side of the radix passes, and the emit pass's output
-  DevBuf<uint2> Va, Vb, Vc;
-  DevBuf<uint2> GP, TP, TR;  // (smallest key, passes) per group and tile; emit tiles' key ranges
-  DevBuf<uint32_t> CP;        // passes per offset chunk
-  DevBuf<uint32_t> Ka, Kb, H, O, CS, CB, argpos, dchunk_tiles;
-  DevBuf<uint2> partial;
-  DevBuf<TileDesc> dtiles;
-  DevBuf<ChildDesc> dchildren;
-  DevBuf<GroupDesc> dgroups;
-  DevBuf<SubGroup> dsub;
-  AUR_HIP(ctx, bb.reserve((size_t)3 * N));
-  AUR_HIP(ctx, Va.reserve(N));
-  AUR_HIP(ctx, Vb.reserve(N));
-  AUR_HIP(ctx, ctx->perm.reserve(N));
-  if (!plan.empty()) {
-    AUR_HIP(ctx, Vc.reserve(N));
-    AUR_HIP(ctx, GP.reserve(max_children));
-    AUR_HIP(ctx, TP.reserve(max_tiles));
-    AUR_HIP(ctx, CP.reserve(max_chunks));
-    AUR_HIP(ctx, TR.reserve(max_tiles));
-    AUR_HIP(ctx, Ka.reserve(N));
-    AUR_HIP(ctx, Kb.reserve(N));
-    AUR_HIP(ctx, H.reserve(max_tiles * 256));
-    AUR_HIP(ctx, O.reserve(max_tiles * 256));
-    AUR_HIP(ctx, dchunk_tiles.reserve(chunk_tiles.size()));
-    AUR_HIP(ctx, hipMemcpy(dchunk_tiles.p, chunk_tiles.data(), chunk_tiles.size() * sizeof(uint32_t),
-                           hipMemcpyHostToDevice));
-    AUR_HIP(ctx, CS.reserve(max_chunks * 256));
-    AUR_HIP(ctx, CB.reserve(max_chunks * 256));
-    AUR_HIP(ctx, partial.reserve(max_tiles));
-    AUR_HIP(ctx, argpos.reserve(max_children));
-    AUR_HIP(ctx, dtiles.reserve(tiles.size()));
-    AUR_HIP(ctx, dchildren.reserve(children.size()));
-    AUR_HIP(ctx, dgroups.reserve(groups.size()));
-    AUR_HIP(ctx, hipMemcpy(dtiles.p, tiles.data(), tiles.size() * sizeof(TileDesc), hipMemcpyHostToDevice));
-    AUR_HIP(ctx, hipMemcpy(dchildren.p, children.data(), children.size() * sizeof(ChildDesc),
-                           hipMemcpyHostToDevice));
-    AUR_HIP(ctx, hipMemcpy(dgroups.p, groups.data(), groups.size() * sizeof(GroupDesc),
-                           hipMemcpyHostToDevice));
+aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
+  const uint32_t N = ctx->count;
+  if (N < 2 || (N & 1u)) return ctx->fail(AUR_ERR_STATE, "rebuild: no even-sized geometry uploaded");
+  const uint32_t n = N / 2;
+  hipStream_t s = ctx->stream;
+  if (!ctx->build_plan) ctx->build_plan = std::make_unique<BuildPlan>();
+  BuildPlan& bp = *ctx->build_plan;
+  if (bp.count != N) {
+    bp.count = 0;  // until the device copy is whole
+    BuildPlan next;
+    make_plan(N, next);
+    AUR_HIP(ctx, ctx->build_desc.reserve(next.image.size()));
+    AUR_HIP(ctx, hipMemcpyAsync(ctx->build_desc.p, next.image.data(), next.image.size(), hipMemcpyHostToDevice, s));
+    AUR_HIP(ctx, hipStreamSynchronize(s));
+    next.image = std::vector<uint8_t>();
+    bp = std::move(next);
   }
+  const int L = bp.L, level0 = bp.level0;
+  const std::vector<LevelPlan>& plan = bp.levels;
+  const auto desc = [&](size_t at) { return ctx->build_desc.p + at; };
+  const TileDesc* dtiles = reinterpret_cast<const TileDesc*>(desc(bp.at_tiles));
+  const ChildDesc* dchildren = reinterpret_cast<const ChildDesc*>(desc(bp.at_children));
+  const GroupDesc* dgroups = reinterpret_cast<const GroupDesc*>(desc(bp.at_groups));
+  const uint32_t* dchunk_tiles = reinterpret_cast<const uint32_t*>(desc(bp.at_chunk_tiles));
+  const SubGroup* dsub = reinterpret_cast<const SubGroup*>(desc(bp.at_sub));
+
+  // ---- device scratch, one allocation ----
   // pending triangles when the subtree phase starts
   const uint32_t m0 = level0 > 0 ? (uint32_t)(N - 2 * ((1ull << level0) - 1)) : N;
-  if (level0 > 0) AUR_HIP(ctx, bbR.reserve((size_t)3 * m0));
-  AUR_HIP(ctx, dsub.reserve(sub.size()));
-  AUR_HIP(ctx, hipMemcpy(dsub.p, sub.data(), sub.size() * sizeof(SubGroup), hipMemcpyHostToDevice));
+  size_t ws = 0;
+  const auto take = [&](size_t bytes) {
+    const size_t at = ws;
+    ws = align256(ws + bytes);
+    return at;
+  };
+  const bool large = !plan.empty();  // levels of groups above one workgroup's LDS
+  const size_t at_bb = take((size_t)3 * N * sizeof(float2));  // (min, max) per axis and triangle
+  // the same for the subtree phase's pending region, by position
+  const size_t at_bbR = take(large ? (size_t)3 * m0 * sizeof(float2) : 0);
+  // sort payload (triangle id, max key on the level's axis): the level's
+  // input, the other side of the radix passes, and the emit pass's output
+  const size_t vb = large ? (size_t)N * sizeof(uint2) : 0, kb = large ? (size_t)N * sizeof(uint32_t) : 0;
+  const size_t at_V[3] = {take(vb), take(vb), take(vb)}, at_K[2] = {take(kb), take(kb)};
+  const size_t tb = large ? bp.max_tiles : 0, cb = large ? bp.max_chunks : 0, nb = large ? bp.max_children : 0;
+  // (smallest key, passes) per group and tile, emit tiles' key ranges, passes
+  // per offset chunk, first maxima
+  const size_t at_GP = take(nb * sizeof(uint2)), at_TP = take(tb * sizeof(uint2)), at_TR = take(tb * sizeof(uint2));
+  const size_t at_CP = take(cb * 4), at_partial = take(tb * sizeof(uint2)), at_argpos = take(nb * 4);
+  const size_t at_H = take(tb * 256 * 4), at_O = take(tb * 256 * 4), at_CS = take(cb * 256 * 4), at_CB = take(cb * 256 * 4);
+  AUR_HIP(ctx, ctx->build_scratch.reserve(ws));
+  AUR_HIP(ctx, ctx->perm.reserve(N));
+  const auto u2 = [&](size_t at) { return reinterpret_cast<uint2*>(ctx->build_scratch.p + at); };
+  const auto u1 = [&](size_t at) { return reinterpret_cast<uint32_t*>(ctx->build_scratch.p + at); };
+  float2* const bb = reinterpret_cast<float2*>(ctx->build_scratch.p + at_bb);
+  float2* const bbR = reinterpret_cast<float2*>(ctx->build_scratch.p + at_bbR);
+  uint2 *const GP = u2(at_GP), *const TP = u2(at_TP), *const TR = u2(at_TR), *const partial = u2(at_partial);
+  uint32_t *const Ka = u1(at_K[0]), *const Kb = u1(at_K[1]), *const CP = u1(at_CP), *const argpos = u1(at_argpos);
+  uint32_t *const H = u1(at_H), *const O = u1(at_O), *const CS = u1(at_CS), *const CB = u1(at_CB);
 
-  hipEvent_t e0, e1;
-  AUR_HIP(ctx, hipEventCreate(&e0));
-  AUR_HIP(ctx, hipEventCreate(&e1));
+  hipEvent_t& e0 = ctx->build_event[0];
+  hipEvent_t& e1 = ctx->build_event[1];
+  if (!e0) AUR_HIP(ctx, hipEventCreate(&e0));
+  if (!e1) AUR_HIP(ctx, hipEventCreate(&e1));
   AUR_HIP(ctx, hipEventRecord(e0, s));
 
-  k_bounds<<<blocks(N, 256), 256, 0, s>>>(ctx->in_vertices.p, N, bb.p);
   // level 0's keys come with the identity order; every later level's keys
   // and max keys are gathered by the previous level's emit pass
-  uint2* Vcur = Va.p;  // the level's input (k_iota's, then the previous emit's output)
-  uint2* Valt = Vb.p;  // the other side of the radix passes
-  uint2* Vout = Vc.p;  // the emit pass's output
-  k_iota<<<blocks(N, 256), 256, 0, s>>>(Vcur, N, bb.p, plan.empty() ? nullptr : Ka.p);
-  k_fill0<<<blocks(N, 256), 256, 0, s>>>(ctx->perm.p, N);
-  if (!plan.empty()) k_fill0<<<blocks(max_chunks * 256, 256), 256, 0, s>>>(CS.p, (uint32_t)(max_chunks * 256));
+  uint2* Vcur = u2(at_V[0]);  // the level's input (k_bounds', then the previous emit's output)
+  uint2* Valt = u2(at_V[1]);  // the other side of the radix passes
+  uint2* Vout = u2(at_V[2]);  // the emit pass's output
+  k_bounds<<<blocks(N, 256), 256, 0, s>>>(ctx->in_vertices.p, N, bb, large ? Vcur : nullptr, Ka);
+  if (large) k_fill0<<<blocks(bp.max_chunks * 256, 256), 256, 0, s>>>(CS, (uint32_t)(bp.max_chunks * 256));
   for (size_t li = 0; li < plan.size(); ++li) {
     const LevelPlan& lp = plan[li];
-    const TileDesc* tl = dtiles.p + lp.tile_base;
-    const ChildDesc* ch = dchildren.p + lp.child_base;
-    const GroupDesc* gr = dgroups.p + lp.group_base;
+    const TileDesc* tl = dtiles + lp.tile_base;
+    const ChildDesc* ch = dchildren + lp.child_base;
+    const GroupDesc* gr = dgroups + lp.group_base;
     // the previous level's nodes: group g of this level is node g's remainder
-    const ChildDesc* prev = li == 0 ? nullptr : dchildren.p + plan[li - 1].child_base;
-    uint32_t *kin = Ka.p, *kout = Kb.p;
+    const ChildDesc* prev = li == 0 ? nullptr : dchildren + plan[li - 1].child_base;
+    uint32_t *kin = Ka, *kout = Kb;
     uint2 *vin = Vcur, *vout = Valt;
     // every launch of a pass skips the groups that need fewer passes
     for (uint32_t pass = 0; pass < 4; ++pass) {
-      k_radix_hist<<<lp.ntiles, kThreads, 0, s>>>(tl, gr, TP.p, kin, pass, H.p, CS.p);
-      k_radix_group_scan<<<lp.ngroups, kThreads, 0, s>>>(gr, GP.p, TP.p, CP.p, prev, TR.p, pass, CS.p, CB.p);
-      k_radix_chunk_offsets<<<lp.nchunks, kThreads, 0, s>>>(dchunk_tiles.p + lp.chunk_base, CP.p, pass,
-                                                            H.p, CB.p, O.p);
-      k_radix_scatter<<<lp.ntiles, kThreads, 0, s>>>(tl, TP.p, kin, vin, pass, O.p, lp.m, kout, vout);
+      k_radix_hist<<<lp.ntiles, kThreads, 0, s>>>(tl, gr, TP, kin, pass, H, CS);
+      k_radix_group_scan<<<lp.ngroups, kThreads, 0, s>>>(gr, GP, TP, CP, prev, TR, pass, CS, CB);
+      k_radix_chunk_offsets<<<lp.nchunks, kThreads, 0, s>>>(dchunk_tiles + lp.chunk_base, CP, pass,
+                                                            H, CB, O);
+      k_radix_scatter<<<lp.ntiles, kThreads, 0, s>>>(tl, TP, kin, vin, pass, O, lp.m, kout, vout);
       std::swap(kin, kout);
       std::swap(vin, vout);
     }
     // each group's sorted data is in Vcur or Valt (group_passes); the keys
     // are not read again, so Ka takes the next level's
     const bool last = li + 1 == plan.size();
-    k_argmax_partial<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, TP.p, Vcur, Valt, partial.p);
+    k_argmax_partial<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, TP, Vcur, Valt, partial);
     k_argmax_combine<<<blocks(lp.nchildren, kThreads / 64), kThreads, 0, s>>>(ch, lp.nchildren,
-                                                                              partial.p, argpos.p);
-    k_emit<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, argpos.p, TP.p, Vcur, Valt, Vout, lp.first, lp.level, L,
-                                          bb.p, N, ctx->perm.p, last ? nullptr : Ka.p, TR.p,
-                                          last ? bbR.p : nullptr, last ? Ka.p : nullptr, m0);
+                                                                              partial, argpos);
+    k_emit<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, argpos, TP, Vcur, Valt, Vout, lp.first, lp.level, L,
+                                          bb, N, ctx->perm.p, last ? nullptr : Ka, TR,
+                                          last ? bbR : nullptr, last ? Ka : nullptr, m0);
     // rotate: the emit output is the next level's input
     uint2* const free_buf = Vcur;
     Vcur = Vout;
@@ -1101,9 +1151,9 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
   AUR_LAUNCH_CHECK(ctx, "nmh level kernels");
   if (level0 > 0) {
     // the subtree phase on positions (renumbered by the last k_emit)
-    k_subtree<<<(uint32_t)sub.size(), kSubThreads, 0, s>>>(dsub.p, bbR.p, m0, n, L, level0, ctx->perm.p, Ka.p);
+    k_subtree<<<bp.nsub, kSubThreads, 0, s>>>(dsub, bbR, m0, n, L, level0, ctx->perm.p, Ka);
   } else {
-    k_subtree<<<(uint32_t)sub.size(), kSubThreads, 0, s>>>(dsub.p, bb.p, N, n, L, level0, ctx->perm.p, nullptr);
+    k_subtree<<<bp.nsub, kSubThreads, 0, s>>>(dsub, bb, N, n, L, level0, ctx->perm.p, nullptr);
   }
   AUR_LAUNCH_CHECK(ctx, "k_subtree");
 
@@ -1118,30 +1168,37 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats) {
                                                    ctx->in_shader_ids.p, ctx->vertices.p,
                                                    ctx->normals.p, ctx->texcoords.p,
                                                    ctx->shader_ids.p);
-  k_node_records<<<blocks((uint64_t)n + 1, 256), 256, 0, s>>>(ctx->vertices.p, n, ctx->nodes.p);
+  k_node_records<<<blocks((uint64_t)n + 1, 256), 256, 0, s>>>(ctx->vertices.p, n, ctx->nodes.p, ctx->root_host);
   AUR_LAUNCH_CHECK(ctx, "gather/node records");
   AUR_HIP(ctx, hipEventRecord(e1, s));
-  AUR_HIP(ctx, hipEventSynchronize(e1));
+  const aur_status tangents_status = tangents ? launch_tb(ctx) : AUR_OK;
+  AUR_HIP(ctx, hipStreamSynchronize(s));
   float ms = 0.0f;
   AUR_HIP(ctx, hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   // record 0, for launches that start every ray at the root without reading it
-  NodeRec root;
-  AUR_HIP(ctx, hipMemcpyAsync(&root, ctx->nodes.p, sizeof(root), hipMemcpyDeviceToHost, s));
-  AUR_HIP(ctx, hipStreamSynchronize(s));
-  ctx->root_lo = root.cslab[0];
-  ctx->root_hi = root.cslab[1];
-  ctx->bound = root.ref[0];
+  ctx->root_lo = ctx->root_host->cslab[0];
+  ctx->root_hi = ctx->root_host->cslab[1];
+  ctx->bound = ctx->root_host->ref[0];
+  // A rebuild of the same size (an edit, a deforming mesh) finds its scratch
+  // in place.  Beyond the limit (about 3.3M triangles) the build outweighs the
+  // allocation.
+  if (ws > kKeepScratch) ctx->build_scratch.release();
   ctx->levels = (uint32_t)L;
   ctx->built = true;
-  ctx->has_tb = false;
+  ctx->has_tb = tangents && tangents_status == AUR_OK;
   if (stats) {
     stats->count = N;
     stats->levels = (uint32_t)L;
     stats->build_ms = ms;
   }
-  return AUR_OK;
+  return tangents_status;
 }
 
 }  // namespace aur
+
+aur_context::aur_context() = default;
+aur_context::~aur_context() {
+  for (hipEvent_t e : build_event)
+    if (e) (void)hipEventDestroy(e);
+  if (root_host) (void)hipHostFree(root_host);
+}
