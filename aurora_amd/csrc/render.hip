@@ -384,6 +384,30 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
       });
 }
 
+// Appends a wave's `paths` path entries and `shadows` shadow entries (counts
+// below 2^32) to the queues whose lengths are the two halves of *counter: one
+// atomic per block, whose waves take consecutive parts.  Returns the wave's
+// first positions, packed alike.  Every thread of the block calls it.  One
+// address takes an atomic about every 12 ns: with one per wave, the 16,384
+// waves of a 2^20-path launch took 184 us whatever they computed, now 45 us in
+// blocks of 8 waves (256^2 Cornell frame of 16 samples 2.05 -> 1.46 ms; blocks
+// of 4 waves 1.54, of 16 1.44 there and 1% slower on the others).
+constexpr uint32_t kShadeBlock = 512;
+__device__ __forceinline__ unsigned long long block_append(uint32_t* counter, uint32_t paths, uint32_t shadows) {
+  __shared__ unsigned long long part[kShadeBlock / 64], first;
+  const uint32_t wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63u) == 0) part[wave] = (unsigned long long)paths | ((unsigned long long)shadows << 32);
+  __syncthreads();
+  unsigned long long before = 0;
+  for (uint32_t i = 0; i < wave; ++i) before += part[i];
+  if (threadIdx.x == kShadeBlock - 1) {  // the last wave's prefix and its own part: the block's total
+    const unsigned long long total = before + part[wave];
+    first = total ? atomicAdd(reinterpret_cast<unsigned long long*>(counter), total) : 0ull;
+  }
+  __syncthreads();
+  return first + before;
+}
+
 // What shading one path vertex leaves to the queues.
 struct ShadeOut {
   bool survive;      // the path continues with ray (o, d)
@@ -535,17 +559,17 @@ __device__ __forceinline__ ShadeOut shade_path(const PbrArgs& a, const JobDev& J
   return out;
 }
 
-// Shading of every queued path, then the appends with one atomic per wave,
-// made where every lane of the wave is active: the next bounce's path queue
-// (with its rays, in queue order) and the shadow queue (slot-major within
-// the wave, so neighbouring items trace to the same light).
+// Shading of every queued path, then the appends: the next bounce's path
+// queue (with its rays, in queue order) and the shadow queue (slot-major
+// within the wave, so neighbouring items trace to the same light).
 template <bool kMulti, bool kRecord>
-__global__ __launch_bounds__(128) void k_pbr_shade(PbrArgs a, uint32_t w, uint32_t bounce,
+__global__ __launch_bounds__(kShadeBlock) void k_pbr_shade(PbrArgs a, uint32_t w, uint32_t bounce,
                                                    const uint32_t* __restrict__ qin,
                                                    uint32_t* __restrict__ qout,
                                                    const JobDev* __restrict__ jobs) {
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n_in = a.counters[2 * w];
+  if (blockIdx.x * blockDim.x >= n_in) return;
   const uint32_t roff = (bounce & 1u) * a.cap, roff_next = a.cap - roff;
   ShadeOut out{false, 0ull, make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
   uint32_t p = 0, jb = 0;
@@ -579,12 +603,7 @@ __global__ __launch_bounds__(128) void k_pbr_shade(PbrArgs a, uint32_t w, uint32
   uint32_t nshadow = 0;
   for (uint32_t sl = 0; sl < a.nslots; ++sl) nshadow += (uint32_t)__popcll(__ballot((out.shadows >> sl) & 1ull));
   const uint64_t ms = __ballot(out.survive);
-  if (nshadow == 0 && ms == 0) return;
-  unsigned long long old = 0;
-  if (lane == 0)
-    old = atomicAdd(reinterpret_cast<unsigned long long*>(a.counters + 2 * (w == 2u ? 0u : w + 1u)),
-                    (unsigned long long)__popcll(ms) | ((unsigned long long)nshadow << 32));
-  old = __shfl(old, 0);
+  const unsigned long long old = block_append(a.counters + 2 * (w == 2u ? 0u : w + 1u), (uint32_t)__popcll(ms), nshadow);
   if (out.survive) {
     const uint32_t pos = (uint32_t)old + (uint32_t)__popcll(ms & below);
     qout[pos] = p;
@@ -879,24 +898,6 @@ struct CwArgs {
 
 constexpr uint32_t kCwHit = 1u, kCwMore = 2u;  // c1.w flags: the ray hit; the pixel continues
 
-// Exclusive prefix of n over the wave's lanes plus one atomic per wave on
-// *counter: the position of this lane's first of n appended entries.  Every
-// lane of the wave calls it.
-__device__ __forceinline__ uint32_t wave_append(uint32_t* counter, uint32_t n) {
-  const uint32_t lane = threadIdx.x & 63u;
-  uint32_t incl = n;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t t = __shfl_up(incl, off);
-    if (lane >= (uint32_t)off) incl += t;
-  }
-  const uint32_t total = __shfl(incl, 63);
-  uint32_t base = 0;
-  if (lane == 0 && total) base = atomicAdd(counter, total);
-  base = __shfl(base, 0);
-  return base + incl - n;
-}
-
 __device__ __forceinline__ CompatRng compat_rng(uint32_t seed, uint32_t pix, uint32_t sample, uint32_t k) {
   CompatRng r{seed, pix, sample, k, U4{0, 0, 0, 0}};
   if (k & 3u) r.cache = philox(U4{pix, sample, 0x40000000u | (k >> 2), 0u}, seed, kKeyCompat);
@@ -928,11 +929,12 @@ __global__ void k_cw_init(CwArgs c, PbrArgs a, uint32_t* __restrict__ qin) {
 // whose stacks go on enter the next level's queue with their next ray.
 // Queue counts as in the PBR passes: word w holds this level's entries;
 // shadow rays and the next level's entries are appended to word wn.
-__global__ __launch_bounds__(kBlock) void k_cw_shade(CwArgs c, PbrArgs a, uint32_t w, uint32_t wn,
+__global__ __launch_bounds__(kShadeBlock) void k_cw_shade(CwArgs c, PbrArgs a, uint32_t w, uint32_t wn,
                                                      const uint32_t* __restrict__ qin,
                                                      uint32_t* __restrict__ qout, uint32_t roff_next) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n = a.counters[2 * w];
+  if (blockIdx.x * blockDim.x >= n) return;
   const bool act = i < n;
   const int kMaxDepth = 8;
   uint32_t ncast = 0;
@@ -1082,15 +1084,15 @@ __global__ __launch_bounds__(kBlock) void k_cw_shade(CwArgs c, PbrArgs a, uint32
   }
   // the cast slots enter the shadow queue slot by slot, each slot's rays in
   // lane order (neighbouring pixels' rays toward the same light sample stay
-  // together for the traversal); one atomic per wave
+  // together for the traversal)
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
   uint32_t total = 0;
   for (uint32_t slot = 0; slot < c.nslots; ++slot)
     total += (uint32_t)__popcll(__ballot(act && ncast && c.contrib[(size_t)slot * c.stride + i].w != 0.0f));
-  uint32_t run = 0;
-  if (lane == 0 && total) run = atomicAdd(&a.counters[2 * wn + 1], total);
-  run = __shfl(run, 0);
+  const uint64_t go = __ballot(more);
+  const unsigned long long old = block_append(a.counters + 2 * wn, (uint32_t)__popcll(go), total);
+  uint32_t run = (uint32_t)(old >> 32);
   for (uint32_t slot = 0; slot < c.nslots && total; ++slot) {
     const size_t e = (size_t)slot * c.stride + i;
     const bool cast = act && ncast && c.contrib[e].w != 0.0f;
@@ -1098,8 +1100,8 @@ __global__ __launch_bounds__(kBlock) void k_cw_shade(CwArgs c, PbrArgs a, uint32
     if (cast) a.sh_queue[run + (uint32_t)__popcll(m & lt)] = (uint32_t)e;
     run += (uint32_t)__popcll(m);
   }
-  const uint32_t p = wave_append(&a.counters[2 * wn], more ? 1u : 0u);
   if (more) {
+    const uint32_t p = (uint32_t)old + (uint32_t)__popcll(go & lt);
     qout[p] = l;
     a.ray_o[roff_next + p] = make_float4(next.pos.x, next.pos.y, next.pos.z, 0.0f);
     a.ray_d[roff_next + p] = make_float4(next.dir.x, next.dir.y, next.dir.z, 0.0f);
@@ -1285,9 +1287,9 @@ void pbr_pass(aur_context* ctx, PbrArgs& a, size_t lds, uint32_t grid_trace,
     uint32_t* qin = fr.queue[b & 1u].p;
     uint32_t* qout = fr.queue[(b + 1u) & 1u].p;
     if (adj)
-      k_pbr_shade<kMulti, true><<<nblocks(cap, 128), 128, 0, s>>>(a, w, b, qin, qout, a.jobs);
+      k_pbr_shade<kMulti, true><<<nblocks(cap, kShadeBlock), kShadeBlock, 0, s>>>(a, w, b, qin, qout, a.jobs);
     else
-      k_pbr_shade<kMulti, false><<<nblocks(cap, 128), 128, 0, s>>>(a, w, b, qin, qout, a.jobs);
+      k_pbr_shade<kMulti, false><<<nblocks(cap, kShadeBlock), kShadeBlock, 0, s>>>(a, w, b, qin, qout, a.jobs);
     const uint32_t parts = (b + 1u < a.max_depth ? 1u : 0u) | sh;
     if (parts)
       trace(wn, parts, ((b + 1u) & 1u) * cap);
@@ -1583,7 +1585,7 @@ aur_status compat_passes(aur_context* ctx, const aur_camera* cam, const aur_rend
         trace(w, 1u | (it > 0 && nslots ? 2u : 0u), (it & 1u) * cap);
         if (it > 0)
           k_cw_resolve<<<nblocks(c.n, kBlock), kBlock, 0, s>>>(c, a, wp, fr.queue[(it + 1u) & 1u].p);
-        k_cw_shade<<<nblocks(c.n, kBlock), kBlock, 0, s>>>(c, a, w, wn, fr.queue[it & 1u].p,
+        k_cw_shade<<<nblocks(c.n, kShadeBlock), kShadeBlock, 0, s>>>(c, a, w, wn, fr.queue[it & 1u].p,
                                                           fr.queue[(it + 1u) & 1u].p, ((it + 1u) & 1u) * cap);
         AUR_LAUNCH_CHECK(ctx, "compat wavefront");
         uint32_t more = 0;
