@@ -1250,7 +1250,14 @@ aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, Pb
   const uint32_t want = !ctx->render_rows_default ? ctx->render_params.stack_lds_rows
                                                   : (kMulti ? kDefaultRenderStackRows : maxrows);
   const uint32_t rows = want >= maxrows ? maxrows : want;
-  lds = (size_t)rows * kBlock * sizeof(float2);
+  // Waves per CU, as for the standalone launches (trace.hip); a render's
+  // neighbouring shadow rays share more lines, so more waves pay: 28 / 24 / 20 /
+  // 16 take 1.46 / 1.46 / 1.52 / 1.55 ms for a 256^2 frame of 2,584 triangles
+  // (32: 1.53), - / 17.5 / 17.6 / 18.6 for the differentiable step of 102,424
+  // and 21.3 / 18.5 / 17.7 / 18.4 for a batch of 16 jobs.
+  const size_t tree_bytes = (size_t)a.job.n_nodes * sizeof(NodeRec);
+  const uint32_t cu_waves = !kMulti && tree_bytes < (1u << 20) ? 28 : 20;
+  lds = lds_for_blocks((size_t)rows * kBlock * sizeof(float2), cu_waves * 64 / kBlock);
   grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, a.job.n_nodes), lds, max_items);
   a.gstack = nullptr;
   a.klds = rows;
