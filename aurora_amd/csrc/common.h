@@ -252,6 +252,17 @@ __host__ __device__ inline uint64_t desc_count(uint64_t a, uint64_t b, uint64_t 
   return total;
 }
 
+// The same in 32 bits (n <= 2^29).
+__device__ inline uint32_t desc_count32(uint32_t a, uint32_t b, uint32_t n) {
+  uint32_t total = 0;
+  while (a < n) {
+    total += (b < n ? b : n) - a;
+    a = 2 * a + 1;
+    b = 2 * b + 1;
+  }
+  return total;
+}
+
 __host__ __device__ inline uint32_t depth_of(uint32_t k) {
   uint32_t d = 0;
   uint32_t x = k + 1;

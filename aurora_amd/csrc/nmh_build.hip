@@ -42,8 +42,9 @@ namespace {
 
 constexpr uint32_t kTile = 2048;  // radix / emit tile (elements)
 constexpr uint32_t kChunk = 32;   // tiles per chunk of the radix offset scan
-constexpr uint32_t kSubT = 2048;  // max elements of an LDS-resident subtree
+constexpr uint32_t kSubT = 4096;  // max elements of an LDS-resident subtree
 constexpr int kThreads = 256;
+constexpr int kSubThreads = 1024;  // k_subtree
 
 struct TileDesc {
   uint32_t start, count, child, group;
@@ -529,45 +530,167 @@ __global__ __launch_bounds__(kThreads) void k_emit(const TileDesc* __restrict__ 
   }
 }
 
+// The keys of sort_slots: positive normal doubles, which v_min_f64 and
+// v_max_f64 order as their bits and return unchanged.
+constexpr unsigned long long kSlotKey = 1ull << 62, kSlotEnd = 0x7FEull << 52;
+
+// LDS position of entry i.  Linear over xor and a permutation of each aligned
+// run of 32 entries; the passes below, whose lanes read entries 4t + const at
+// the small distances, then meet each bank pair once per half wave.
+__device__ __forceinline__ uint32_t slot_pos(uint32_t i) { return i ^ ((i >> 2) & 31u) ^ ((i >> 5) & 1u); }
+
+// Bitonic sort of each aligned run of S entries (S a power of two >= 2) of the
+// entries [0, span), entry i at K[slot_pos(i)], ascending.  A run holds at most
+// `fill` entries, then kSlotEnd.  A merge begins by comparing mirrored entries:
+// every comparison then has the same direction, one minimum and one maximum,
+// and the ends stay where they are, so that comparisons with them are left out.
+// What binds is the chain of passes, each of which reads and writes LDS (4096
+// entries: 512 cycles at 128 bytes per cycle) and waits for it.  A pass takes
+// two stages of four entries per thread in registers, and the first stage of an
+// odd number of them goes alone: 41 passes for 4096 entries instead of 78.
+// Wave w owns entries [256w, 256w + 256) in every pass whose distances are at
+// most 128, so a wave barrier orders those.  (2584 triangles, one group: 184 us
+// with 64-bit compares and selects and entry i at K[i], 144 with minima and
+// maxima and slot_pos, 139 with `fill`.  Three stages of eight entries in 28
+// passes leave half of the waves without work: 158 us.)
+__device__ __forceinline__ void sort_slots(double* K, uint32_t span, uint32_t S, uint32_t fill) {
+  static_assert(kSubThreads == kSubT / 4, "four entries per thread");
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const auto order = [](double& x, double& y) {
+    double lo, hi;  // no canonicalisation before the minimum: never NaN
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(x), "v"(y));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(x), "v"(y));
+    x = lo;
+    y = hi;
+  };
+  const auto barrier = [](bool wave_only) {
+    if (wave_only) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+      __syncthreads();
+    }
+  };
+  // runs of 2 or 4
+  if (4 * tid < span) {
+    const uint32_t p = slot_pos(4 * tid);
+    double x0 = K[p], x1 = K[p ^ slot_pos(1)], x2 = K[p ^ slot_pos(2)], x3 = K[p ^ slot_pos(3)];
+    order(x0, x1);
+    order(x2, x3);
+    if (S > 2) {
+      order(x0, x3);
+      order(x1, x2);
+      order(x0, x1);
+      order(x2, x3);
+    }
+    K[p] = x0;
+    K[p ^ slot_pos(1)] = x1;
+    K[p ^ slot_pos(2)] = x2;
+    K[p ^ slot_pos(3)] = x3;
+  }
+  barrier(S > 4);
+  for (uint32_t k = 8; k <= S; k <<= 1) {
+    uint32_t j = k >> 1, mirror = k - 1;
+    if (__builtin_ctz(k) & 1) {
+#pragma unroll
+      for (uint32_t r = 0; r < 2; ++r) {
+        const uint32_t t = 2 * (tid & ~63u) + 64 * r + lane;
+        const uint32_t i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
+        if (i < span && (i & (S - 1)) < fill) {
+          const uint32_t p = slot_pos(i), q = p ^ slot_pos(mirror);
+          double x = K[p], y = K[q];
+          order(x, y);
+          K[p] = x;
+          K[q] = y;
+        }
+      }
+      barrier(j <= 128);
+      j >>= 1;
+      mirror = 0;
+    }
+    for (; j > 1; j >>= 2) {
+      const uint32_t h = j >> 1;
+      const uint32_t i = ((tid & ~(h - 1)) << 2) | (tid & (h - 1));
+      if (i < span && (i & (S - 1)) + h < fill) {
+        // distances (j, h): entries i, i + h and their partners, which are
+        // mirrored within the run of k in a merge's first stage
+        const uint32_t far = mirror ? mirror : j;
+        const uint32_t p0 = slot_pos(i), p1 = p0 ^ slot_pos(h);
+        const uint32_t p2 = p0 ^ slot_pos(mirror ? far ^ h : far), p3 = p0 ^ slot_pos(mirror ? far : far ^ h);
+        double x0 = K[p0], x1 = K[p1], x2 = K[p2], x3 = K[p3];
+        if (mirror) {
+          order(x0, x3);
+          order(x1, x2);
+        } else {
+          order(x0, x2);
+          order(x1, x3);
+        }
+        order(x0, x1);
+        order(x2, x3);
+        K[p0] = x0;
+        K[p1] = x1;
+        K[p2] = x2;
+        K[p3] = x3;
+      }
+      mirror = 0;
+      // after (2, 1): the next size 2k starts with distance k
+      const uint32_t jn = j > 2 ? j >> 2 : k;
+      barrier(j <= 128 && jn <= 128 && !(j == 2 && k == S));
+    }
+  }
+}
+
 // One workgroup per group: all remaining levels of the group's subtree(s),
 // in LDS.  Elements are their positions in the group's window of bb (the
 // bounds in position order: written by the last k_emit, or the input order of
 // a tree that starts here); orig (optional) maps positions to triangle ids
 // where the tree order is written.
 //
-// A group is one chain of dependent stages (286 compare stages of the sorts
-// over the 11 levels of 2048 elements, and about ten LDS round trips a level),
-// so its latency is the launch: 1M triangles give two groups per CU.  1024
-// threads take a stage in one step, and the keys of all axes are in LDS (six
-// dwords per element), so that no level waits for global memory; the triangle
-// ids of a level's pairs, read from orig, are stored one level later.  A launch
-// of two groups takes 101 us and one of 512 (1M triangles) 163; with 256
-// threads in four rounds per stage and the bounds gathered from memory at
-// every level they took 227 and 268 (8192 groups of 10M triangles gain
-// nothing: there the sorts' LDS traffic binds, 1.5 ms either way).
-// 77 KB of LDS and at most 64 VGPRs: two groups reside per CU.
-constexpr int kSubThreads = 1024;
-__global__ __launch_bounds__(kSubThreads, 8) void k_subtree(const SubGroup* __restrict__ groups,
-                                                            const float2* __restrict__ bb, uint32_t N,
-                                                            uint32_t n, int L, int level0,
-                                                            uint32_t* __restrict__ P,
+// A level sorts each sort group, the remainder of one node of the previous
+// level: a range of its own in the sorted order of that level, holding the
+// nodes 2q and 2q + 1 of this one.  Group q is sorted in its own slot of S
+// entries, S the power of two that holds the first (largest) group.  The
+// slots fit kSubT = T: the workgroup's first group has at most T triangles, so its
+// parent heads at most T/2 + 1 nodes; in a left-complete tree the leftmost
+// node r levels below then heads at most T/2^(r+1) + 1, its children hold at
+// most T/2^r triangles, and there are at most 2^r groups at that depth.
+//
+// A group is one chain of dependent steps (the passes of the sorts, 230 over
+// the 12 levels of 4096 elements, and eight barriers a level), so its latency
+// is the launch for trees of up to a million triangles: 139 us for the 2584 of
+// one group, 133 us for the 256 groups of 1M.  1024 threads take a pass in one
+// step, and the keys of all axes are in LDS (six dwords per element), so that
+// no level waits for global memory; the triangle ids of a level's pairs, read
+// from orig, are stored one level later.
+// 146 KB of LDS: one group of 16 waves per CU.  Groups of 2048, two per CU,
+// take 112 us at 1M but leave one more level to the radix passes, 19 launches
+// of 130 us together: a build of 1M triangles took 1.70 ms instead of 1.62, of
+// 10M 11.3 ms on the device instead of 11.0, and a tree of 2050 to 4096
+// triangles, which is one group here, 0.30 ms instead of 0.18.
+__global__ __launch_bounds__(kSubThreads, 4) void k_subtree(const SubGroup* __restrict__ groups,
+                                                            const float2* __restrict__ bb,
+                                                            uint32_t N, uint32_t n, int L,
+                                                            int level0, uint32_t* __restrict__ P,
                                                             const uint32_t* __restrict__ orig) {
-  __shared__ uint32_t kmin[3][kSubT], kmax[3][kSubT];
-  __shared__ unsigned long long K[kSubT];
-  __shared__ uint16_t E[kSubT], G[kSubT];
-  __shared__ uint16_t nodeOff[kSubT / 2 + 1];
-  __shared__ uint16_t nodeArg[kSubT / 2];
-  __shared__ uint32_t gmax;  // largest sort group of the level
+  constexpr uint32_t T = kSubT;
+  constexpr uint32_t kPer = T / kSubThreads;        // elements per thread
+  constexpr uint32_t kNodes = T / 2 / kSubThreads;  // nodes per thread
+  constexpr uint32_t kPosBits = 12;
+  static_assert(1u << kPosBits == T, "");
+  __shared__ uint32_t kmin[3][T], kmax[3][T];
+  __shared__ double K[T];
+  __shared__ uint16_t E[T];
+  __shared__ uint16_t nodeOff[T / 2 + 1];
+  __shared__ uint16_t nodeArg[T / 2];
   // once the sorted order is read out, the sort buffer holds the sorted
   // elements (E2) and their max keys (MK)
   uint32_t* E2 = reinterpret_cast<uint32_t*>(K);
-  uint32_t* MK = E2 + kSubT;
-  constexpr int kPer = kSubT / kSubThreads;  // elements per thread
-  static_assert(kSubT / 2 <= kSubThreads, "one node per thread");
+  uint32_t* MK = E2 + T;
 
   const SubGroup g = groups[blockIdx.x];
   const uint32_t tid = threadIdx.x;
-  uint32_t m = min(g.size, kSubT);
+  uint32_t m = min(g.size, T);
   for (uint32_t i = tid; i < m; i += kSubThreads) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -576,131 +699,91 @@ __global__ __launch_bounds__(kSubThreads, 8) void k_subtree(const SubGroup* __re
       kmax[a][i] = fkey(b.y);
     }
     E[i] = (uint16_t)i;
-    G[i] = 0;
   }
   uint32_t f = g.first, c = g.count;
-  // the pair of the previous level's node `tid`: written once its ids are here
-  bool held = false;
-  uint32_t held_h = 0, held_x = 0, held_y = 0;
-  const auto put = [&](uint32_t h, uint32_t x, uint32_t y) {
-    held = true;
-    held_h = h;
-    held_x = orig ? orig[g.off + x] : g.off + x;
-    held_y = orig ? orig[g.off + y] : g.off + y;
+  // the pairs of this thread's nodes of the previous level: written once
+  // their ids are here
+  bool held[kNodes];
+  uint32_t held_h[kNodes], held_x[kNodes], held_y[kNodes];
+#pragma unroll
+  for (uint32_t r = 0; r < kNodes; ++r) held[r] = false;
+  const auto put = [&](uint32_t r, uint32_t h, uint32_t x, uint32_t y) {
+    held[r] = true;
+    held_h[r] = h;
+    held_x[r] = orig ? orig[g.off + x] : g.off + x;
+    held_y[r] = orig ? orig[g.off + y] : g.off + y;
   };
   const auto flush = [&]() {
-    if (held) {
-      P[2 * (size_t)held_h] = held_x;
-      P[2 * (size_t)held_h + 1] = held_y;
+#pragma unroll
+    for (uint32_t r = 0; r < kNodes; ++r) {
+      if (held[r]) {
+        P[2 * (size_t)held_h[r]] = held_x[r];
+        P[2 * (size_t)held_h[r] + 1] = held_y[r];
+      }
+      held[r] = false;
     }
-    held = false;
   };
-  __syncthreads();
   for (int level = level0; level < L && m > 0; ++level) {
     const int a = level % 3;
-    if (tid <= c) nodeOff[tid] = (uint16_t)(2u * (uint32_t)desc_count(f, f + tid, n));
-    if (tid == 0) {
-      gmax = 0;
-      if (c == kSubThreads) nodeOff[c] = (uint16_t)m;
-    }
+    for (uint32_t j = tid; j <= c; j += kSubThreads) nodeOff[j] = (uint16_t)(2u * desc_count32(f, f + j, n));
     __syncthreads();
-    // Sort groups are the remainders of one node of the previous level: the
-    // ranges of this level's node pairs (2q, 2q+1), contiguous and in order,
-    // with G = q.  When every group fits a power-of-two slot of S entries and
-    // the slots fit the sort buffer, each group is sorted in its own slot
-    // (log2(S) bitonic phases instead of log2(M)); otherwise the whole region
-    // is sorted on (group, key, position).
-    const uint32_t ng = (c + 1) / 2;
-    if (tid < ng) atomicMax(&gmax, (uint32_t)nodeOff[min(2 * tid + 2, c)] - nodeOff[2 * tid]);
-    uint32_t M = 1;
-    while (M < m) M <<= 1;
-    __syncthreads();
-    const uint32_t gm = gmax;
-    uint32_t S = 2;
-    while (S < gm) S <<= 1;
-    const bool seg = (uint64_t)ng * S <= kSubT;
-    const uint32_t span = seg ? ng * S : M;  // sorted entries
-    const uint32_t top = seg ? S : M;        // size of one sorted run
-    for (uint32_t q = tid; q < span; q += kSubThreads) K[q] = ~0ull;
-    __syncthreads();
+    // sort groups q < ng = the nodes' pairs, entry p of group q in slot entry
+    // q * S + p (kSlotEnd beyond the group's size)
+    const uint32_t ng = (c + 1) / 2, size0 = nodeOff[min(2u, c)];
+    const uint32_t ls = size0 > 2 ? 32u - (uint32_t)__clz((int)(size0 - 1)) : 1u, S = 1u << ls;
+    const uint32_t span = min(ng << ls, T);
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kSubThreads;
-      if (i >= m) break;
-      const unsigned long long key = kmin[a][E[i]];
-      const uint32_t q = G[i];
-      if (seg) {
-        const uint32_t p = i - nodeOff[2 * q];
-        K[q * S + p] = (key << 11) | p;
-      } else {
-        K[i] = ((unsigned long long)q << 43) | (key << 11) | i;
-      }
+    for (uint32_t r = 0; r < kPer; ++r) {
+      const uint32_t sl = tid + r * kSubThreads;
+      if (sl >= span) break;
+      const uint32_t q = sl >> ls, p = sl & (S - 1), o = nodeOff[2 * q];
+      const uint32_t i = o + p;
+      K[slot_pos(sl)] = __longlong_as_double((long long)(
+          i < nodeOff[min(2 * q + 2, c)] ? kSlotKey | ((unsigned long long)kmin[a][E[i]] << kPosBits) | p : kSlotEnd));
     }
     flush();
     __syncthreads();
-    for (uint32_t k = 2; k <= top; k <<= 1) {
-      for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-        if (tid < span / 2) {
-          const uint32_t i = ((tid & ~(j - 1)) << 1) | (tid & (j - 1));  // j is a power of two
-          const uint32_t ixj = i + j;
-          const bool up = (i & k & (top - 1)) == 0;  // every run ascending at k == top
-          const unsigned long long x = K[i], y = K[ixj];
-          if ((x > y) == up) {
-            K[i] = y;
-            K[ixj] = x;
-          }
-        }
-        // With j <= 64, the pairs of a wave's threads lie in its own 128
-        // entries in this stage, and in the next one if that also has
-        // j <= 64, so a wave barrier orders it.
-        const uint32_t jn = j > 1 ? (j >> 1) : k;  // next stage: (k, j/2) or (2k, k)
-        if ((j == 1 && k == top) || j > 64 || jn > 64) {
-          __syncthreads();
-        } else {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-      }
-    }
+    sort_slots(K, span, S, size0);
     const bool last = level == L - 1;
-    uint32_t ev[kPer], kv[kPer], qv[kPer];
+    // sorted entry p of group q is sorted position nodeOff[2q] + p
+    uint32_t ev[kPer], kv[kPer], at[kPer];
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kSubThreads;
-      ev[r] = kv[r] = qv[r] = 0;
-      if (i < m) {
-        const uint32_t q = G[i];
-        if (seg) {
-          const uint32_t gs = nodeOff[2 * q];
-          ev[r] = E[gs + (uint32_t)(K[q * S + (i - gs)] & 0x7FFull)];
-        } else {
-          ev[r] = E[(uint32_t)(K[i] & 0x7FFull)];
+    for (uint32_t r = 0; r < kPer; ++r) {
+      const uint32_t sl = tid + r * kSubThreads;
+      ev[r] = kv[r] = 0;
+      at[r] = ~0u;
+      if (sl < span) {
+        const uint32_t q = sl >> ls, o = nodeOff[2 * q], i = o + (sl & (S - 1));
+        if (i < nodeOff[min(2 * q + 2, c)]) {
+          at[r] = i;
+          ev[r] = E[min(o + ((uint32_t)__double_as_longlong(K[slot_pos(sl)]) & ((1u << kPosBits) - 1)), m - 1)];
+          kv[r] = kmax[a][ev[r]];
         }
-        qv[r] = q;
-        kv[r] = kmax[a][ev[r]];
       }
     }
     __syncthreads();  // every sorted slot is read: E2 and MK overwrite them
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kSubThreads;
-      if (i < m) {
-        E2[i] = ev[r];
-        MK[i] = kv[r];
+    for (uint32_t r = 0; r < kPer; ++r)
+      if (at[r] != ~0u) {
+        E2[at[r]] = ev[r];
+        MK[at[r]] = kv[r];
       }
-    }
     __syncthreads();
     if (last) {
-      if (tid < c) put(f + tid, E2[nodeOff[tid]], E2[nodeOff[tid] + 1]);
+#pragma unroll
+      for (uint32_t r = 0; r < kNodes; ++r) {
+        const uint32_t j = tid + r * kSubThreads;
+        if (j < c) put(r, f + j, E2[nodeOff[j]], E2[nodeOff[j] + 1]);
+      }
       break;
     }
     // first maximum of the max key over each node's [o + 1, e): W lanes per
     // node, as many as there are threads for
-    uint32_t W = 64;
-    while (W > 1 && W * c > kSubThreads) W >>= 1;
-    for (uint32_t j0 = 0; j0 < c; j0 += kSubThreads / W) {
-      const uint32_t j = j0 + tid / W, w = tid & (W - 1);
+    uint32_t lw = 6;
+    while (lw > 0 && (c << lw) > kSubThreads) --lw;
+    const uint32_t W = 1u << lw;
+    for (uint32_t j0 = 0; j0 < c; j0 += kSubThreads >> lw) {
+      const uint32_t j = j0 + (tid >> lw), w = tid & (W - 1);
       uint32_t bk = 0, bp = 0xFFFFFFFFu, o = 0, e = 0;
       if (j < c) {
         o = nodeOff[j];
@@ -723,25 +806,24 @@ __global__ __launch_bounds__(kSubThreads, 8) void k_subtree(const SubGroup* __re
       if (j < c && w == 0) nodeArg[j] = (uint16_t)((bp > o && bp < e) ? bp : o + 1);  // sizes are >= 2
     }
     __syncthreads();
-    if (tid < c) {
-      const uint32_t x = E2[nodeOff[tid]], y = E2[nodeArg[tid]];
-      const bool swap = second_first(x, y, level, L, [&](int ax, uint32_t i) { return kmin[ax][i]; });
-      put(f + tid, swap ? y : x, swap ? x : y);
-    }
-    // compaction: the node of sorted position i is one of its sort group's
-    // two nodes (groups are contiguous and keep their ranges through the
-    // sort); G and E were read above
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint32_t i = tid + r * kSubThreads;
-      if (i >= m) break;
-      uint32_t j = 2u * qv[r];
-      if (j + 1 < c && i >= nodeOff[j + 1]) ++j;
-      if (i >= nodeOff[j] + 2u) {
-        const uint32_t dst = i - 2 * (j + 1);
-        E[dst] = (uint16_t)((i == nodeArg[j]) ? E2[nodeOff[j] + 1] : ev[r]);
-        G[dst] = (uint16_t)j;
+    for (uint32_t r = 0; r < kNodes; ++r) {
+      const uint32_t j = tid + r * kSubThreads;
+      if (j < c) {
+        const uint32_t x = E2[nodeOff[j]], y = E2[nodeArg[j]];
+        const bool swap = second_first(x, y, level, L, [&](int ax, uint32_t i) { return kmin[ax][i]; });
+        put(r, f + j, swap ? y : x, swap ? x : y);
       }
+    }
+    // compaction: the node of a sorted position is one of its group's two
+#pragma unroll
+    for (uint32_t r = 0; r < kPer; ++r) {
+      const uint32_t i = at[r];
+      if (i == ~0u) continue;
+      uint32_t j = 2u * ((tid + r * kSubThreads) >> ls);
+      if (j + 1 < c && i >= nodeOff[j + 1]) ++j;
+      if (i >= nodeOff[j] + 2u)
+        E[i - 2 * (j + 1)] = (uint16_t)((i == nodeArg[j]) ? E2[nodeOff[j] + 1] : ev[r]);
     }
     __syncthreads();
     m -= 2 * c;
@@ -1149,12 +1231,10 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
     Valt = free_buf;
   }
   AUR_LAUNCH_CHECK(ctx, "nmh level kernels");
-  if (level0 > 0) {
-    // the subtree phase on positions (renumbered by the last k_emit)
-    k_subtree<<<bp.nsub, kSubThreads, 0, s>>>(dsub, bbR, m0, n, L, level0, ctx->perm.p, Ka);
-  } else {
-    k_subtree<<<bp.nsub, kSubThreads, 0, s>>>(dsub, bb, N, n, L, level0, ctx->perm.p, nullptr);
-  }
+  // the subtree phase, on positions renumbered by the last k_emit if levels
+  // came before it
+  k_subtree<<<bp.nsub, kSubThreads, 0, s>>>(dsub, large ? bbR : bb, m0, n, L, level0, ctx->perm.p,
+                                            large ? Ka : nullptr);
   AUR_LAUNCH_CHECK(ctx, "k_subtree");
 
   AUR_HIP(ctx, ctx->vertices.reserve((size_t)N * 9));
