@@ -17,15 +17,15 @@
 //     lexicographic comparison of the later levels' keys (newest first; only
 //     the last three levels can differ since axes cycle with period 3);
 //   * while node groups are larger than one workgroup's LDS tile, a level is a
-//     segmented stable LSD radix sort (8-bit digits, tile histograms,
-//     per-group digit offsets, wave-ballot stable ranking) followed by a
+//     segmented stable LSD radix sort (8-bit digits; a pass is a launch for
+//     the tile histograms and one that sums every tile's offsets, ranks with
+//     wave ballots and scatters) followed by a
 //     tiled first-maximum reduction and an emit pass that writes finished
 //     pairs and compacts the remainders for the next level.  The digits are
 //     those of key - (the group's smallest key), so a group whose keys span
 //     fewer than 2^24 values needs 3 passes (2^16: 2, ...): the emit pass
-//     records each tile's key range, the next level's first group scan
-//     reduces them per group and hands (smallest key, passes) to every tile
-//     and chunk of the group;
+//     records each tile's key range, and the next level's first scatter
+//     reduces them to its group's (smallest key, passes);
 //   * once every group fits (<= kSubT elements) one workgroup takes a whole
 //     subtree and runs all remaining levels in LDS with a bitonic sort on
 //     (group, key, position) composite keys.
@@ -42,6 +42,11 @@ namespace {
 
 constexpr uint32_t kTile = 2048;  // radix / emit tile (elements)
 constexpr uint32_t kChunk = 32;   // tiles per chunk of the radix offset scan
+// Levels with a group of more chunks than this (4.2M triangles) sum the chunks
+// in a launch of their own: otherwise every tile of the group reads all of them.
+// Device time per build with and without it: 10.76 and 10.91 ms at 10M, 24.0
+// and 25.1 ms at 20M.  Limits of 24 and 120 differ by less than 1% at 1M to 20M.
+constexpr uint32_t kScanChunks = 64;
 constexpr uint32_t kSubT = 4096;  // max elements of an LDS-resident subtree
 constexpr int kThreads = 256;
 constexpr int kSubThreads = 1024;  // k_subtree
@@ -116,8 +121,8 @@ __device__ __forceinline__ uint32_t clampi(uint32_t i, uint32_t N) { return i < 
 // histograms).  Pass p of a level moves the groups with group_passes > p,
 // from buffer p & 1 to the other, so a group's sorted data ends in buffer
 // group_passes & 1.  Kernels read a tile's (smallest key, passes) as
-// TP[tile] and a chunk's passes as CP[chunk] (by block index, so the load
-// does not wait for the tile's descriptor).
+// TP[tile] (by block index, so the load does not wait for the tile's
+// descriptor).
 __device__ __forceinline__ uint32_t group_passes(uint2 r) {
   const uint32_t d = r.y - r.x;
   return d < 0x10000u ? (d < 0x100u ? 1u : 2u) : (d < 0x1000000u ? 3u : 4u);
@@ -126,136 +131,6 @@ __device__ __forceinline__ uint32_t group_passes(uint2 r) {
 __global__ void k_fill0(uint32_t* __restrict__ p, uint32_t N) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < N) p[i] = 0;
-}
-
-// Per-tile digit histogram H[tile][digit], also added into its chunk's digit
-// counts CS[chunk][digit] (integer atomics: the sums are exact whatever the
-// order).  CS starts at zero: zeroed once per build and again by
-// k_radix_group_scan after it reads a pass's counts.  Pass 0 counts the
-// key's low byte (indexed so; k_radix_group_scan orders the digits).
-__global__ __launch_bounds__(kThreads) void k_radix_hist(const TileDesc* __restrict__ tiles,
-                                                         const GroupDesc* __restrict__ groups,
-                                                         const uint2* __restrict__ TP,
-                                                         const uint32_t* __restrict__ K,
-                                                         uint32_t pass,
-                                                         uint32_t* __restrict__ H,
-                                                         uint32_t* __restrict__ CS) {
-  __shared__ uint32_t h[256];
-  const TileDesc t = tiles[blockIdx.x];
-  uint32_t kmin = 0;
-  if (pass > 0) {
-    const uint2 tp = TP[blockIdx.x];
-    if (tp.y <= pass) return;  // uniform per block
-    kmin = tp.x;
-  }
-  const uint32_t shift = 8u * pass;
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < t.count; i += kThreads)
-    atomicAdd(&h[((K[t.start + i] - kmin) >> shift) & 255u], 1u);
-  __syncthreads();
-  const uint32_t v = h[threadIdx.x];
-  H[(size_t)blockIdx.x * 256 + threadIdx.x] = v;
-  const GroupDesc g = groups[t.group];
-  const uint32_t chunk = g.cb + (blockIdx.x - g.tb) / kChunk;
-  if (v) atomicAdd(&CS[(size_t)chunk * 256 + threadIdx.x], v);
-}
-
-// Per group: exclusive digit offsets of the group (digit-major), and the base
-// B[chunk][digit] of every chunk of the group (the counts of the group's
-// earlier chunks added); then the chunk counts are zeroed for the next pass.
-// (A group that skips the pass has no counts: they stay zero.)
-// Pass 0 first sets the group's key range: from the previous level's emit
-// tiles of the group's parent node (prev_children[group], tile ranges TR),
-// or the full range on the first level (prev_children null); GP[group],
-// TP[tile] and CP[chunk] of the group take (smallest key, passes).  Its
-// digits are the keys' low bytes, scanned in the order of
-// (low byte - smallest key) & 255.
-__global__ __launch_bounds__(kThreads) void k_radix_group_scan(const GroupDesc* __restrict__ groups,
-                                                               uint2* __restrict__ GP,
-                                                               uint2* __restrict__ TP,
-                                                               uint32_t* __restrict__ CP,
-                                                               const ChildDesc* __restrict__ prev_children,
-                                                               const uint2* __restrict__ TR,
-                                                               uint32_t pass,
-                                                               uint32_t* __restrict__ S,
-                                                               uint32_t* __restrict__ B) {
-  __shared__ uint32_t s[256];
-  __shared__ uint32_t rmin[kThreads / 64], rmax[kThreads / 64];
-  const uint32_t d = threadIdx.x;
-  uint32_t rot = 0;  // scan position of digit d: (d - rot) & 255
-  const GroupDesc g = groups[blockIdx.x];
-  const bool reduce = pass == 0 && prev_children != nullptr;
-  const ChildDesc pc = reduce ? prev_children[blockIdx.x] : ChildDesc{0u, 0u, 0u, 0u};
-  if (pass > 0 && GP[blockIdx.x].y <= pass) return;  // uniform per block
-  // the group's digit counts first: their loads then overlap the range's
-  uint32_t total = 0;
-#pragma unroll 8
-  for (uint32_t c = g.cb; c < g.ce; ++c) total += S[(size_t)c * 256 + d];
-  if (pass == 0) {
-    uint2 r = make_uint2(0u, 0xFFFFFFFFu);
-    if (reduce) {
-      uint32_t mn = 0xFFFFFFFFu, mx = 0u;
-      for (uint32_t t = pc.tb + d; t < pc.te; t += kThreads) {
-        const uint2 tr = TR[t];
-        mn = min(mn, tr.x);
-        mx = max(mx, tr.y);
-      }
-      for (int off = 32; off > 0; off >>= 1) {
-        mn = min(mn, (uint32_t)__shfl_xor(mn, off));
-        mx = max(mx, (uint32_t)__shfl_xor(mx, off));
-      }
-      if ((d & 63u) == 0) {
-        rmin[d >> 6] = mn;
-        rmax[d >> 6] = mx;
-      }
-      __syncthreads();
-      r = make_uint2(rmin[0], rmax[0]);
-#pragma unroll
-      for (int w = 1; w < kThreads / 64; ++w) r = make_uint2(min(r.x, rmin[w]), max(r.y, rmax[w]));
-    }
-    const uint2 gp = make_uint2(r.x, group_passes(r));
-    if (d == 0) GP[blockIdx.x] = gp;
-    for (uint32_t t = g.tb + d; t < g.te; t += kThreads) TP[t] = gp;
-    for (uint32_t c = g.cb + d; c < g.ce; c += kThreads) CP[c] = gp.y;
-    rot = r.x & 255u;
-  }
-  const uint32_t sp = (d - rot) & 255u;
-  s[sp] = total;
-  __syncthreads();
-  for (uint32_t off = 1; off < 256; off <<= 1) {
-    const uint32_t v = d >= off ? s[d - off] : 0u;
-    __syncthreads();
-    s[d] += v;
-    __syncthreads();
-  }
-  uint32_t run = g.off + s[sp] - total;
-#pragma unroll 8
-  for (uint32_t c = g.cb; c < g.ce; ++c) {
-    B[(size_t)c * 256 + d] = run;
-    run += S[(size_t)c * 256 + d];
-    S[(size_t)c * 256 + d] = 0u;
-  }
-}
-
-// Output offsets of every tile, O[tile][digit]: the chunk's base plus the
-// counts of the chunk's earlier tiles (one block per chunk; the chunk's
-// tiles are found from the tile's group).
-__global__ __launch_bounds__(kThreads) void k_radix_chunk_offsets(const uint32_t* __restrict__ chunk_tile,
-                                                                  const uint32_t* __restrict__ CP,
-                                                                  uint32_t pass,
-                                                                  const uint32_t* __restrict__ H,
-                                                                  const uint32_t* __restrict__ B,
-                                                                  uint32_t* __restrict__ O) {
-  const uint32_t tb = chunk_tile[blockIdx.x], te = chunk_tile[blockIdx.x + 1];
-  if (pass > 0 && CP[blockIdx.x] <= pass) return;  // uniform per block
-  const uint32_t d = threadIdx.x;
-  uint32_t run = B[(size_t)blockIdx.x * 256 + d];
-#pragma unroll 8
-  for (uint32_t t = tb; t < te; ++t) {
-    O[(size_t)t * 256 + d] = run;
-    run += H[(size_t)t * 256 + d];
-  }
 }
 
 // Inclusive scan of one value per thread over the 256 threads (4 waves):
@@ -273,6 +148,135 @@ __device__ __forceinline__ uint32_t block_incl_scan256(uint32_t v, uint32_t* __r
   return v;
 }
 
+// Key range of a group, by a block: from the previous level's emit tiles of the
+// group's parent node (prev_children[group], tile ranges TR), or the full range
+// on the first level (prev_children null).
+__device__ __forceinline__ uint2 group_range(const ChildDesc* __restrict__ prev_children, uint32_t group,
+                                             const uint2* __restrict__ TR) {
+  __shared__ uint32_t rmin[kThreads / 64], rmax[kThreads / 64];
+  if (!prev_children) return make_uint2(0u, 0xFFFFFFFFu);  // uniform: a kernel argument
+  const ChildDesc pc = prev_children[group];
+  uint32_t mn = 0xFFFFFFFFu, mx = 0u;
+  for (uint32_t t = pc.tb + threadIdx.x; t < pc.te; t += kThreads) {
+    const uint2 tr = TR[t];
+    mn = min(mn, tr.x);
+    mx = max(mx, tr.y);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    mn = min(mn, (uint32_t)__shfl_xor(mn, off));
+    mx = max(mx, (uint32_t)__shfl_xor(mx, off));
+  }
+  if ((threadIdx.x & 63u) == 0) {
+    rmin[threadIdx.x >> 6] = mn;
+    rmax[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  uint2 r = make_uint2(rmin[0], rmax[0]);
+#pragma unroll
+  for (int w = 1; w < kThreads / 64; ++w) r = make_uint2(min(r.x, rmin[w]), max(r.y, rmax[w]));
+  return r;
+}
+
+// f(row, R[row][threadIdx.x]) for the rows [b, e) of 256 counts, eight loads in
+// flight (the last eight repeat a row rather than go one at a time).
+template <class F>
+__device__ __forceinline__ void each_row(const uint32_t* __restrict__ R, uint32_t b, uint32_t e, F&& f) {
+  for (uint32_t r = b; r < e; r += 8) {
+    uint32_t v[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) v[u] = R[(size_t)min(r + u, e - 1) * 256 + threadIdx.x];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u)
+      if (r + u < e) f(r + u, v[u]);
+  }
+}
+
+// Exclusive sum over the digits before digit threadIdx.x of `total`, in the
+// order of (digit - rot) & 255.  s: 256 words of LDS.
+__device__ __forceinline__ uint32_t digit_offset(uint32_t total, uint32_t rot, uint32_t* s, uint32_t* wsum) {
+  const uint32_t sp = (threadIdx.x - rot) & 255u;
+  s[sp] = total;
+  __syncthreads();
+  const uint32_t own = s[threadIdx.x];
+  s[threadIdx.x] = block_incl_scan256(own, wsum) - own;
+  __syncthreads();
+  return s[sp];
+}
+
+// Per-tile digit histogram H[tile][digit], also added into its chunk's digit
+// counts CS[chunk][digit] (integer atomics: the sums are exact whatever the
+// order).  CS starts at zero: all of it before the first level, and the rows of
+// the next pass's counts (CSnext) are zeroed here, by the first tile of each
+// chunk.  Pass 0 counts the key's low byte (indexed so; k_radix_scatter and
+// k_radix_group_scan order the digits).
+__global__ __launch_bounds__(kThreads) void k_radix_hist(const TileDesc* __restrict__ tiles,
+                                                         const GroupDesc* __restrict__ groups,
+                                                         const uint2* __restrict__ TP,
+                                                         const uint32_t* __restrict__ K,
+                                                         uint32_t pass,
+                                                         uint32_t* __restrict__ H,
+                                                         uint32_t* __restrict__ CS,
+                                                         uint32_t* __restrict__ CSnext) {
+  __shared__ uint32_t h[256];
+  const TileDesc t = tiles[blockIdx.x];
+  const GroupDesc g = groups[t.group];
+  const uint32_t in_group = blockIdx.x - g.tb, chunk = g.cb + in_group / kChunk;
+  if (in_group % kChunk == 0) CSnext[(size_t)chunk * 256 + threadIdx.x] = 0u;
+  uint32_t kmin = 0;
+  if (pass > 0) {
+    const uint2 tp = TP[blockIdx.x];
+    if (tp.y <= pass) return;  // uniform per block
+    kmin = tp.x;
+  }
+  const uint32_t shift = 8u * pass;
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < t.count; i += kThreads)
+    atomicAdd(&h[((K[t.start + i] - kmin) >> shift) & 255u], 1u);
+  __syncthreads();
+  const uint32_t v = h[threadIdx.x];
+  H[(size_t)blockIdx.x * 256 + threadIdx.x] = v;
+  if (v) atomicAdd(&CS[(size_t)chunk * 256 + threadIdx.x], v);
+}
+
+// For levels with groups of many chunks (kScanChunks).  Per group: exclusive
+// digit offsets of the group (digit-major), and the base B[chunk][digit] of
+// every chunk of the group (the counts of the group's earlier chunks added).
+// Pass 0 first sets the group's key range: GP[group] and TP[tile] of the group
+// take (smallest key, passes).  Its digits are the keys' low bytes, scanned in
+// the order of (low byte - smallest key) & 255.
+__global__ __launch_bounds__(kThreads) void k_radix_group_scan(const GroupDesc* __restrict__ groups,
+                                                               uint2* __restrict__ GP,
+                                                               uint2* __restrict__ TP,
+                                                               const ChildDesc* __restrict__ prev_children,
+                                                               const uint2* __restrict__ TR,
+                                                               uint32_t pass,
+                                                               const uint32_t* __restrict__ S,
+                                                               uint32_t* __restrict__ B) {
+  __shared__ uint32_t s[256], wsum[kThreads / 64];
+  const uint32_t d = threadIdx.x;
+  uint32_t rot = 0;  // scan position of digit d: (d - rot) & 255
+  const GroupDesc g = groups[blockIdx.x];
+  if (pass > 0 && GP[blockIdx.x].y <= pass) return;  // uniform per block
+  // the group's digit counts first: their loads then overlap the range's
+  uint32_t total = 0;
+#pragma unroll 8
+  for (uint32_t c = g.cb; c < g.ce; ++c) total += S[(size_t)c * 256 + d];
+  if (pass == 0) {
+    const uint2 r = group_range(prev_children, blockIdx.x, TR);
+    const uint2 gp = make_uint2(r.x, group_passes(r));
+    if (d == 0) GP[blockIdx.x] = gp;
+    for (uint32_t t = g.tb + d; t < g.te; t += kThreads) TP[t] = gp;
+    rot = r.x & 255u;
+  }
+  uint32_t run = g.off + digit_offset(total, rot, s, wsum);
+#pragma unroll 8
+  for (uint32_t c = g.cb; c < g.ce; ++c) {
+    B[(size_t)c * 256 + d] = run;
+    run += S[(size_t)c * 256 + d];
+  }
+}
+
 // Stable scatter of one 2048-element tile, staged through LDS.  Ranking:
 // wave w owns the tile's elements [512w, 512w + 512) in rounds of 64; lanes
 // with the same digit are found with 8 ballots, and the wave keeps its
@@ -281,15 +285,25 @@ __device__ __forceinline__ uint32_t block_incl_scan256(uint32_t v, uint32_t* __r
 // round).  Each element (key and 8-byte payload) then lands in LDS at its
 // digit-sorted tile position, and the tile is written out in that order: a
 // digit's run is one contiguous store at the tile's output offset for the
-// digit, O[tile][digit].  (Ranking in rounds of 256 elements across the
+// digit.  (Ranking in rounds of 256 elements across the
 // workgroup, with four barriers per round, took 20-35% longer; staging only
 // a 16-bit tile index and re-reading the payload at write-out measured 6%
 // slower despite the smaller LDS footprint.)
+// The tile's output offsets: the group's digit offsets and the counts of the
+// group's earlier chunks (from the chunks' counts CS, or with B as
+// k_radix_group_scan left them), and the counts of the chunk's earlier tiles.
+// Without B, pass 0 also sets the tile's (smallest key, passes), TP[tile].
+// They are summed here, once per tile and after the ranking (the payload's
+// loads are then still in flight behind it), because two launches for them, per
+// group and per chunk, cost 9 us of a pass of 29 at 1M triangles and not less
+// at 10M (1.35 -> 1.17 ms and 11.0 -> 10.9 ms of device time per build; before
+// the ranking: 11.1).
 __global__ __launch_bounds__(kThreads) void k_radix_scatter(
-    const TileDesc* __restrict__ tiles, const uint2* __restrict__ TP,
+    const TileDesc* __restrict__ tiles, const GroupDesc* __restrict__ groups, uint2* __restrict__ TP,
+    const ChildDesc* __restrict__ prev_children, const uint2* __restrict__ TR,
     const uint32_t* __restrict__ Kin, const uint2* __restrict__ Vin, uint32_t pass,
-    const uint32_t* __restrict__ O, uint32_t m, uint32_t* __restrict__ Kout,
-    uint2* __restrict__ Vout) {
+    const uint32_t* __restrict__ H, const uint32_t* __restrict__ CS, const uint32_t* __restrict__ B,
+    uint32_t m, uint32_t* __restrict__ Kout, uint2* __restrict__ Vout) {
   constexpr uint32_t kWaves = kThreads / 64;
   constexpr uint32_t kRounds = kTile / kThreads;  // rounds of 64 per wave
   __shared__ uint32_t sk[kTile];
@@ -299,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
   __shared__ uint32_t wsum[kWaves];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const TileDesc t = tiles[blockIdx.x];
-  uint32_t kmin = 0;  // pass 0: the low byte itself (the offsets O follow the group's digit order)
+  uint32_t kmin = 0;  // pass 0: the low byte itself (the offsets follow the group's digit order)
   if (pass > 0) {
     const uint2 tp = TP[blockIdx.x];
     if (tp.y <= pass) return;  // uniform per block
@@ -335,6 +349,27 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     if (valid && rank == 0) wc[wave][dg] = off + (uint32_t)__popcll(mask);
     loc[r] = off + rank;
   }
+  // thread tid = digit d: the tile's output offset
+  const GroupDesc g = groups[t.group];
+  const uint32_t in_group = blockIdx.x - g.tb, chunk = g.cb + in_group / kChunk;
+  uint32_t base = 0;
+  if (B) {
+    base = B[(size_t)chunk * 256 + tid];
+  } else {
+    uint32_t total = 0;
+    each_row(CS, g.cb, g.ce, [&](uint32_t c, uint32_t v) {
+      total += v;
+      base += c < chunk ? v : 0u;
+    });
+    uint32_t rot = 0;
+    if (pass == 0) {
+      const uint2 r = group_range(prev_children, t.group, TR);
+      if (tid == 0) TP[blockIdx.x] = make_uint2(r.x, group_passes(r));
+      rot = r.x & 255u;
+    }
+    base += g.off + digit_offset(total, rot, delta, wsum);
+  }
+  each_row(H, blockIdx.x - in_group % kChunk, blockIdx.x, [&](uint32_t, uint32_t v) { base += v; });
   __syncthreads();
   // thread tid = digit d: the tile's count, its first tile position, and
   // the first tile position of each wave's elements with digit d
@@ -353,7 +388,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
       run += c[w];
     }
   }
-  delta[tid] = O[(size_t)blockIdx.x * 256 + tid] - first;
+  delta[tid] = base - first;
   __syncthreads();
 #pragma unroll
   for (uint32_t r = 0; r < kRounds; ++r) {
@@ -422,31 +457,22 @@ __global__ __launch_bounds__(kThreads) void k_argmax_partial(const TileDesc* __r
   }
 }
 
-// One wave per child: (max key, lowest position) over the child's tiles.
-__global__ __launch_bounds__(kThreads) void k_argmax_combine(const ChildDesc* __restrict__ children,
-                                                             uint32_t nchildren,
-                                                             const uint2* __restrict__ partial,
-                                                             uint32_t* __restrict__ argpos) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t c = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  if (c >= nchildren) return;  // uniform per wave
-  const ChildDesc d = children[c];
-  uint32_t bk = 0, bp = 0xFFFFFFFFu;
-  for (uint32_t t = d.tb + lane; t < d.te; t += 64) {
-    const uint2 p = partial[t];
-    if (p.x > bk || (p.x == bk && p.y < bp)) {
-      bk = p.x;
-      bp = p.y;
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t ok = __shfl_xor(bk, off), op = __shfl_xor(bp, off);
-    if (ok > bk || (ok == bk && op < bp)) {
-      bk = ok;
-      bp = op;
-    }
-  }
-  if (lane == 0) argpos[c] = bp;
+// (max key, lowest position) over a child's tiles, by a block: every block of
+// k_emit takes its own, as a launch for it cost 4 us a level (8 at 10M).
+__device__ __forceinline__ uint32_t child_argmax(const ChildDesc& d, const uint2* __restrict__ partial) {
+  __shared__ uint2 best[kThreads / 64];
+  uint2 b = make_uint2(0u, 0xFFFFFFFFu);
+  const auto take = [&](uint2 p) {
+    if (p.x > b.x || (p.x == b.x && p.y < b.y)) b = p;
+  };
+  for (uint32_t t = d.tb + threadIdx.x; t < d.te; t += kThreads) take(partial[t]);
+  for (int off = 32; off > 0; off >>= 1)
+    take(make_uint2((uint32_t)__shfl_xor(b.x, off), (uint32_t)__shfl_xor(b.y, off)));
+  if ((threadIdx.x & 63u) == 0) best[threadIdx.x >> 6] = b;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kThreads / 64; ++w) take(best[w]);
+  return b.y;
 }
 
 // Writes finished pairs (tree positions 2h, 2h+1) and compacts remainders
@@ -462,7 +488,7 @@ __global__ __launch_bounds__(kThreads) void k_argmax_combine(const ChildDesc* __
 // contiguous window of bounds.
 __global__ __launch_bounds__(kThreads) void k_emit(const TileDesc* __restrict__ tiles,
                                                    const ChildDesc* __restrict__ children,
-                                                   const uint32_t* __restrict__ argpos,
+                                                   const uint2* __restrict__ partial,
                                                    const uint2* __restrict__ TP,
                                                    const uint2* __restrict__ V0,
                                                    const uint2* __restrict__ V1,
@@ -477,7 +503,7 @@ __global__ __launch_bounds__(kThreads) void k_emit(const TileDesc* __restrict__ 
   const ChildDesc c = children[t.child];
   const uint2* __restrict__ V = (TP[blockIdx.x].y & 1u) ? V1 : V0;
   const float2* bnext = bb + (size_t)((level + 1) % 3) * N;
-  uint32_t am = argpos[t.child];
+  uint32_t am = child_argmax(c, partial);
   if (am <= c.off || am >= c.off + c.size) am = c.off + 1;  // cannot happen for sizes >= 2
   uint32_t kmin = 0xFFFFFFFFu, kmax = 0u;
   for (uint32_t r = threadIdx.x; r < t.count; r += kThreads) {
@@ -664,9 +690,9 @@ __device__ __forceinline__ void sort_slots(double* K, uint32_t span, uint32_t S,
 // no level waits for global memory; the triangle ids of a level's pairs, read
 // from orig, are stored one level later.
 // 146 KB of LDS: one group of 16 waves per CU.  Groups of 2048, two per CU,
-// take 112 us at 1M but leave one more level to the radix passes, 19 launches
-// of 130 us together: a build of 1M triangles took 1.70 ms instead of 1.62, of
-// 10M 11.3 ms on the device instead of 11.0, and a tree of 2050 to 4096
+// take 112 us at 1M but leave one more level to the radix passes (then of 130
+// us): a build of 1M triangles took 1.70 ms instead of 1.62, of 10M 11.3 ms on
+// the device instead of 11.0, and a tree of 2050 to 4096
 // triangles, which is one group here, 0.30 ms instead of 0.18.
 __global__ __launch_bounds__(kSubThreads, 4) void k_subtree(const SubGroup* __restrict__ groups,
                                                             const float2* __restrict__ bb,
@@ -976,18 +1002,19 @@ constexpr size_t kKeepScratch = 256ull << 20;
 
 struct LevelPlan {
   int level;
-  uint32_t m, first, nchildren, ngroups, ntiles, nchunks;
-  size_t child_base, group_base, tile_base, chunk_base;
+  uint32_t m, first, ngroups, ntiles;
+  size_t child_base, group_base, tile_base;
+  bool scan;  // k_radix_group_scan runs
 };
 
 struct BuildPlan {
   uint32_t count = 0;  // triangles (0: none)
   int L = 0, level0 = 0;
   uint32_t nsub = 0;
-  size_t max_tiles = 1, max_children = 1, max_chunks = 1;
+  size_t max_tiles = 1, max_groups = 1, max_chunks = 1;
   std::vector<LevelPlan> levels;
   std::vector<uint8_t> image;  // every descriptor array; empty once on the device
-  size_t at_tiles = 0, at_children = 0, at_groups = 0, at_chunk_tiles = 0, at_sub = 0;
+  size_t at_tiles = 0, at_children = 0, at_groups = 0, at_sub = 0;
 };
 
 // Queues the tangent frames of the tree-order normals.
@@ -1032,10 +1059,9 @@ void make_plan(uint32_t N, BuildPlan& bp) {
   std::vector<ChildDesc> children;
   std::vector<GroupDesc> groups;
   uint32_t chunk_count = 0;  // chunks of kChunk tiles of one group, per level
-  std::vector<uint32_t> chunk_tiles;  // per level: first tile of each chunk, then the level's tile count
   std::vector<LevelPlan>& plan = bp.levels;
   plan.clear();
-  size_t max_tiles = 1, max_children = 1, max_chunks = 1;
+  size_t max_tiles = 1, max_groups = 1, max_chunks = 1;
   for (int l = 0; l < level0; ++l) {
     LevelPlan lp{};
     lp.level = l;
@@ -1067,23 +1093,19 @@ void make_plan(uint32_t N, BuildPlan& bp) {
       off += size;
     }
     groups.back().te = (uint32_t)(tiles.size() - lp.tile_base);
-    lp.nchildren = (uint32_t)(children.size() - lp.child_base);
     lp.ngroups = (uint32_t)(groups.size() - lp.group_base);
     lp.ntiles = (uint32_t)(tiles.size() - lp.tile_base);
     chunk_count = 0;
-    lp.chunk_base = chunk_tiles.size();
     for (size_t gi = lp.group_base; gi < groups.size(); ++gi) {
       GroupDesc& g = groups[gi];
       g.cb = chunk_count;
-      for (uint32_t t = g.tb; t < g.te; t += kChunk) chunk_tiles.push_back(t);
       chunk_count += (g.te - g.tb + kChunk - 1) / kChunk;
       g.ce = chunk_count;
+      lp.scan = lp.scan || g.ce - g.cb > kScanChunks;
     }
-    chunk_tiles.push_back(lp.ntiles);
-    lp.nchunks = chunk_count;
-    max_chunks = std::max<size_t>(max_chunks, lp.nchunks);
+    max_chunks = std::max<size_t>(max_chunks, chunk_count);
     max_tiles = std::max<size_t>(max_tiles, lp.ntiles);
-    max_children = std::max<size_t>(max_children, lp.nchildren);
+    max_groups = std::max<size_t>(max_groups, lp.ngroups);
     plan.push_back(lp);
   }
   std::vector<SubGroup> sub;
@@ -1107,7 +1129,7 @@ void make_plan(uint32_t N, BuildPlan& bp) {
   bp.level0 = level0;
   bp.nsub = (uint32_t)sub.size();
   bp.max_tiles = max_tiles;
-  bp.max_children = max_children;
+  bp.max_groups = max_groups;
   bp.max_chunks = max_chunks;
   // one image of every descriptor array, 256-byte aligned
   bp.image.clear();
@@ -1120,7 +1142,6 @@ void make_plan(uint32_t N, BuildPlan& bp) {
   bp.at_tiles = put(tiles.data(), tiles.size() * sizeof(TileDesc));
   bp.at_children = put(children.data(), children.size() * sizeof(ChildDesc));
   bp.at_groups = put(groups.data(), groups.size() * sizeof(GroupDesc));
-  bp.at_chunk_tiles = put(chunk_tiles.data(), chunk_tiles.size() * sizeof(uint32_t));
   bp.at_sub = put(sub.data(), sub.size() * sizeof(SubGroup));
 }
 
@@ -1147,7 +1168,6 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   const TileDesc* dtiles = reinterpret_cast<const TileDesc*>(desc(bp.at_tiles));
   const ChildDesc* dchildren = reinterpret_cast<const ChildDesc*>(desc(bp.at_children));
   const GroupDesc* dgroups = reinterpret_cast<const GroupDesc*>(desc(bp.at_groups));
-  const uint32_t* dchunk_tiles = reinterpret_cast<const uint32_t*>(desc(bp.at_chunk_tiles));
   const SubGroup* dsub = reinterpret_cast<const SubGroup*>(desc(bp.at_sub));
 
   // ---- device scratch, one allocation ----
@@ -1167,12 +1187,12 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   // input, the other side of the radix passes, and the emit pass's output
   const size_t vb = large ? (size_t)N * sizeof(uint2) : 0, kb = large ? (size_t)N * sizeof(uint32_t) : 0;
   const size_t at_V[3] = {take(vb), take(vb), take(vb)}, at_K[2] = {take(kb), take(kb)};
-  const size_t tb = large ? bp.max_tiles : 0, cb = large ? bp.max_chunks : 0, nb = large ? bp.max_children : 0;
+  const size_t tb = large ? bp.max_tiles : 0, cb = large ? bp.max_chunks : 0, nb = large ? bp.max_groups : 0;
   // (smallest key, passes) per group and tile, emit tiles' key ranges, passes
   // per offset chunk, first maxima
   const size_t at_GP = take(nb * sizeof(uint2)), at_TP = take(tb * sizeof(uint2)), at_TR = take(tb * sizeof(uint2));
-  const size_t at_CP = take(cb * 4), at_partial = take(tb * sizeof(uint2)), at_argpos = take(nb * 4);
-  const size_t at_H = take(tb * 256 * 4), at_O = take(tb * 256 * 4), at_CS = take(cb * 256 * 4), at_CB = take(cb * 256 * 4);
+  const size_t at_partial = take(tb * sizeof(uint2)), at_H = take(tb * 256 * 4);
+  const size_t at_CS = take(2 * cb * 256 * 4), at_CB = take(cb * 256 * 4);  // CS: this pass's and the next's
   AUR_HIP(ctx, ctx->build_scratch.reserve(ws));
   AUR_HIP(ctx, ctx->perm.reserve(N));
   const auto u2 = [&](size_t at) { return reinterpret_cast<uint2*>(ctx->build_scratch.p + at); };
@@ -1180,8 +1200,8 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   float2* const bb = reinterpret_cast<float2*>(ctx->build_scratch.p + at_bb);
   float2* const bbR = reinterpret_cast<float2*>(ctx->build_scratch.p + at_bbR);
   uint2 *const GP = u2(at_GP), *const TP = u2(at_TP), *const TR = u2(at_TR), *const partial = u2(at_partial);
-  uint32_t *const Ka = u1(at_K[0]), *const Kb = u1(at_K[1]), *const CP = u1(at_CP), *const argpos = u1(at_argpos);
-  uint32_t *const H = u1(at_H), *const O = u1(at_O), *const CS = u1(at_CS), *const CB = u1(at_CB);
+  uint32_t *const Ka = u1(at_K[0]), *const Kb = u1(at_K[1]), *const H = u1(at_H), *const CB = u1(at_CB);
+  uint32_t* const CS[2] = {u1(at_CS), u1(at_CS) + cb * 256};
 
   hipEvent_t& e0 = ctx->build_event[0];
   hipEvent_t& e1 = ctx->build_event[1];
@@ -1195,7 +1215,7 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   uint2* Valt = u2(at_V[1]);  // the other side of the radix passes
   uint2* Vout = u2(at_V[2]);  // the emit pass's output
   k_bounds<<<blocks(N, 256), 256, 0, s>>>(ctx->in_vertices.p, N, bb, large ? Vcur : nullptr, Ka);
-  if (large) k_fill0<<<blocks(bp.max_chunks * 256, 256), 256, 0, s>>>(CS, (uint32_t)(bp.max_chunks * 256));
+  if (large) k_fill0<<<blocks(bp.max_chunks * 256, 256), 256, 0, s>>>(CS[0], (uint32_t)(bp.max_chunks * 256));
   for (size_t li = 0; li < plan.size(); ++li) {
     const LevelPlan& lp = plan[li];
     const TileDesc* tl = dtiles + lp.tile_base;
@@ -1207,11 +1227,11 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
     uint2 *vin = Vcur, *vout = Valt;
     // every launch of a pass skips the groups that need fewer passes
     for (uint32_t pass = 0; pass < 4; ++pass) {
-      k_radix_hist<<<lp.ntiles, kThreads, 0, s>>>(tl, gr, TP, kin, pass, H, CS);
-      k_radix_group_scan<<<lp.ngroups, kThreads, 0, s>>>(gr, GP, TP, CP, prev, TR, pass, CS, CB);
-      k_radix_chunk_offsets<<<lp.nchunks, kThreads, 0, s>>>(dchunk_tiles + lp.chunk_base, CP, pass,
-                                                            H, CB, O);
-      k_radix_scatter<<<lp.ntiles, kThreads, 0, s>>>(tl, TP, kin, vin, pass, O, lp.m, kout, vout);
+      uint32_t* const cs = CS[pass & 1];
+      k_radix_hist<<<lp.ntiles, kThreads, 0, s>>>(tl, gr, TP, kin, pass, H, cs, CS[~pass & 1]);
+      if (lp.scan) k_radix_group_scan<<<lp.ngroups, kThreads, 0, s>>>(gr, GP, TP, prev, TR, pass, cs, CB);
+      k_radix_scatter<<<lp.ntiles, kThreads, 0, s>>>(tl, gr, TP, prev, TR, kin, vin, pass, H, cs,
+                                                     lp.scan ? CB : nullptr, lp.m, kout, vout);
       std::swap(kin, kout);
       std::swap(vin, vout);
     }
@@ -1219,9 +1239,7 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
     // are not read again, so Ka takes the next level's
     const bool last = li + 1 == plan.size();
     k_argmax_partial<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, TP, Vcur, Valt, partial);
-    k_argmax_combine<<<blocks(lp.nchildren, kThreads / 64), kThreads, 0, s>>>(ch, lp.nchildren,
-                                                                              partial, argpos);
-    k_emit<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, argpos, TP, Vcur, Valt, Vout, lp.first, lp.level, L,
+    k_emit<<<lp.ntiles, kThreads, 0, s>>>(tl, ch, partial, TP, Vcur, Valt, Vout, lp.first, lp.level, L,
                                           bb, N, ctx->perm.p, last ? nullptr : Ka, TR,
                                           last ? bbR : nullptr, last ? Ka : nullptr, m0);
     // rotate: the emit output is the next level's input
