@@ -196,8 +196,8 @@ aur_status aur_trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int3
 /* Launch shape of the trace entry points (no reference counterpart: the
  * reference launched one thread per ray in blocks of 64,
  * src/kernels/monteCarloRaytracer.cu:119-124).  persistent = 1: resident
- * waves each own a contiguous ray range and refill idle lanes once `refill`
- * (1..64) lanes are idle; waves_per_cu = 0 uses the occupancy
+ * waves take ranges of the rays and refill idle lanes once `refill` (1..64)
+ * lanes are idle; waves_per_cu = 0 uses the occupancy
  * limit, at most 16 to 24 by the tree's size.  persistent = 0: one lane per ray.  block: 64, 128 or 256.
  * stack_lds_rows: how many rows of each lane's stack of deferred ranges
  * (a compact stack of at most levels - 1 entries) live in LDS (0 = all);
