@@ -60,11 +60,6 @@ aur_status aur_create(int32_t device, aur_context** out) {
     delete ctx;
     return AUR_ERR_DEVICE;
   }
-  if (hipHostMalloc((void**)&ctx->root_host, sizeof(aur::NodeRec)) != hipSuccess) {
-    (void)hipStreamDestroy(ctx->stream);
-    delete ctx;
-    return AUR_ERR_OOM;
-  }
   // device address of the allocation-free entry points' scratch on this
   // device (once per device); on failure only those entry points refuse
   (void)aur::scratch_setup(device);
