@@ -111,6 +111,11 @@ constexpr uint32_t kDefaultRenderStackRows = 12;
 // and the work counters (kWorkWords) of the trace launches that use each word.
 constexpr uint32_t kStatsOffset = 8;
 constexpr uint32_t kWorkWords = 8 * 32;
+// Sets of work counters of the standalone traces: one for the launches queued
+// on the context's stream, which run one after the other, and one for each
+// launch recorded into a graph, which may be replayed beside them on any
+// stream.  Recorded launches beyond these take fixed ranges.
+constexpr uint32_t kTraceWorkSets = 128;
 constexpr uint32_t kTicketOffset = 32;
 constexpr uint32_t kCounterWords = kTicketOffset + 3 * kWorkWords;
 
@@ -207,7 +212,8 @@ struct aur_context {
   // limited residency: fastest shape measured at 1M triangles / 2^24 rays
   aur_trace_params trace_params{1, 256, 24, 0, 0};
   aur::DevBuf<float2> gstack;  // global rows of the persistent traversal stack
-  aur::DevBuf<uint32_t> trace_work;  // work counters of the persistent trace launches
+  aur::DevBuf<uint32_t> trace_work;  // kTraceWorkSets sets of work counters
+  uint32_t trace_work_recorded = 0;  // sets given to launches recorded into graphs
   aur_render_params render_params{aur::kDefaultMaxPaths, 0, aur::kDefaultRenderRefill,
                                   aur::kDefaultRenderStackRows};
   bool render_rows_default = true;  // stack_lds_rows was not chosen by the caller

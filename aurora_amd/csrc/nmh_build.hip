@@ -1262,7 +1262,7 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   AUR_HIP(ctx, ctx->texcoords.reserve((size_t)N * 6));
   AUR_HIP(ctx, ctx->shader_ids.reserve(N));
   AUR_HIP(ctx, ctx->nodes.reserve((size_t)n + 1));
-  AUR_HIP(ctx, ctx->trace_work.reserve(kWorkWords));
+  AUR_HIP(ctx, ctx->trace_work.reserve((size_t)kTraceWorkSets * kWorkWords));
   k_gather_geometry<<<blocks(N, 256), 256, 0, s>>>(ctx->perm.p, N, ctx->in_vertices.p,
                                                    ctx->in_normals.p, ctx->in_texcoords.p,
                                                    ctx->in_shader_ids.p, ctx->vertices.p,

@@ -230,12 +230,21 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
   }
   // (Clearing the counters in the launch itself, by the last block of each
   // group, put 128 atomics on one address at its end: 36 us at 2^20 rays.)
+  uint32_t* work = nullptr;
   if (n > (uint64_t)grid * block) {
-    k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(ctx->trace_work.p);
+    hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
+    AUR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &recording));
+    if (recording == hipStreamCaptureStatusNone)
+      work = ctx->trace_work.p;
+    else if (ctx->trace_work_recorded + 1 < kTraceWorkSets)
+      work = ctx->trace_work.p + (size_t)++ctx->trace_work_recorded * kWorkWords;
+  }
+  if (work) {
+    k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
     AUR_LAUNCH_CHECK(ctx, "k_zero_work");
   }
   hipLaunchKernelGGL(fn, dim3(grid), dim3(block), lds_pt, ctx->stream, ctx->nodes.p, ctx->vertices.p,
-                     ctx->count / 2, rays, n, hits, ids, ctx->trace_work.p, tp.refill, gstack, klds, maxrows - rows);
+                     ctx->count / 2, rays, n, hits, ids, work, tp.refill, gstack, klds, maxrows - rows);
   AUR_LAUNCH_CHECK(ctx, "k_trace_pt");
   return AUR_OK;
 }

@@ -190,7 +190,9 @@ uint32_t aur_geometry_count(const aur_context* ctx);
 
 /* ---- traversal (the device functions intersect()/intersectAny(),
  * src/kernels/lib/intersect.cuh:36-152, as standalone launches).  Device
- * pointers; queued on the context stream. ---- */
+ * pointers; queued on the context stream, or recorded into the graph that the
+ * stream is capturing (replay such a graph on any stream, one replay at a
+ * time). ---- */
 aur_status aur_trace_closest(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_hit* hits);
 aur_status aur_trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int32_t* hit_ids);
 /* Launch shape of the trace entry points (no reference counterpart: the
