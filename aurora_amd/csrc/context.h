@@ -114,7 +114,7 @@ constexpr uint32_t kWorkWords = 8 * 32;
 // Sets of work counters of the standalone traces: one for the launches queued
 // on the context's stream, which run one after the other, and one for each
 // launch recorded into a graph, which may be replayed beside them on any
-// stream.  Recorded launches beyond these take fixed ranges.
+// stream.  Recorded launches beyond these give every wave one range of 64 rays.
 constexpr uint32_t kTraceWorkSets = 128;
 constexpr uint32_t kTicketOffset = 32;
 constexpr uint32_t kCounterWords = kTicketOffset + 3 * kWorkWords;

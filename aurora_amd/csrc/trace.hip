@@ -238,8 +238,20 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
       work = ctx->trace_work.p;
     else if (ctx->trace_work_recorded + 1 < kTraceWorkSets)
       work = ctx->trace_work.p + (size_t)++ctx->trace_work_recorded * kWorkWords;
-  }
-  if (work) {
+    else {  // no set left: one range per wave (the test on a null counter in the kernel cost any-hit queries 1.5%)
+      const Kern all = wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>;
+      constexpr uint64_t kSlice = 1ull << 30;
+      for (uint64_t at = 0; at < n; at += kSlice) {
+        const uint64_t m = std::min(kSlice, n - at);
+        hipLaunchKernelGGL(all, dim3((uint32_t)((m + block - 1) / block)), dim3(block),
+                           (size_t)maxrows * block * sizeof(float2), ctx->stream, ctx->nodes.p, ctx->vertices.p,
+                           ctx->count / 2, rays + at, m, hits ? hits + at : nullptr, ids ? ids + at : nullptr, nullptr,
+                           tp.refill, nullptr, 0u, 0u);
+        AUR_LAUNCH_CHECK(ctx, "k_trace_pt");
+      }
+      return AUR_OK;
+    }
+    k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
     k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
     AUR_LAUNCH_CHECK(ctx, "k_zero_work");
   }

@@ -539,8 +539,7 @@ __device__ __forceinline__ uint64_t trav_visit(Trav& s, WaveState& w, const Tree
 // chunk is a sixteenth of a share, at least one ray per lane (first ranges of
 // 128 and 192 rays, chunks of 128 and first ranges of 3/4 of a share were up
 // to 25% slower on the camera rays).  Launches of at most one first range per
-// wave use no counter, and a null counter gives every wave one range.  The
-// blocks form kWorkGroups groups, each with a
+// wave use no counter.  The blocks form kWorkGroups groups, each with a
 // counter of its own in its own cache line (group g's t-th chunk is chunk
 // t * groups + g): one address takes an atomic about every 12 ns, which
 // bounded launches of short rays (the Cornell frame took 2.68 ms with a
@@ -559,7 +558,7 @@ struct WaveWork {
     const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const uint64_t share = n >> 32 ? n / waves : (uint64_t)((uint32_t)n / waves);
-    const uint64_t first = !tickets ? (share + 64) & ~63ull : (share < 512 ? 64 : (share / 2) & ~63ull);
+    const uint64_t first = share < 512 ? 64 : (share / 2) & ~63ull;
     const uint64_t sixteenth = (share / 16 + 63) & ~63ull;
     chunk = sixteenth < 64 ? 64u : (sixteenth > (1u << 20) ? 1u << 20 : (uint32_t)sixteenth);
     groups = gridDim.x < kWorkGroups ? gridDim.x : kWorkGroups;

@@ -64,7 +64,7 @@ def test_replays_beside_queued_traces(setup):
 
 
 def test_more_recorded_launches_than_counter_sets(setup):
-    """Launches recorded after the counter sets are used up take fixed ranges."""
+    """Launches recorded after the counter sets are used up need none."""
     import torch
 
     ctx, stream, rays, want = setup
