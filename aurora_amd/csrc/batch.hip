@@ -50,7 +50,6 @@ aur_status aur_scene_add(aur_context* ctx, uint32_t count, const float* vertices
   sc->nodes.swap(ctx->nodes);
   sc->root_lo = ctx->root_lo;
   sc->root_hi = ctx->root_hi;
-  sc->bound = ctx->bound;
   sc->vertices.swap(ctx->vertices);
   sc->normals.swap(ctx->normals);
   sc->shader_ids.swap(ctx->shader_ids);
@@ -119,7 +118,6 @@ aur_status aur_batch_render(aur_context* ctx, uint32_t njobs, const aur_job* job
     J.n_nodes = sc.count / 2;
     J.root_lo = sc.root_lo;
     J.root_hi = sc.root_hi;
-    J.bound = sc.bound;
     J.num_shaders = sc.num_shaders;
     J.num_lights = sc.num_lights;
     J.nslots = sc.nslots;

@@ -305,6 +305,12 @@ aur_status aur_check_division(aur_context* ctx, uint64_t samples, uint64_t seed,
   return aur::division_check(ctx, samples, seed, recip_checked, recip_bad, quot_bad);
 }
 
+aur_status aur_check_reject(aur_context* ctx, uint64_t n, const aur_ray* rays, uint64_t* visits, uint64_t* exact,
+                            uint64_t* missed) {
+  if (!ctx) return AUR_ERR_INVALID_ARG;
+  return aur::reject_check(ctx, n, rays, visits, exact, missed);
+}
+
 aur_status aur_trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int32_t* hit_ids) {
   if (!ctx) return AUR_ERR_INVALID_ARG;
   return aur::trace_any(ctx, n, rays, hit_ids);

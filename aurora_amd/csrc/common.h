@@ -196,7 +196,8 @@ constexpr uint32_t kKeyCompat = 0x2545F491u;
 // need the reference's triangle test on their exact vertices:
 //   scale     2^(1-k) with 2^k at least the extent of the node's two triangles
 //             and of its group (its own, its parent's and its grandparent's
-//             slabs), or infinity: no reject test for this node
+//             slabs, but for far larger ones), or infinity: no reject test
+//             for this node
 //   ref       scale * v1 of the first triangle (exact float)
 //   e         half pairs (first, second triangle) of scale / 2 * e1.xyz, e2.xyz
 //   dxy, dz_a half pairs (dx, dy) and (dz, size of the first triangle):
@@ -205,8 +206,7 @@ constexpr uint32_t kKeyCompat = 0x2545F491u;
 //             triangle's size (half) in bits 0..15 and kNodeSlabsOdd as the sign
 // A triangle's size is at least the largest |component| of its scaled edges,
 // and at least 2^-10.  Record K holds node K - 1, so that siblings share a
-// 128-byte line; record 0 holds the root's own slab (axis 0) in cslab[0..1]
-// and the largest |coordinate| of the tree's vertices in ref[0].
+// 128-byte line; record 0 holds the root's own slab (axis 0) in cslab[0..1].
 constexpr uint32_t kNodeSlabsOdd = 1u << 31;  // some cslab value fails normal_coord
 // Trees from here on have records beyond a 32-bit byte offset.
 constexpr uint32_t kWideNodes = 1u << 26;
@@ -236,7 +236,7 @@ static_assert(sizeof(NodeRec) == 64, "node record");
 // these ranges and coordinates up to kRejectCoord; outside them every
 // triangle takes the exact test.
 constexpr float kRejectScaleMin = 0x1p-40f, kRejectScaleMax = 0x1p40f;
-constexpr float kRejectDirMin = 0x1p-20f, kRejectDirMax = 0x1p20f;
+constexpr float kRejectDirMin = 0x1p-40f, kRejectDirMax = 0x1p40f;
 constexpr float kRejectCoord = 0x1p40f;
 
 // Subtree arithmetic of a left-complete binary tree of n nodes in heap order.

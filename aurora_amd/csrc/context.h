@@ -141,14 +141,14 @@ struct JobDev {
   uint32_t n_nodes, num_shaders, num_lights, nslots;
   uint32_t w, h, npix, spp, max_depth, rr_start, seed, paths;
   uint32_t rx0, ry0, rw;
-  float root_lo, root_hi, bound;  // record 0 of the tree's nodes
+  float root_lo, root_hi;  // record 0 of the tree's nodes
   aur_camera cam;
 };
 
 // A built scene kept for batches: tree-order arrays as the frame render uses.
 struct SceneStore {
   uint32_t count = 0, levels = 0, num_shaders = 0, num_lights = 0, nslots = 0;
-  float root_lo = 0.0f, root_hi = 0.0f, bound = 0.0f;  // record 0 of the nodes
+  float root_lo = 0.0f, root_hi = 0.0f;  // record 0 of the nodes
   DevBuf<NodeRec> nodes;
   DevBuf<float> vertices;
   DevBuf<float> normals;
@@ -239,7 +239,7 @@ struct aur_context {
   aur::DevBuf<uint16_t> shader_ids;
   aur::DevBuf<uint32_t> perm;
   aur::DevBuf<aur::NodeRec> nodes;
-  float root_lo = 0.0f, root_hi = 0.0f, bound = 0.0f;  // host copy of record 0
+  float root_lo = 0.0f, root_hi = 0.0f;  // host copy of record 0
 
   // materials and lights
   aur::DevBuf<aur_shader> shaders;
@@ -323,6 +323,8 @@ aur_status trace_closest(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_
 aur_status trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int32_t* ids);
 aur_status division_check(aur_context* ctx, uint64_t samples, uint64_t seed, uint64_t* recip_checked,
                           uint64_t* recip_bad, uint64_t* quot_bad);
+aur_status reject_check(aur_context* ctx, uint64_t n, const aur_ray* rays, uint64_t* visits, uint64_t* exact,
+                        uint64_t* missed);
 aur_status trace_closest_count(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_hit* hits,
                                uint64_t* popped, uint64_t* passed);
 // Argument and state checks of frame_render; no work is queued.

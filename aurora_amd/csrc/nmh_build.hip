@@ -900,10 +900,6 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
   NodeRec r = {};
   if (K == 0) {
     slab_of(v, 0, r.cslab[0], r.cslab[1]);
-    // the triangles of depths 0..2 hold the extremes of x, y and z
-    for (uint32_t k = 0; k < min(n, 7u); ++k)
-#pragma unroll
-      for (int i = 0; i < 18; ++i) r.ref[0] = fmaxf(r.ref[0], fabsf(v[18 * k + i]));
     nodes[0] = r;
     *root = r;
     return;
@@ -921,8 +917,15 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
 #pragma unroll
   for (int c = 0; c < 4; ++c) normal = normal && normal_coord(r.cslab[c]);
   // the group's extent: the two triangles on every axis, and the slabs of
-  // the parent and the grandparent on theirs (the node's own is its triangles')
-  float extent = 0.0f, coord = 0.0f;
+  // the parent and the grandparent on theirs (the node's own is its triangles').
+  // A slab 2^15 times as large as a triangle of the node and 2^8 times the
+  // extent of both (under a ground plane or a sky dome) is left out: the halves
+  // could not hold the triangle in its units, and in the triangles' own the test
+  // works for the rays that meet the node near them.
+  float extent = 0.0f, coord = 0.0f, larger[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < 18; ++i)
+    if (i % 3) larger[i / 9] = fmaxf(larger[i / 9], fabsf(p[i] - p[i - i % 3]));
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     float lo, hi;
@@ -931,11 +934,12 @@ __global__ void k_node_records(const float* __restrict__ v, uint32_t n, NodeRec*
     coord = fmaxf(coord, fmaxf(fabsf(lo), fabsf(hi)));
   }
   uint32_t anc = k;
+  const float limit = fmaxf(0x1p8f * extent, 0x1p15f * fminf(larger[0], larger[1]));
   for (uint32_t up = 1; up <= 2 && up <= d; ++up) {
     float lo, hi;
     anc = (anc - 1) / 2;
     slab_of(v + (size_t)anc * 18, (int)((d - up) % 3), lo, hi);
-    extent = fmaxf(extent, hi - lo);
+    if (hi - lo <= limit) extent = fmaxf(extent, hi - lo);
   }
   int ex = 0;
   (void)frexpf(extent, &ex);  // extent < 2^ex
@@ -1278,7 +1282,6 @@ aur_status nmh_build(aur_context* ctx, aur_build_stats* stats, bool tangents) {
   // record 0, for launches that start every ray at the root without reading it
   ctx->root_lo = ctx->root_host->cslab[0];
   ctx->root_hi = ctx->root_host->cslab[1];
-  ctx->bound = ctx->root_host->ref[0];
   // A rebuild of the same size (an edit, a deforming mesh) finds its scratch
   // in place.  Beyond the limit (about 3.3M triangles) the build outweighs the
   // allocation.

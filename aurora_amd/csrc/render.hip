@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
     for (uint32_t i = threadIdx.x; i < kWorkWords; i += blockDim.x)
       a.counters[kTicketOffset + (w == 2u ? 0u : w + 1u) * kWorkWords + i] = 0;
   persistent_trace<false, true, kWide>(
-      TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, RootInfo{a.job.root_lo, a.job.root_hi, a.job.bound}}, (uint64_t)n_ext + n_sh,
+      TreeRef{a.job.nodes, a.job.tris, a.job.n_nodes, RootInfo{a.job.root_lo, a.job.root_hi}}, (uint64_t)n_ext + n_sh,
       a.counters + kTicketOffset + w * kWorkWords, a.refill, stack,
       [&](uint64_t i, V3& o, V3& d, float& tmax, TreeRef& tree, bool& any) {
         float4 o4, d4;
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void k_pbr_trace(PbrArgs a, uint32_t w, uin
         }
         if constexpr (kMulti) {
           const JobDev& J = a.jobs[jb];
-          tree = TreeRef{J.nodes, J.tris, J.n_nodes, RootInfo{J.root_lo, J.root_hi, J.bound}};
+          tree = TreeRef{J.nodes, J.tris, J.n_nodes, RootInfo{J.root_lo, J.root_hi}};
         }
         o = mk(o4.x, o4.y, o4.z);
         d = mk(d4.x, d4.y, d4.z);
@@ -1469,7 +1469,6 @@ JobDev frame_job(aur_context* ctx, const aur_camera* cam, const aur_render_opts*
   J.n_nodes = ctx->count / 2;
   J.root_lo = ctx->root_lo;
   J.root_hi = ctx->root_hi;
-  J.bound = ctx->bound;
   J.num_shaders = ctx->num_shaders;
   J.num_lights = ctx->num_lights;
   J.nslots = ctx->num_slots;

@@ -120,8 +120,36 @@ __global__ __launch_bounds__(kMaxBlock) void k_trace_count(const NodeRec* __rest
   }
 }
 
-__global__ void k_zero2(unsigned long long* p) {
-  if (threadIdx.x < 2) p[threadIdx.x] = 0ull;
+// Self-check of the reject test: RejectCount summed over the rays.
+__global__ __launch_bounds__(kMaxBlock) void k_reject_check(const NodeRec* __restrict__ nodes,
+                                                            const float* __restrict__ tris, uint32_t n_nodes,
+                                                            const aur_ray* __restrict__ rays, uint64_t n,
+                                                            unsigned long long* __restrict__ sums) {
+  extern __shared__ float2 stk_mem[];
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  RejectCount c;
+  if (i < n) {
+    const float4* r = reinterpret_cast<const float4*>(rays + i);
+    const float4 a = r[0], b = r[1];
+    Trav s;
+    trace_ray<false, false, true>(s, TreeRef{nodes, tris, n_nodes, {}}, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w,
+                                  stk_mem + threadIdx.x, blockDim.x, nullptr, &c);
+  }
+  uint32_t v = c.visits, e = c.exact, m = c.missed;
+  for (int off = 32; off > 0; off >>= 1) {
+    v += __shfl_xor(v, off);
+    e += __shfl_xor(e, off);
+    m += __shfl_xor(m, off);
+  }
+  if ((threadIdx.x & 63u) == 0) {
+    atomicAdd(&sums[0], (unsigned long long)v);
+    atomicAdd(&sums[1], (unsigned long long)e);
+    if (m) atomicAdd(&sums[2], (unsigned long long)m);
+  }
+}
+
+__global__ void k_zero3(unsigned long long* p) {
+  if (threadIdx.x < 3) p[threadIdx.x] = 0ull;
 }
 
 // Self-check of the division shortcuts used by the traversal:
@@ -268,8 +296,8 @@ aur_status trace_closest_count(aur_context* ctx, uint64_t n, const aur_ray* rays
   if (!ctx->built) return ctx->fail(AUR_ERR_STATE, "trace: geometry not built");
   if (!rays || !hits) return ctx->fail(AUR_ERR_INVALID_ARG, "trace: null buffer");
   DevBuf<unsigned long long> sums;
-  AUR_HIP(ctx, sums.reserve(2));
-  k_zero2<<<1, 64, 0, ctx->stream>>>(sums.p);
+  AUR_HIP(ctx, sums.reserve(3));
+  k_zero3<<<1, 64, 0, ctx->stream>>>(sums.p);
   if (n) {
     const uint32_t block = 128;
     const uint64_t nb = (n + block - 1) / block;
@@ -287,11 +315,36 @@ aur_status trace_closest_count(aur_context* ctx, uint64_t n, const aur_ray* rays
   return AUR_OK;
 }
 
+aur_status reject_check(aur_context* ctx, uint64_t n, const aur_ray* rays, uint64_t* visits, uint64_t* exact,
+                        uint64_t* missed) {
+  if (!ctx->built) return ctx->fail(AUR_ERR_STATE, "check: geometry not built");
+  if (n && !rays) return ctx->fail(AUR_ERR_INVALID_ARG, "check: null buffer");
+  DevBuf<unsigned long long> sums;
+  AUR_HIP(ctx, sums.reserve(3));
+  k_zero3<<<1, 64, 0, ctx->stream>>>(sums.p);
+  if (n) {
+    const uint32_t block = 128;
+    const uint64_t nb = (n + block - 1) / block;
+    if (nb > 0x7FFFFFFFull) return ctx->fail(AUR_ERR_INVALID_ARG, "check: too many rays");
+    const size_t lds = (size_t)ctx->levels * block * sizeof(float2);
+    k_reject_check<<<(uint32_t)nb, block, lds, ctx->stream>>>(ctx->nodes.p, ctx->vertices.p, ctx->count / 2, rays, n,
+                                                              sums.p);
+    AUR_LAUNCH_CHECK(ctx, "k_reject_check");
+  }
+  unsigned long long h[3] = {0, 0, 0};
+  AUR_HIP(ctx, hipMemcpyAsync(h, sums.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+  AUR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  if (visits) *visits = h[0];
+  if (exact) *exact = h[1];
+  if (missed) *missed = h[2];
+  return AUR_OK;
+}
+
 aur_status division_check(aur_context* ctx, uint64_t samples, uint64_t seed, uint64_t* recip_checked,
                           uint64_t* recip_bad, uint64_t* quot_bad) {
   DevBuf<unsigned long long> sums;
-  AUR_HIP(ctx, sums.reserve(2));
-  k_zero2<<<1, 64, 0, ctx->stream>>>(sums.p);
+  AUR_HIP(ctx, sums.reserve(3));
+  k_zero3<<<1, 64, 0, ctx->stream>>>(sums.p);
   const uint32_t lo = 0x21800000u, hi = 0x5F800000u;  // 2^-60 .. 2^64
   k_division_check<<<4096, 256, 0, ctx->stream>>>(lo, hi, samples, seed, sums.p);
   AUR_LAUNCH_CHECK(ctx, "k_division_check");

@@ -122,12 +122,18 @@ struct TraceCount {
   uint32_t popped = 0, passed = 0;
 };
 
+// Counters of the reject test: node visits, triangles it left to the exact
+// test, and rejected triangles that the exact test accepts.
+struct RejectCount {
+  uint32_t visits = 0, exact = 0, missed = 0;
+};
+
 // Node indices are kept 1-based (K = k + 1: children 2K and 2K + 1, sibling
 // K ^ 1, ancestor by shift) and depths one-hot (depth d: 1 << d), so that the
 // axis and a pending entry's depth are bit tests.
 struct Trav {
   V3 o, d, y;      // origin, direction, RN(1/direction)
-  float rj_size, rj_scale, rj;  // the reject test's threshold terms (trav_test)
+  float rj_size, rj_far, rj;  // the reject test's threshold terms (trav_test)
   uint32_t fast;   // bit m: the children of a node at depth m take the reciprocal quotient
   float t, u, v;   // current closest hit (t = ray.t)
   int32_t id;
@@ -212,10 +218,9 @@ __device__ __forceinline__ bool fast_axis(float o, float d) {
   return (a >= 0x1p-60f) & (a <= 16.0f) & normal & (fabsf(o) <= 0x1p57f);
 }
 
-// What record 0 says of a tree: the root's own slab and the largest
-// |coordinate| of its vertices.
+// The root's own slab (record 0 of a tree).
 struct RootInfo {
-  float lo, hi, bound;
+  float lo, hi;
 };
 
 // The tree a lane traverses: node records, the triangles' vertices in tree
@@ -228,14 +233,14 @@ struct TreeRef {
 };
 
 __device__ __forceinline__ RootInfo root_info(const NodeRec* __restrict__ nodes) {
-  return RootInfo{nodes[0].cslab[0], nodes[0].cslab[1], nodes[0].ref[0]};
+  return RootInfo{nodes[0].cslab[0], nodes[0].cslab[1]};
 }
 
 // The reject test's threshold (trav_test).
 constexpr float kRejA = 1.6e-3f;                            // times 2 |C|max
 constexpr float kRejSize = 2.0f * 3.4f * kRejA;             // 2 thr's terms times D: z,
 constexpr float kRejB = 2.0f * 8.125f * 0x1p-12f;           // constant,
-constexpr float kRejScale = 0x1p-18f;                       // and the record's scale (2 P + O)
+constexpr float kRejFar = 48.0f * 0x1p-24f;                 // and D times 2 sigma t
 
 // Sets up a ray; returns false when the root's slab culls it (finished, miss).
 // The reciprocals y serve only axes with 2^-60 <= |d| <= 16, where recip_rn
@@ -260,7 +265,7 @@ __device__ __forceinline__ bool trav_init_root(Trav& s, RootInfo root, V3 o, V3 
     const bool in = (dm >= kRejectDirMin) & (dm <= kRejectDirMax) & (om <= kRejectCoord) & (all == all);
     s.rj = in ? dm * kRejB : __builtin_nanf("");
     s.rj_size = dm * kRejSize;
-    s.rj_scale = dm * __builtin_fmaf(2.0f, root.bound, om) * kRejScale;
+    s.rj_far = dm * dm * kRejFar;
   }
   s.t = tmax;
   s.u = s.v = 0.0f;
@@ -284,7 +289,7 @@ __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3
 // pass the reference's test.  Two things bound a visit when every lane reads
 // another node: VALU issue and the vector L1, which looks up one lane's 16
 // bytes per cycle and CU.  Both triangles' exact test took 125 VALU
-// instructions and a 96-byte record 6 loads; this test takes 66 and the
+// instructions and a 96-byte record 6 loads; this test takes 67 and the
 // 64-byte record 4, and what it leaves over (1.2% of the visits at 1M
 // triangles) costs 6 more per visit.  2^24 incoherent rays into 1M triangles
 // take 4.6 ms (7.3 with the exact tests in every visit): 2.35e9 VALU
@@ -296,31 +301,37 @@ __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3
 // Moller-Trumbore numerators are u det = e2 . C, v det = -(e1 . C) and
 // det = -d . (e1 x e2); the reference's test accepts only if none of the
 // three edge functions u det, v det and (1 - u - v) det is negative (but for
-// rounding).  p is the ray's entry into the node's range, so that T is no
-// larger than the node's group, and lengths are in units of the group's size.
+// rounding).  p = o + t d is the ray's entry into the node's range, so that T
+// is no larger than the node's group, and lengths are in units of the group's
+// size.  T is computed as (o - v1) + t d, whose rounding does not grow with the
+// coordinates: with p computed first and a threshold for the largest coordinate
+// of the tree, 2^22 incoherent rays into 1M triangles over a ground plane 2000 km
+// wide took 2.95 ms, 1.56 now (1.40 without the plane), 1000 km 2.20 ms, 1.55 now.
 //
 // Bound.  D = the largest |direction component|, z = the triangle's size (each
-// |e| component <= z), q = 2^-11 + 2^-15, t = the range's entry, P = the
-// largest |coordinate| of the tree, O of the origin; sigma = 2^-k, half of
-// the record's scale (T, and so C and the numerators, come out doubled).
+// |e| component <= z), q = 2^-11 + 2^-15, t = the range's entry; sigma = 2^-k,
+// half of the record's scale (T, and so C and the numerators, come out doubled).
 //   edges: rounding to half moves a component by at most q z (2^-11 relative,
 //     2^-25 absolute, z >= 2^-10);
 //   T: off by at most 2^-12 (dv, |dv| <= 1) + 2^-15 (roundings of dv and T,
-//     |T| <= 4) + 2^-24 sigma |p|max (one fma for p); C by 2 D times that and
-//     2^-22 D;
-//   u det, v det: z (3 q |C|max + D (6.82 2^-12 + 6 2^-24 sigma |p|max));
+//     |T| <= 4) + 2^-24 sigma |o - v1|max (one fma for o - v1; the scale is a
+//     power of two); C by 2 D times that and 2^-22 D;
+//   u det, v det: z (3 q |C|max + D (6.82 2^-12 + 6 2^-24 sigma |o - v1|max));
 //   det: e1 x e2 in half, 3 D ((4.01 q + 3 2^-11) z^2 + 2^-24);
 //   the reference's floats: 36 2^-24 z D sigma |o - v1|max per numerator
-//     (T, P or Q and the dot product), sigma |o - v1|max <= sigma t D + 5.
-// With |T| <= 4, |p|max <= P + 4 / sigma and t D <= |p|max + O, so the terms in
-// sigma are at most 36 2^-24 z D (sigma (2 P + O) + 8).  A triangle that the
-// reference accepts has, with
-//   thr = A |C|max + 3.4 A z D + D (B + 2^-18 sigma (2 P + O)),
+//     (T, P or Q and the dot product).
+// With |T| <= 4 (5 for the second triangle), sigma |o - v1|max <= sigma t D + 5,
+// so the terms in sigma are at most 42 2^-24 z D (sigma t D + 5): only a ray
+// that comes from some 10^5 sizes of the group away loses the test's use.  A
+// triangle that the reference accepts has, with
+//   thr = A |C|max + 3.4 A z D + D (B + 48 2^-24 sigma t D),
 // u det >= -z thr, v det >= -z thr and (1 - u - v) det >= -2 z thr:
 // A = 1.6e-3 >= 3 q = 1.557e-3; half the third function's error is that of
 // one numerator plus z D 5.32e-3 z, below 3.4 A z = 5.44e-3 z, plus 0.38 2^-12
-// z D, and B = 8.125 2^-12 >= (6.82 + 0.38) 2^-12 + 2^-15 with a margin for the
-// float roundings of this test itself (below 2^-18 z D).
+// z D, and B = 8.125 2^-12 >= (6.82 + 0.38 + 0.06) 2^-12 + 2^-15 with a margin for
+// the float roundings of this test itself (below 2^-18 z D).  Nothing here over-
+// or underflows for D in 2^-40 .. 2^40 and coordinates up to 2^40, nor does
+// the reference's test of a triangle that it accepts.
 // Comparisons are written so that NaN and infinity keep a triangle.
 __device__ __forceinline__ float lo16(half2v h) { return (float)h.x; }
 __device__ __forceinline__ float hi16(half2v h) { return (float)h.y; }
@@ -342,7 +353,7 @@ __device__ __forceinline__ float sub_hi16(float a, half2v h) {
 }
 
 // Whether the triangle may be accepted: T doubled, edges e1 and e2, size and
-// det in the record's units; base = 2 D (B + 2^-18 sigma (2 P + O)).
+// det in the record's units; base = 2 D (B + 48 2^-24 sigma t D).
 __device__ __forceinline__ bool may_hit(V3 T, V3 d, V3 e1, V3 e2, float det, float size, float rj_size, float base) {
   const float cx = __builtin_fmaf(T.y, d.z, -(T.z * d.y));
   const float cy = __builtin_fmaf(T.z, d.x, -(T.x * d.z));
@@ -374,12 +385,12 @@ __device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCou
   const half2v dxy = h2(a3.z), dza = h2(a3.w), szb = h2(a1.w);
   const float scale = __uint_as_float(a1.w & 0x7F800000u);
   const V3 d = s.d;
-  const V3 p = mk(__builtin_fmaf(s.r.x, d.x, s.o.x), __builtin_fmaf(s.r.x, d.y, s.o.y),
-                  __builtin_fmaf(s.r.x, d.z, s.o.z));
-  const V3 Ta = mk(__builtin_fmaf(p.x, scale, -__uint_as_float(a1.x)), __builtin_fmaf(p.y, scale, -__uint_as_float(a1.y)),
-                   __builtin_fmaf(p.z, scale, -__uint_as_float(a1.z)));
+  const float ts = s.r.x * scale;
+  const V3 Ta = mk(__builtin_fmaf(ts, d.x, __builtin_fmaf(s.o.x, scale, -__uint_as_float(a1.x))),
+                   __builtin_fmaf(ts, d.y, __builtin_fmaf(s.o.y, scale, -__uint_as_float(a1.y))),
+                   __builtin_fmaf(ts, d.z, __builtin_fmaf(s.o.z, scale, -__uint_as_float(a1.z))));
   const V3 Tb = mk(sub_lo16(Ta.x, dxy), sub_hi16(Ta.y, dxy), sub_lo16(Ta.z, dza));
-  const float base = __builtin_fmaf(scale, s.rj_scale, s.rj);
+  const float base = __builtin_fmaf(ts, s.rj_far, s.rj);
   // e1 x e2 of both triangles at once
   const half2v nx = __builtin_elementwise_fma(e1y, e2z, -(e1z * e2y));
   const half2v ny = __builtin_elementwise_fma(e1z, e2x, -(e1x * e2z));
@@ -397,11 +408,10 @@ __device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCou
   __asm__ volatile("" : "+v"(s.slab.x), "+v"(s.slab.y), "+v"(s.slab.z), "+v"(s.slab.w));
 }
 
-// The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of the
-// node's first or second triangle, on the vertices it was uploaded with;
-// returns whether it became the closest hit.
-__device__ __forceinline__ bool trav_exact(Trav& s, const float* __restrict__ tris, bool first) {
-  const uint32_t tri = 2 * s.K - (first ? 2u : 1u);
+// The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of a
+// triangle on the vertices it was uploaded with, for any t above kEpsilon.
+__device__ __forceinline__ bool tri_accept(const Trav& s, const float* __restrict__ tris, uint32_t tri, float& u,
+                                           float& v, float& t) {
   const float* p = tris + (size_t)tri * 9;  // points layout: x1 x2 x3 y1 y2 y3 z1 z2 z3
   const V3 v1 = mk(p[0], p[3], p[6]);
   const V3 e1 = mk(p[1], p[4], p[7]) - v1, e2 = mk(p[2], p[5], p[8]) - v1;
@@ -409,8 +419,15 @@ __device__ __forceinline__ bool trav_exact(Trav& s, const float* __restrict__ tr
   const float det = dot(e1, P);
   float inv = recip_rn(det);
   if (det > kRecipMax) inv = 1.0f / det;
+  return tri_finish(s.o, s.d, v1, e1, e2, P, det, inv, u, v, t) & (t > kEpsilon);
+}
+
+// The same of the node's first or second triangle; returns whether it became
+// the closest hit.
+__device__ __forceinline__ bool trav_exact(Trav& s, const float* __restrict__ tris, bool first) {
+  const uint32_t tri = 2 * s.K - (first ? 2u : 1u);
   float u, v, t;
-  const bool hit = tri_finish(s.o, s.d, v1, e1, e2, P, det, inv, u, v, t) & (t > kEpsilon) & (t < s.t);
+  const bool hit = tri_accept(s, tris, tri, u, v, t) & (t < s.t);
   if (hit) {
     s.t = t;
     s.u = u;
@@ -638,9 +655,9 @@ __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint
 
 // Whole traversal of one ray by one lane.
 // stk: this lane's stack column, stk[depth * stride].
-template <bool kAny, bool kCount = false>
+template <bool kAny, bool kCount = false, bool kCheck = false>
 __device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3 d, float tmax, float2* stk,
-                                          uint32_t stride, TraceCount* cnt = nullptr) {
+                                          uint32_t stride, TraceCount* cnt = nullptr, RejectCount* rej = nullptr) {
   const LdsStack st = lds_stack(stk, stride);
   if (!trav_init<kCount>(s, tree, o, d, tmax, cnt)) return;
   bool popping = false;
@@ -648,6 +665,14 @@ __device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3
     if (!popping) {
       bool a, b;
       trav_test<kCount, true>(s, tree, cnt, a, b);
+      if (kCheck) {
+        float u, v, t;
+        const bool hit_a = tri_accept(s, tree.tris, 2 * s.K - 2, u, v, t);
+        const bool hit_b = tri_accept(s, tree.tris, 2 * s.K - 1, u, v, t);
+        rej->visits += 1;
+        rej->exact += (uint32_t)a + (uint32_t)b;
+        rej->missed += (uint32_t)(!a & hit_a) + (uint32_t)(!b & hit_b);
+      }
       if (a && trav_exact(s, tree.tris, true) && kAny) return;
       if (b && trav_exact(s, tree.tris, false) && kAny) return;
     }

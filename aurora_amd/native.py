@@ -129,6 +129,7 @@ def load():
         "aur_trace_closest_stats": ([P, u64, P, P, ctypes.POINTER(u64), ctypes.POINTER(u64)], i32),
         "aur_check_division": ([P, u64, u64, ctypes.POINTER(u64), ctypes.POINTER(u64),
                                 ctypes.POINTER(u64)], i32),
+        "aur_check_reject": ([P, u64, P, ctypes.POINTER(u64), ctypes.POINTER(u64), ctypes.POINTER(u64)], i32),
         "aur_set_trace_params": ([P, ctypes.POINTER(TraceParams)], i32),
         "aur_get_trace_params": ([P, ctypes.POINTER(TraceParams)], i32),
         "aur_set_render_params": ([P, ctypes.POINTER(RenderParams)], i32),
@@ -423,6 +424,18 @@ class Context:
                                                  ctypes.byref(r), ctypes.byref(q)),
                     "check_division")
         return int(c.value), int(r.value), int(q.value)
+
+    def check_reject(self, rays: np.ndarray) -> tuple[int, int, int]:
+        """(node visits, triangles left to the exact test, wrongly rejected
+        triangles) of the traversal's reject test over host rays (n, 8)."""
+        import torch
+
+        r = torch.from_numpy(np.ascontiguousarray(rays, dtype=np.float32)).to("cuda")
+        torch.cuda.synchronize()
+        v, e, m = ctypes.c_uint64(), ctypes.c_uint64(), ctypes.c_uint64()
+        self._check(self._lib.aur_check_reject(self._h, r.shape[0], ctypes.c_void_p(r.data_ptr()), ctypes.byref(v),
+                                               ctypes.byref(e), ctypes.byref(m)), "check_reject")
+        return int(v.value), int(e.value), int(m.value)
 
     def trace_any_ptr(self, n: int, rays_ptr: int, ids_ptr: int) -> None:
         self._check(self._lib.aur_trace_any(self._h, n, ctypes.c_void_p(rays_ptr),

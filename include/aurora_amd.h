@@ -224,6 +224,14 @@ aur_status aur_trace_closest_stats(aur_context* ctx, uint64_t n, const aur_ray* 
  * 0.  Synchronous. */
 aur_status aur_check_division(aur_context* ctx, uint64_t samples, uint64_t seed,
                               uint64_t* recip_checked, uint64_t* recip_bad, uint64_t* quot_bad);
+/* Device self-check of the traversal's reject test (no reference counterpart:
+ * the reference tests both triangles of every node), over n closest-hit rays
+ * (device pointer): visits counts node visits, exact the triangles that the
+ * reject test leaves to the reference's test (up to two a visit), missed those
+ * it rejects although the reference's test accepts them for some t, which must
+ * be 0.  Synchronous. */
+aur_status aur_check_reject(aur_context* ctx, uint64_t n, const aur_ray* rays, uint64_t* visits, uint64_t* exact,
+                            uint64_t* missed);
 
 /* ---- frame (replaces MonteCarloRaytracer::createFrame/destroyFrame/
  * setRegion/render/framebuffer, src/render/monteCarloRaytracer.cpp:23-127,
