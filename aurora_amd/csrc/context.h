@@ -12,6 +12,7 @@
 
 #include "../../include/aurora_amd.h"
 #include "common.h"
+#include "launch_shape.h"
 
 namespace aur {
 
@@ -92,14 +93,6 @@ struct DevBuf {
     return hipSuccess;
   }
 };
-
-// LDS of a block so that at most `blocks` of them reside on a CU: `need`, or
-// that share of its 160 KB (a block less than fits, for the 1280-byte
-// allocation granules).
-inline size_t lds_for_blocks(size_t need, uint32_t blocks) {
-  const size_t share = 162560 / blocks / 1280 * 1280;
-  return need > share ? need : share;
-}
 
 // Default paths in flight per PBR wavefront pass (2^24 paths: about 2 GB of
 // path state plus 56 B per next-event slot and path).
