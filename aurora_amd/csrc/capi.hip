@@ -97,7 +97,8 @@ aur_status aur_set_render_params(aur_context* ctx, const aur_render_params* p) {
   ctx->render_params.max_paths = p->max_paths ? p->max_paths : aur::kDefaultMaxPaths;
   ctx->render_params.graph = p->graph;
   ctx->render_params.refill = p->refill ? p->refill : aur::kDefaultRenderRefill;
-  ctx->render_rows_default = p->stack_lds_rows == 0;
+  // the reported default selects it too: what aur_get_render_params gave can be set again
+  ctx->render_rows_default = p->stack_lds_rows == 0 || p->stack_lds_rows == aur::kDefaultRenderStackRows;
   ctx->render_params.stack_lds_rows = p->stack_lds_rows ? p->stack_lds_rows : aur::kDefaultRenderStackRows;
   return AUR_OK;
 }

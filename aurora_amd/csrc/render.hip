@@ -1238,18 +1238,15 @@ template <bool kMulti>
 aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, PbrArgs& a, size_t& lds,
                        uint32_t& grid) {
   FrameState& fr = ctx->frame;
-  const uint32_t maxrows = levels > 1 ? levels - 1 : 1;
-  // By default a frame keeps every row in LDS, which leaves 10 (30 levels) to
-  // 28 waves per CU.  A 12-row window lets 28 reside at any depth, but the
-  // lines of that many waves' visits push each other out of the L1: 1080p
-  // frame of 1M triangles (19 levels) 32.1 ms with the window, 27.3 with all
-  // rows; compat 7.70 / 7.12 ms; 102,424 triangles at 512^2 21.0 / 18.9 ms.  A
-  // batch's lanes walk several smaller trees and spend more instructions per
-  // visit on them, so it keeps the window: 5 jobs of two bounces 4.00 ms with
-  // it, 4.18 with all rows; 16 jobs of six 25.2 / 25.6 ms.
-  const uint32_t want = !ctx->render_rows_default ? ctx->render_params.stack_lds_rows
-                                                  : (kMulti ? kDefaultRenderStackRows : maxrows);
-  const uint32_t rows = want >= maxrows ? maxrows : want;
+  // By default a frame keeps every row in LDS and a batch 12, or as many more as
+  // the LDS holds that its residency reserves (15).  The more waves, the more
+  // the lines of their visits push each other out of the L1: a 640x360 frame of
+  // 1M triangles (19 levels, 16 waves per CU) takes 3.10 ms with all rows, 3.20
+  // with a chosen window of 10 rows and the 28 waves that it leaves room for;
+  // batches with 15 rows (20 waves), a window of 10 (28) and all rows: 17 levels,
+  // 16 jobs 17.8 / 20.9 / 17.5 ms (18 waves), 19 levels, 4 jobs 6.9 / 7.9 / 6.9
+  // (16 waves); 16 levels, 16 jobs 15.0 with 15 rows, which is all of them, and
+  // 15.1 with 12.
   // Waves per CU, as for the standalone launches (trace.hip); a render's
   // neighbouring shadow rays share more lines, so more waves pay: 28 / 24 / 20 /
   // 16 take 1.46 / 1.46 / 1.52 / 1.55 ms for a 256^2 frame of 2,584 triangles
@@ -1257,7 +1254,11 @@ aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, Pb
   // and 21.3 / 18.5 / 17.7 / 18.4 for a batch of 16 jobs.
   const size_t tree_bytes = (size_t)a.job.n_nodes * sizeof(NodeRec);
   const uint32_t cu_waves = !kMulti && tree_bytes < (1u << 20) ? 28 : 20;
-  lds = lds_for_blocks((size_t)rows * kBlock * sizeof(float2), cu_waves * 64 / kBlock);
+  const bool chosen = !ctx->render_rows_default;
+  const StackShape shape = stack_shape(
+      levels, chosen ? ctx->render_params.stack_lds_rows : (kMulti ? kDefaultRenderStackRows : 0u), chosen, kBlock, cu_waves);
+  const uint32_t rows = shape.rows, maxrows = shape.maxrows;
+  lds = shape.lds;
   grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, a.job.n_nodes), lds, max_items);
   a.gstack = nullptr;
   a.klds = rows;

@@ -214,12 +214,6 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
     AUR_LAUNCH_CHECK(ctx, "k_trace_flat");
     return AUR_OK;
   }
-  // stack rows: at most levels - 1 deferred entries; the first `rows` in
-  // LDS, the rest in global memory
-  const uint32_t L = ctx->levels;
-  const uint32_t maxrows = L > 1 ? L - 1 : 1;
-  const uint32_t rows = (tp.stack_lds_rows == 0 || tp.stack_lds_rows >= maxrows) ? maxrows : tp.stack_lds_rows;
-  const uint32_t klds = rows < maxrows ? rows : 0;
   // Waves per CU: each visits 64 records at a time, and the more waves, the
   // fewer of their lines stay in the L1 (32 KB) between a record's four loads;
   // the larger the tree, the more a refetch costs.  2^22 rays, ms with the
@@ -229,8 +223,12 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
   // 1.31; 204,802 (6.6 MB) 0.82 / 0.76 / 0.78 / 0.65.
   const size_t tree_bytes = (size_t)(ctx->count / 2) * sizeof(NodeRec);
   const uint32_t cu_waves = tree_bytes < (1u << 20) ? 24 : (tree_bytes < (5u << 19) ? 20 : 16);
-  const size_t need = (size_t)rows * block * sizeof(float2);
-  const size_t lds_pt = tp.waves_per_cu ? need : lds_for_blocks(need, cu_waves * 64 / block);
+  // stack rows: at most levels - 1 deferred entries; the first `rows` in
+  // LDS, the rest in global memory
+  const StackShape shape =
+      stack_shape(ctx->levels, tp.stack_lds_rows, tp.stack_lds_rows != 0, block, tp.waves_per_cu ? 0 : cu_waves);
+  const uint32_t rows = shape.rows, maxrows = shape.maxrows, klds = rows < maxrows ? rows : 0;
+  const size_t lds_pt = shape.lds;
   // resident waves: occupancy-limited blocks per CU times CUs (or the request)
   int per_cu = 0;
   if (tp.refill < 1 || tp.refill > 64)

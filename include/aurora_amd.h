@@ -200,7 +200,8 @@ aur_status aur_trace_any(aur_context* ctx, uint64_t n, const aur_ray* rays, int3
  * src/kernels/monteCarloRaytracer.cu:119-124).  persistent = 1: resident
  * waves take ranges of the rays and refill idle lanes once `refill` (1..64)
  * lanes are idle; waves_per_cu = 0 uses the occupancy
- * limit, at most 16 to 24 by the tree's size.  persistent = 0: one lane per ray.  block: 64, 128 or 256.
+ * limit, without a window of stack rows at most 16 to 24 by the tree's size.
+ * persistent = 0: one lane per ray.  block: 64, 128 or 256.
  * stack_lds_rows: how many rows of each lane's stack of deferred ranges
  * (a compact stack of at most levels - 1 entries) live in LDS (0 = all);
  * deeper entries spill to global memory, leaving LDS for more waves.
@@ -254,9 +255,10 @@ aur_status aur_frame_render(aur_context* ctx, const aur_camera* camera,
  * this many (1..64) are idle; 0 selects the default (16).
  * stack_lds_rows: how many rows of each lane's traversal stack live in LDS
  * in those launches; deeper rows go to global memory, leaving LDS for more
- * resident waves.  0 selects the default (aur_get_render_params reports 12):
- * 12 rows in batches, every row in frames, as a value of at least the tree's
- * levels - 1 does.
+ * resident waves than the default has.  0, or 12 as aur_get_render_params
+ * reports it, selects the default: at least 12 rows in batches, every row in
+ * frames, as a value of at least the tree's levels - 1 does, and at most 20 or
+ * 28 waves per CU by the tree's size.
  * Images do not depend on any of them: samples are accumulated in sample
  * order. */
 typedef struct aur_render_params {
