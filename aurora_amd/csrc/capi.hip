@@ -80,6 +80,13 @@ aur_status aur_set_trace_params(aur_context* ctx, const aur_trace_params* p) {
   return AUR_OK;
 }
 
+aur_status aur_set_wide_records(aur_context* ctx, uint32_t on) {
+  if (!ctx) return AUR_ERR_INVALID_ARG;
+  if (on > 1) return ctx->fail(AUR_ERR_INVALID_ARG, "wide records: must be 0 or 1");
+  ctx->wide_records = on != 0;
+  return AUR_OK;
+}
+
 aur_status aur_get_trace_params(aur_context* ctx, aur_trace_params* p) {
   if (!ctx || !p) return AUR_ERR_INVALID_ARG;
   *p = ctx->trace_params;

@@ -210,6 +210,9 @@ struct aur_context {
   aur_render_params render_params{aur::kDefaultMaxPaths, 0, aur::kDefaultRenderRefill,
                                   aur::kDefaultRenderStackRows};
   bool render_rows_default = true;  // stack_lds_rows was not chosen by the caller
+  bool wide_records = false;        // aur_set_wide_records
+  // Whether a tree's records are addressed in 64 bits.
+  bool wide(uint32_t n_nodes) const { return wide_records || n_nodes >= aur::kWideNodes; }
   std::atomic<uint32_t> cancel{0};  // set by aur_cancel, consumed by the render it stops
 
   // uploaded geometry (input order)

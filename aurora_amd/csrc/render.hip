@@ -1223,10 +1223,10 @@ aur_status pbr_reserve(aur_context* ctx, uint32_t cap, uint32_t nslots, uint32_t
 }
 
 // k_pbr_trace with part of the stack in global memory (split) or not, for one
-// tree of n_nodes (kMulti: each lane's own tree, always 64-bit addresses).
+// tree (kMulti: each lane's own tree, always 64-bit addresses).
 template <bool kMulti>
-void (*trace_kernel(bool split, uint32_t n_nodes))(PbrArgs, uint32_t, uint32_t, uint32_t) {
-  if (kMulti || n_nodes >= kWideNodes)
+void (*trace_kernel(bool split, bool wide))(PbrArgs, uint32_t, uint32_t, uint32_t) {
+  if (kMulti || wide)
     return split ? k_pbr_trace<kMulti, true, true> : k_pbr_trace<kMulti, false, true>;
   return split ? k_pbr_trace<kMulti, true, kMulti> : k_pbr_trace<kMulti, false, kMulti>;
 }
@@ -1259,7 +1259,7 @@ aur_status trace_shape(aur_context* ctx, uint32_t levels, uint64_t max_items, Pb
       levels, chosen ? ctx->render_params.stack_lds_rows : (kMulti ? kDefaultRenderStackRows : 0u), chosen, kBlock, cu_waves);
   const uint32_t rows = shape.rows, maxrows = shape.maxrows;
   lds = shape.lds;
-  grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, a.job.n_nodes), lds, max_items);
+  grid = resident_grid(ctx, (const void*)trace_kernel<kMulti>(rows < maxrows, ctx->wide(a.job.n_nodes)), lds, max_items);
   a.gstack = nullptr;
   a.klds = rows;
   a.gstack_rows = 0;
@@ -1287,7 +1287,7 @@ void pbr_pass(aur_context* ctx, PbrArgs& a, size_t lds, uint32_t grid_trace,
   // with bounce b's shadow rays, then bounce b's next-event resolve
   const uint32_t sh = a.nslots ? 2u : 0u;
   const auto trace = [&](uint32_t w, uint32_t parts, uint32_t roff) {
-    trace_kernel<kMulti>(a.gstack != nullptr, a.job.n_nodes)<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
+    trace_kernel<kMulti>(a.gstack != nullptr, ctx->wide(a.job.n_nodes))<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
   };
   trace(0u, 1u, 0u);
   for (uint32_t b = 0; b < a.max_depth; ++b) {
@@ -1564,7 +1564,7 @@ aur_status compat_passes(aur_context* ctx, const aur_camera* cam, const aur_rend
   c.fin = fr.cw_fin.p;
   c.pixels = fr.pixels.p;
   const auto trace = [&](uint32_t w, uint32_t parts, uint32_t roff) {
-    trace_kernel<false>(a.gstack != nullptr, a.job.n_nodes)<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
+    trace_kernel<false>(a.gstack != nullptr, ctx->wide(a.job.n_nodes))<<<grid_trace, kBlock, lds, s>>>(a, w, parts, roff);
   };
   // every stack ray is a hit of depth <= 8 or below one: at most 1 + 2 * 9
   // rays per pixel sample, so the stacks empty within that many levels

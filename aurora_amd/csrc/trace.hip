@@ -235,7 +235,7 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
     return ctx->fail(AUR_ERR_INVALID_ARG, "trace: refill must be in 1..64");
   using Kern = void (*)(const NodeRec*, const float*, uint32_t, const aur_ray*, uint64_t, aur_hit*,
                         int32_t*, uint32_t*, uint32_t, float2*, uint32_t, uint32_t);
-  const bool wide = ctx->count / 2 >= kWideNodes;
+  const bool wide = ctx->wide(ctx->count / 2);
   const Kern fn = klds != 0 ? (wide ? k_trace_pt<kAny, true, true> : k_trace_pt<kAny, true, false>)
                             : (wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>);
   AUR_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, (int)block, lds_pt));

@@ -132,6 +132,7 @@ def load():
         "aur_check_reject": ([P, u64, P, ctypes.POINTER(u64), ctypes.POINTER(u64), ctypes.POINTER(u64)], i32),
         "aur_set_trace_params": ([P, ctypes.POINTER(TraceParams)], i32),
         "aur_get_trace_params": ([P, ctypes.POINTER(TraceParams)], i32),
+        "aur_set_wide_records": ([P, u32], i32),
         "aur_set_render_params": ([P, ctypes.POINTER(RenderParams)], i32),
         "aur_get_render_params": ([P, ctypes.POINTER(RenderParams)], i32),
         "aur_frame_create": ([P, u32, u32, u32], i32),
@@ -397,6 +398,10 @@ class Context:
         p = TraceParams()
         self._check(self._lib.aur_get_trace_params(self._h, ctypes.byref(p)), "get_trace_params")
         return {k: getattr(p, k) for k, _ in TraceParams._fields_}
+
+    def set_wide_records(self, on: bool) -> None:
+        """64-bit record addresses, as trees of 2^26 nodes and more take (for tests)."""
+        self._check(self._lib.aur_set_wide_records(self._h, int(on)), "set_wide_records")
 
     def set_render_params(self, max_paths: int = 0, graph: int = 0, refill: int = 0,
                           stack_lds_rows: int = 0) -> None:

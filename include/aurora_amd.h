@@ -211,6 +211,10 @@ typedef struct aur_trace_params {
 } aur_trace_params;
 aur_status aur_set_trace_params(aur_context* ctx, const aur_trace_params* params);
 aur_status aur_get_trace_params(aur_context* ctx, aur_trace_params* params);
+/* on = 1: traces and frame renders of this context address the tree's records
+ * in 64 bits, as they do for trees of 2^26 nodes and more by themselves; 0
+ * (default): in 32 bits below that.  For tests: results do not depend on it. */
+aur_status aur_set_wide_records(aur_context* ctx, uint32_t on);
 /* Closest hit plus the reference loop's traversal counters summed over the
  * rays: popped = states popped with index < count, passed = states whose slab
  * test passed.  Synchronous.  Used for the algorithmic-bytes model

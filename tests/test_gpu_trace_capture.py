@@ -15,7 +15,7 @@ N = 200_003
 
 
 @pytest.fixture()
-def setup(oracle):
+def setup(gpu_ctx, oracle):
     import torch
 
     s = scenes.spheres(n_spheres=10)
