@@ -278,7 +278,6 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
       return AUR_OK;
     }
     k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
-    k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
     AUR_LAUNCH_CHECK(ctx, "k_zero_work");
   }
   hipLaunchKernelGGL(fn, dim3(grid), dim3(block), lds_pt, ctx->stream, ctx->nodes.p, ctx->vertices.p,
