@@ -6,8 +6,8 @@
 // Each lane keeps its deferred ranges in an LDS column of levels - 1 float2
 // entries (or the first rows in LDS and the rest in global memory).
 //
-// k_trace_flat: one lane per ray, no refill (reference schedule; used for
-// comparison and by the instrumented counting launch).
+// k_trace_small: one lane per ray, for trees of a few nodes.  The instrumented
+// launches (k_trace_count, k_reject_check) take one lane per ray too.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,20 +76,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_trace_pt(const NodeRec* __restric
   }
 }
 
+// Trees of a few nodes: one lane per ray, both triangles of a node tested exactly.
 template <bool kAny>
-__global__ __launch_bounds__(kMaxBlock) void k_trace_flat(const NodeRec* __restrict__ nodes,
-                                                          const float* __restrict__ tris, uint32_t n_nodes,
-                                                          const aur_ray* __restrict__ rays,
-                                                          uint64_t n, aur_hit* __restrict__ hits,
-                                                          int32_t* __restrict__ ids) {
+__global__ __launch_bounds__(kMaxBlock) void k_trace_small(const NodeRec* __restrict__ nodes,
+                                                           const float* __restrict__ tris, uint32_t n_nodes,
+                                                           const aur_ray* __restrict__ rays, uint64_t n,
+                                                           aur_hit* __restrict__ hits, int32_t* __restrict__ ids) {
   extern __shared__ float2 stk_mem[];
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float4* r = reinterpret_cast<const float4*>(rays + i);
   const float4 a = r[0], b = r[1];
   Trav s;
-  trace_ray<kAny>(s, TreeRef{nodes, tris, n_nodes, {}}, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w,
-                  stk_mem + threadIdx.x, blockDim.x);
+  trace_ray<kAny, false, false, false>(s, TreeRef{nodes, tris, n_nodes, {}}, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w,
+                                       stk_mem + threadIdx.x, blockDim.x);
   store_result(i, s, hits, ids);
 }
 
@@ -197,6 +197,43 @@ __global__ __launch_bounds__(256) void k_division_check(uint32_t lo, uint32_t hi
   }
 }
 
+using TraceKernel = void (*)(const NodeRec*, const float*, uint32_t, const aur_ray*, uint64_t, aur_hit*, int32_t*,
+                             uint32_t*, uint32_t, float2*, uint32_t, uint32_t);
+
+// A wave for every 64 rays, in place of resident ones: the first ranges cover
+// the rays, so there is no counter.  Every stack row is in LDS.  (204,802
+// triangles, 2^20 rays, closest hit 438 us, any hit 388; with one lane walking
+// each ray by itself 683 and 377, as the lanes then take the exact tests one by
+// one; with both triangles tested exactly at every visit 561 and 511.)
+// Trees of up to this many levels (7 nodes) take k_trace_small.  2^20 rays, us
+// before the reject test and the work counters / with both / now: 2 triangles
+// 16 / 45 / 15, 6 29 / 50 / 25, 14 56 / 64 / 52; 24 triangles (4 levels) 78 / 73,
+// 93 with k_trace_small.
+constexpr uint32_t kSmallLevels = 3;
+
+template <bool kAny>
+aur_status launch_all(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_hit* hits, int32_t* ids) {
+  const uint32_t block = ctx->trace_params.block;
+  const StackShape shape = stack_shape(ctx->levels, 0, false, block, 0);
+  const TraceKernel fn = ctx->wide(ctx->count / 2) ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>;
+  constexpr uint64_t kSlice = 1ull << 30;  // rays of a launch
+  const bool small = ctx->levels <= kSmallLevels;
+  for (uint64_t at = 0; at < n; at += kSlice) {
+    const uint64_t m = std::min(kSlice, n - at);
+    const dim3 grid((uint32_t)((m + block - 1) / block));
+    aur_hit* const h = hits ? hits + at : nullptr;
+    int32_t* const id = ids ? ids + at : nullptr;
+    if (small)
+      k_trace_small<kAny><<<grid, block, shape.lds, ctx->stream>>>(ctx->nodes.p, ctx->vertices.p, ctx->count / 2,
+                                                                   rays + at, m, h, id);
+    else
+      hipLaunchKernelGGL(fn, grid, dim3(block), shape.lds, ctx->stream, ctx->nodes.p, ctx->vertices.p, ctx->count / 2,
+                         rays + at, m, h, id, nullptr, 64u, nullptr, 0u, 0u);
+    AUR_LAUNCH_CHECK(ctx, "k_trace");
+  }
+  return AUR_OK;
+}
+
 // The work counters of the next persistent launch.
 __global__ void k_zero_work(uint32_t* p) { p[threadIdx.x] = 0u; }
 
@@ -205,14 +242,9 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
                         int32_t* ids) {
   const aur_trace_params& tp = ctx->trace_params;
   const uint32_t block = tp.block;
-  const size_t lds = (size_t)ctx->levels * block * sizeof(float2);
-  if (!tp.persistent) {
-    const uint64_t nb = (n + block - 1) / block;
-    if (nb > 0x7FFFFFFFull) return ctx->fail(AUR_ERR_INVALID_ARG, "trace: too many rays");
-    k_trace_flat<kAny><<<(uint32_t)nb, block, lds, ctx->stream>>>(ctx->nodes.p, ctx->vertices.p, ctx->count / 2,
-                                                                  rays, n, hits, ids);
-    AUR_LAUNCH_CHECK(ctx, "k_trace_flat");
-    return AUR_OK;
+  if (!tp.persistent || (ctx->levels <= kSmallLevels && !tp.waves_per_cu)) {
+    if ((n + block - 1) / block > 0x7FFFFFFFull) return ctx->fail(AUR_ERR_INVALID_ARG, "trace: too many rays");
+    return launch_all<kAny>(ctx, n, rays, hits, ids);
   }
   // Waves per CU: each visits 64 records at a time, and the more waves, the
   // fewer of their lines stay in the L1 (32 KB) between a record's four loads;
@@ -233,11 +265,9 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
   int per_cu = 0;
   if (tp.refill < 1 || tp.refill > 64)
     return ctx->fail(AUR_ERR_INVALID_ARG, "trace: refill must be in 1..64");
-  using Kern = void (*)(const NodeRec*, const float*, uint32_t, const aur_ray*, uint64_t, aur_hit*,
-                        int32_t*, uint32_t*, uint32_t, float2*, uint32_t, uint32_t);
   const bool wide = ctx->wide(ctx->count / 2);
-  const Kern fn = klds != 0 ? (wide ? k_trace_pt<kAny, true, true> : k_trace_pt<kAny, true, false>)
-                            : (wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>);
+  const TraceKernel fn = klds != 0 ? (wide ? k_trace_pt<kAny, true, true> : k_trace_pt<kAny, true, false>)
+                                   : (wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>);
   AUR_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, (int)block, lds_pt));
   if (per_cu < 1) per_cu = 1;
   uint64_t blocks_total = (uint64_t)per_cu * ctx->num_cus;
@@ -264,19 +294,8 @@ aur_status launch_trace(aur_context* ctx, uint64_t n, const aur_ray* rays, aur_h
       work = ctx->trace_work.p;
     else if (ctx->trace_work_recorded + 1 < kTraceWorkSets)
       work = ctx->trace_work.p + (size_t)++ctx->trace_work_recorded * kWorkWords;
-    else {  // no set left: one range per wave (the test on a null counter in the kernel cost any-hit queries 1.5%)
-      const Kern all = wide ? k_trace_pt<kAny, false, true> : k_trace_pt<kAny, false, false>;
-      constexpr uint64_t kSlice = 1ull << 30;
-      for (uint64_t at = 0; at < n; at += kSlice) {
-        const uint64_t m = std::min(kSlice, n - at);
-        hipLaunchKernelGGL(all, dim3((uint32_t)((m + block - 1) / block)), dim3(block),
-                           (size_t)maxrows * block * sizeof(float2), ctx->stream, ctx->nodes.p, ctx->vertices.p,
-                           ctx->count / 2, rays + at, m, hits ? hits + at : nullptr, ids ? ids + at : nullptr, nullptr,
-                           tp.refill, nullptr, 0u, 0u);
-        AUR_LAUNCH_CHECK(ctx, "k_trace_pt");
-      }
-      return AUR_OK;
-    }
+    else  // no set left (a test on a null counter in the kernel cost any-hit queries 1.5%)
+      return launch_all<kAny>(ctx, n, rays, hits, ids);
     k_zero_work<<<1, kWorkWords, 0, ctx->stream>>>(work);
     AUR_LAUNCH_CHECK(ctx, "k_zero_work");
   }

@@ -408,6 +408,14 @@ __device__ __forceinline__ void trav_test(Trav& s, const TreeRef& tree, TraceCou
   __asm__ volatile("" : "+v"(s.slab.x), "+v"(s.slab.y), "+v"(s.slab.z), "+v"(s.slab.w));
 }
 
+// The slabs and flags alone, for visits that test both triangles exactly.
+__device__ __forceinline__ void trav_slabs(Trav& s, const TreeRef& tree) {
+  const uint4* rec = reinterpret_cast<const uint4*>(tree.nodes + s.K);
+  const uint4 a0 = rec[0];
+  s.flags = rec[1].w;
+  s.slab = make_float4(__uint_as_float(a0.x), __uint_as_float(a0.y), __uint_as_float(a0.z), __uint_as_float(a0.w));
+}
+
 // The reference's test (Ray::intersect, src/kernels/lib/ray.cuh:22-47) of a
 // triangle on the vertices it was uploaded with, for any t above kEpsilon.
 __device__ __forceinline__ bool tri_accept(const Trav& s, const float* __restrict__ tris, uint32_t tri, float& u,
@@ -655,7 +663,7 @@ __device__ __forceinline__ void persistent_trace(TreeRef tree0, uint64_t n, uint
 
 // Whole traversal of one ray by one lane.
 // stk: this lane's stack column, stk[depth * stride].
-template <bool kAny, bool kCount = false, bool kCheck = false>
+template <bool kAny, bool kCount = false, bool kCheck = false, bool kReject = true>
 __device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3 d, float tmax, float2* stk,
                                           uint32_t stride, TraceCount* cnt = nullptr, RejectCount* rej = nullptr) {
   const LdsStack st = lds_stack(stk, stride);
@@ -663,8 +671,11 @@ __device__ __forceinline__ void trace_ray(Trav& s, const TreeRef& tree, V3 o, V3
   bool popping = false;
   for (;;) {
     if (!popping) {
-      bool a, b;
-      trav_test<kCount, true>(s, tree, cnt, a, b);
+      bool a = true, b = true;
+      if (kReject)
+        trav_test<kCount, true>(s, tree, cnt, a, b);
+      else
+        trav_slabs(s, tree);
       if (kCheck) {
         float u, v, t;
         const bool hit_a = tri_accept(s, tree.tris, 2 * s.K - 2, u, v, t);
