@@ -286,16 +286,17 @@ __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3
 // ---- the reject test ----
 //
 // Loads the node's record and says which of its triangles may
-// pass the reference's test.  Two things bound a visit when every lane reads
-// another node: VALU issue and the vector L1, which looks up one lane's 16
-// bytes per cycle and CU.  Both triangles' exact test took 125 VALU
-// instructions and a 96-byte record 6 loads; this test takes 67 and the
-// 64-byte record 4, and what it leaves over (1.2% of the visits at 1M
-// triangles) costs 6 more per visit.  2^24 incoherent rays into 1M triangles
-// take 4.6 ms (7.3 with the exact tests in every visit): 2.35e9 VALU
-// instructions at 0.86 of the issue rate, 2.97e9 L1 lookups at 1.08 per cycle
-// and CU.  More resident waves than 16 per CU are slower: the lines of their
-// visits no longer fit the 32 KB L1 between a record's four loads.
+// pass the reference's test.  VALU issue bounds a visit, and the vector L1
+// comes next: a load of 64 lanes that read 64 nodes is 64 lookups.  Both
+// triangles' exact test took 125 VALU instructions and a 96-byte record 6
+// loads; this test takes 67 and the 64-byte record 4, and what it leaves over
+// (1.2% of the visits at 1M triangles) costs 6 more per visit.  2^24 incoherent
+// rays into 1M triangles take 4.6 ms (7.3 with the exact tests in every visit):
+// 2.38e9 VALU instructions at 0.88 of the issue rate, 2.98e9 L1 lookups at 1.10
+// per cycle and CU (lanes that read random 64-byte records of a buffer that the
+// L1 holds reach 1.48).  More resident waves than 16 per CU are slower: the
+// lines of their visits no longer fit the 32 KB L1 between a record's four
+// loads.
 //
 // With T = p - v1 for any point p of the ray's line and C = T x d, the
 // Moller-Trumbore numerators are u det = e2 . C, v det = -(e1 . C) and
@@ -305,8 +306,9 @@ __device__ __forceinline__ bool trav_init(Trav& s, const TreeRef& tree, V3 o, V3
 // is no larger than the node's group, and lengths are in units of the group's
 // size.  T is computed as (o - v1) + t d, whose rounding does not grow with the
 // coordinates: with p computed first and a threshold for the largest coordinate
-// of the tree, 2^22 incoherent rays into 1M triangles over a ground plane 2000 km
-// wide took 2.95 ms, 1.56 now (1.40 without the plane), 1000 km 2.20 ms, 1.55 now.
+// of the tree, 2^22 incoherent rays into 1M triangles in a box of 100 over a
+// ground plane 2e6 wide took 2.95 ms, 1.56 now (1.40 without the plane; 2.10 with
+// the exact tests in every visit), 2e5 wide 2.20 ms, 1.55 now.
 //
 // Bound.  D = the largest |direction component|, z = the triangle's size (each
 // |e| component <= z), q = 2^-11 + 2^-15, t = the range's entry; sigma = 2^-k,
